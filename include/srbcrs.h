@@ -209,7 +209,15 @@ int srbcrs_plan_set_schedule(srbcrs_plan *plan, const char *policy, int32_t para
  * and stay allocated until srbcrs_plan_trim or srbcrs_plan_destroy, so a HIP
  * graph captured on an earlier run keeps valid addresses.  Capture after one
  * eager run with the same N, ldc and schedule (a growing run allocates,
- * which graph capture forbids).  A call that is refused (a negative status)
+ * which graph capture forbids).
+ * On matrices of low block fill (16x8 blocks, under a ninth of the positions
+ * stored) the default launch is the column sweep, a vector kernel over the
+ * stored values that gives the block kernels' bits (infinities and NaNs of B
+ * included); it needs ldb, ldc multiples of 4, 16-byte aligned B and C and
+ * K * ldb * 4 < 2^32, and runs from a width's second run on, which builds its
+ * entry stream (it allocates 8 bytes per stored value, kept until the plan is
+ * destroyed): capture after two eager runs to capture it.  Elsewhere, under
+ * capture before that, and on small products, the block kernels run.  A call that is refused (a negative status)
  * has launched nothing and left C untouched. */
 int srbcrs_run(srbcrs_plan *plan, const float *d_B, int64_t K, int64_t N, int64_t ldb,
                float *d_C, int64_t ldc, int64_t c_rows, void *stream);
@@ -239,7 +247,8 @@ int srbcrs_plan_trim(srbcrs_plan *plan, void *stream);
  *                256-column waves (four groups per lane, N % 256 == 0) in
  *                workgroups of 256 columns or more, 128-column waves at 128,
  *                64-column waves at 64;
- *   grid_order   0 = default (chunk-major), 1 = chunk-major: one column
+ *   grid_order   0 = default (chunk-major; with all knobs 0, the column
+ *                sweep where srbcrs_run describes it), 1 = chunk-major: one column
  *                chunk of every window before the next chunk (narrower B
  *                working set per XCD), 2 = window-major, 3 = chunk sweep:
  *                chunk-major in dispatch order, all XCDs on one chunk at a
@@ -375,7 +384,10 @@ size_t srbcrs_noalloc_scratch_floats(void);
  * 4), (128, 4, 2), (64, 8, 2), (64, 4, 4) where N allows it (a setting the
  * operands' alignment refuses is skipped).  Each gets one warm-up
  * and `reps` timed launches on `stream`; the first candidate within 3 % of
- * the fastest wins, so near-ties resolve the same way on every run.  Later
+ * the fastest wins, so near-ties resolve the same way on every run.  The
+ * default launch is timed first where it is the column sweep; if it wins,
+ * default-knob runs keep it and best receives the fastest other setting of
+ * the same bits.  Later
  * srbcrs_run calls, and srbcrs_run_ex calls whose knobs are all 0, use it
  * at that N until the schedule changes.  C is overwritten (with the
  * product).  Every candidate gives the same bits: tuning changes only the

@@ -13,8 +13,10 @@
 #include <new>
 #include <string>
 #include <thread>
+#include <tuple>
 #include <map>
 #include <mutex>
+#include <set>
 #include <vector>
 
 #include "../../include/srbcrs.h"
@@ -462,6 +464,22 @@ struct srbcrs_plan {
     int64_t entries = 0;
   };
   std::map<int64_t, Nz> nz;
+  // The column sweep's entry streams, per schedule (policy, parameter) and
+  // rows per list, built by the second run of a width and kept until the
+  // plan is destroyed (a HIP graph may hold their addresses).
+  struct Sweep {
+    std::set<int64_t> seen;   // widths that have run
+    int32_t longest = 0;   // blocks of the schedule's longest task
+    bool failed = false;   // cannot be built: the block kernels run, with the same bits
+    bool built = false;
+    srbcrs::ColSweep s;
+  };
+  std::mutex sweep_mu;   // runs on several threads may come first together
+  std::map<std::tuple<std::string, int32_t, int>, Sweep> sweeps;
+  // non-finite marks of the runs in flight: run i (from 1) raises slot i %
+  // kSweepFlags to i, its repair pass looks whether the slot has reached i
+  unsigned long long* d_sweep_flags = nullptr;
+  std::atomic<unsigned long long> sweep_runs{0};
 
   template <class T>
   void retire(T*& p) {
@@ -494,6 +512,12 @@ struct srbcrs_plan {
     dev_free(d_bp);
     dev_free(d_awords);
     dev_free(d_apacked);
+    dev_free(d_sweep_flags);
+    for (auto& kv : sweeps) {
+      srbcrs::ColSweep& w = kv.second.s;
+      dev_free(w.entries);
+      for (int** p : {&w.start, &w.nblk, &w.dest, &w.wblk8, &w.wblk4, &w.lstart, &w.lnblk, &w.ldest}) dev_free(*p);
+    }
     for (auto& kv : merged) {
       dev_free(kv.second.d_moff);
       dev_free(kv.second.d_sidx);
@@ -738,6 +762,76 @@ const srbcrs_plan::Merged& merged_stream(srbcrs_plan& plan, int W, hipStream_t s
   }
   m.units = units;
   return plan.merged.emplace(W, m).first->second;
+}
+
+constexpr int kSweepFlags = 256;
+constexpr int kSweepKeyCols = 1 << 24;   // an entry holds 24 bits of B row
+
+srbcrs::ColSweepTasks sweep_tasks(const srbcrs_plan& plan) {
+  if (plan.sched.policy == "row") return {plan.d_soff, plan.d_soff + 1, nullptr, nullptr, plan.Mo};
+  return {plan.d_task_begin, plan.d_task_end, plan.d_task_window, plan.d_task_slot, (int)plan.sched.task_begin.size()};
+}
+
+// Whether the default launch of this plan is the column sweep: 16x8 blocks
+// with the compact copy, less than a ninth of the block positions stored.
+// Measured at 65536 rows of 16 with window-clustered columns (us, sweep / block
+// kernel): fill 0.094 N = 64 28 / 31, N = 512 152 / 187; fill 0.116 28 / 27,
+// 150 / 156, and above it the block kernel shares each B row among more rows.
+bool sweep_wanted(const srbcrs_plan& plan) {
+  return plan.blk_h == 16 && plan.packing == SRBCRS_PACK_CONDENSED && plan.d_awords && plan.total > 0 &&
+         plan.max_col < kSweepKeyCols && 9 * plan.n_apacked < plan.total * 128;
+}
+
+// The column sweep stream for a run of N columns; null: run the block
+// kernels, which give the same bits.  The first run of a width does that: a
+// plan run once (a sampled graph) does not pay for the stream, which takes
+// about as long as a few runs gain.  Not built under graph capture or for a
+// caller that may not allocate.
+const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_build, hipStream_t st) {
+  const srbcrs::ColSweepTasks t = sweep_tasks(plan);
+  const int RL = srbcrs::colsweep_rows_per_list((int64_t)t.n * 16, (int)N);
+  std::lock_guard<std::mutex> lock(plan.sweep_mu);
+  srbcrs_plan::Sweep& w = plan.sweeps[{plan.sched.policy, plan.sched.param, RL}];
+  if (!w.longest)
+    for (int32_t i = 0; i < plan.Mo; ++i) w.longest = std::max(w.longest, plan.h_soff[i + 1] - plan.h_soff[i]);
+  // Small products stay with the block kernel's one launch (the sweep's repair
+  // pass is a second one, 4 us of host time): under 64 MB of gathers both take
+  // less than their launches, unless long windows make the block kernel a
+  // chain (about 0.4 us a block: 40 blocks 17.9 us, sweep 8 + 1.5).
+  if (plan.n_apacked * N < (16 << 20) && w.longest < 24) return nullptr;
+  if (w.built) return &w.s;
+  if (w.failed || !may_build) return nullptr;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (w.seen.insert(N).second) return nullptr;
+  srbcrs::ColSweep s;
+  s.RL = RL;
+  // phases of 4096 columns (512 KB of a 32-column slice; 2048 to 16384 ran
+  // within 3 % of it), one phase where B's slice fits the L2
+  s.shift = 12;
+  while ((plan.max_col >> s.shift) >= 128) ++s.shift;
+  if (plan.max_col < 16384) s.shift = 24;
+  s.phases = (plan.max_col >> s.shift) + 1;
+  hipError_t e = hipSuccess;
+  if (!plan.d_sweep_flags) {
+    e = hipMalloc(reinterpret_cast<void**>(&plan.d_sweep_flags), kSweepFlags * 8);
+    if (e == hipSuccess) e = hipMemsetAsync(plan.d_sweep_flags, 0, kSweepFlags * 8, st);
+  }
+  srbcrs::ColSweepIn in{t, plan.d_awords, plan.d_sidx, plan.d_apacked, plan.n_apacked, plan.d_rowmap,
+                        (int)plan.packed_rows};
+  if (e == hipSuccess) e = srbcrs::build_colsweep(in, s, conv_alloc, conv_free, nullptr, st);
+  if (e == hipErrorOutOfMemory || e == hipErrorInvalidValue) {
+    (void)hipGetLastError();
+    w.failed = true;
+    return nullptr;
+  }
+  hip_check(e, "column sweep stream");
+  w.s = s;
+  w.built = true;
+  return &w.s;
 }
 
 int64_t nz_key(int W, int U, int D) { return ((int64_t)W << 16) | ((int64_t)U << 8) | (int64_t)D; }
@@ -1425,10 +1519,29 @@ static void run_impl(srbcrs_plan* plan, const float* d_B, int64_t K, int64_t N, 
       hip_check(srbcrs::launch_nzsweep(za, a, U, D, st), "launch spmm_nzsweep");
       return;
     }
+    // No knobs at low block fill: the column sweep, where its 32-bit offsets
+    // and 16-byte accesses reach (the block kernels' bits either way).
+    const srbcrs::ColSweep* sweep = nullptr;
+    if ((!opts || all_default(*opts)) && sweep_wanted(*plan) && ldb % 4 == 0 && ldc % 4 == 0 &&
+        (reinterpret_cast<uintptr_t>(d_B) | reinterpret_cast<uintptr_t>(d_C)) % 16 == 0 &&
+        (uint64_t)K * (uint64_t)ldb * 4u < (1ull << 32) && (uint64_t)ldb * 4u < (1ull << 24))
+      sweep = sweep_stream(*plan, N, !fixed_partial, st);
+    auto launch_sweep = [&](float* partial) {
+      const unsigned long long run = ++plan->sweep_runs;
+      unsigned long long* flag = plan->d_sweep_flags + run % kSweepFlags;
+      srbcrs::StreamArgs sa = a;
+      sa.partial = partial;
+      hip_check(srbcrs::launch_colsweep(*sweep, sa, K, run, flag, st), "launch spmm_colsweep");
+      hip_check(srbcrs::launch_colsweep_repair(sweep_tasks(*plan), sa, run, flag, st), "launch sweep repair");
+    };
     if (plan->sched.policy == "row") {
       if (plan->n_zero_rows)
         hip_check(srbcrs::launch_zero_rows(d_C, plan->d_zero_rows, plan->n_zero_rows, (int)N, ldc, st),
                   "launch zero_rows");
+      if (sweep) {
+        launch_sweep(nullptr);
+        return;
+      }
       hip_check(srbcrs::launch_row(a, plan->d_soff, plan->Mo, vec, ro, st), "launch spmm_stream(row)");
       return;
     }
@@ -1461,7 +1574,10 @@ static void run_impl(srbcrs_plan* plan, const float* d_B, int64_t K, int64_t N, 
                 "launch zero_rows");
     srbcrs::TaskTable tt{plan->d_group_off, plan->d_task_begin, plan->d_task_end, plan->d_task_window,
                          plan->d_task_slot, (int)s.group_off.size() - 1};
-    hip_check(srbcrs::launch_tasks(a, tt, vec, ro, st), "launch spmm_stream(tasks)");
+    if (sweep)
+      launch_sweep(partial);
+    else
+      hip_check(srbcrs::launch_tasks(a, tt, vec, ro, st), "launch spmm_stream(tasks)");
     srbcrs::ReduceArgs ra{partial, d_C, plan->d_red_window, plan->d_red_slot_off,
                           (int)s.red_window.size(), plan->blk_h, (int)plan->packed_rows, (int)N, ldc,
                           plan->d_rowmap, a.relu};
@@ -1665,6 +1781,10 @@ int srbcrs_plan_tune_ex(srbcrs_plan* plan, const float* d_B, int64_t K, int64_t 
   // merged-window and nonzero-sweep candidates last (a near-tie keeps the
   // plainer setting); one the operands cannot run (N, B / C alignment, ldb /
   // ldc, B's extent) is dropped here
+  // first the default launch, where it is not one of the settings below (the
+  // column sweep; its two extra warm-ups build its stream)
+  const bool has_default = sweep_wanted(*plan);
+  if (has_default) cand.insert(cand.begin(), srbcrs_run_opts{});
   const size_t n_plain = cand.size();
   cand.insert(cand.end(), merged_cand.begin(), merged_cand.end());
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1675,6 +1795,8 @@ int srbcrs_plan_tune_ex(srbcrs_plan* plan, const float* d_B, int64_t K, int64_t 
   std::vector<float> ms_of(cand.size(), -1.f);
   for (size_t i = 0; rc == SRBCRS_OK && i < cand.size(); ++i) {
     rc = srbcrs_run_ex(plan, d_B, K, N, ldb, d_C, ldc, c_rows, &cand[i], stream);   // warm-up, validates
+    for (int r = 0; r < 2 && rc == SRBCRS_OK && has_default && i == 0; ++r)
+      rc = srbcrs_run_ex(plan, d_B, K, N, ldb, d_C, ldc, c_rows, &cand[i], stream);
     if (rc == SRBCRS_EINVAL && i >= n_plain) {   // a merged / sweep setting these operands cannot run
       rc = SRBCRS_OK;
       continue;
@@ -1700,13 +1822,22 @@ int srbcrs_plan_tune_ex(srbcrs_plan* plan, const float* d_B, int64_t K, int64_t 
   float best_ms = -1.f;
   for (float ms : ms_of)
     if (ms >= 0.f && (best_ms < 0.f || ms < best_ms)) best_ms = ms;
+  // Where the default launch wins, it stays: no setting is kept for N, and
+  // best receives the fastest setting with the same bits.
+  const bool keep_default = has_default && ms_of[0] >= 0.f && ms_of[0] <= best_ms * 1.03f;
+  if (keep_default) {
+    best_ms = -1.f;
+    for (size_t i = 1; i < cand.size(); ++i)
+      if (cand[i].grid_order != SRBCRS_GRID_NZSWEEP && ms_of[i] >= 0.f && (best_ms < 0.f || ms_of[i] < best_ms))
+        best_ms = ms_of[i];
+  }
   srbcrs_run_opts best_o{};
-  for (size_t i = 0; i < cand.size(); ++i)
-    if (ms_of[i] >= 0.f && ms_of[i] <= best_ms * 1.03f) {
+  for (size_t i = has_default ? 1 : 0; i < cand.size(); ++i)
+    if (ms_of[i] >= 0.f && ms_of[i] <= best_ms * 1.03f && !(keep_default && cand[i].grid_order == SRBCRS_GRID_NZSWEEP)) {
       best_o = cand[i];
       break;
     }
-  if (best_ms >= 0.f) plan->tuned[N] = best_o;
+  if (best_ms >= 0.f && !keep_default) plan->tuned[N] = best_o;
   if (best) *best = best_o;
   return SRBCRS_OK;
 }

@@ -1,0 +1,215 @@
+// Column sweep (srbcrs_colsweep.hpp): launcher and the device-side build of
+// its entry stream.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <algorithm>
+
+#include "srbcrs_colsweep.hpp"
+#include "srbcrs_convert.h"
+#include "srbcrs_kernels.h"
+
+namespace srbcrs {
+
+template <int C, int RL, int WV>
+static hipError_t launch_t(const ColSweep& s, const StreamArgs& a, int64_t K, int swept, unsigned long long token,
+                           unsigned long long* flag, hipStream_t st) {
+  const int n_chunks = (a.N + C - 1) / C;
+  const int n_waves = s.n_lists / (256 / C);
+  const int64_t n_wg = (n_waves + WV - 1) / WV;
+  int64_t grid = n_wg * n_chunks;
+  if (!swept && n_chunks <= kNumXcd && kNumXcd % n_chunks == 0) {
+    const int per = kNumXcd / n_chunks;
+    grid = (n_wg + per - 1) / per * kNumXcd;
+  }
+  const int64_t long_waves = (int64_t)s.n_long * ((a.N + 63) / 64);
+  const int64_t long_wgs = ((long_waves + WV - 1) / WV + kNumXcd - 1) / kNumXcd * kNumXcd;
+  grid += long_wgs;
+  if (grid == 0) return hipSuccess;
+  if (long_waves > INT32_MAX || grid > INT32_MAX) return hipErrorInvalidConfiguration;
+  const uint64_t bytes = ((uint64_t)(K - 1) * (uint64_t)a.ldb + (uint64_t)a.N) * 4u;
+  const SweepStream ss{s.entries, s.start, s.nblk, C == 32 ? s.wblk8 : s.wblk4, s.dest, n_waves,
+                       s.lstart, s.lnblk, s.ldest, s.n_long};
+  hipLaunchKernelGGL((spmm_colsweep<C, RL, WV>), dim3((unsigned)grid), dim3(64 * WV), 0, st, ss, a.B, (uint32_t)bytes,
+                     a.C, a.partial, a.N, (uint32_t)(a.ldb * 4), a.ldc, n_chunks, swept, a.relu, token, flag, (int)long_wgs);
+  return hipGetLastError();
+}
+
+// Which kernel a launch runs, from sweeps of every (columns, waves per
+// workgroup, mapping) over 17 matrices and widths 48-512 on one MI355X
+// (fastest setting / the setting the rule would otherwise take, us).
+//
+// 64 columns where 32-column segments would straddle cache lines (N = 112,
+// 100000 rows of 30: 143 / 157) or where the columns' 64-wide slice of B fits
+// an XCD's L2 anyway (K = 8000, N = 256: 54 / 61); below 200000 rows also
+// where the 32-column chunks are exactly 8, one per XCD: with B rows of 1 KB
+// each XCD then sees one 128-byte phase of every KB, which its L2 channels do
+// not spread (N = 256, 65536 rows: 85 / 92).  Else 32 columns: twice the rows
+// in flight per CU (65536 rows of 16, N = 64: 29 / 32; power-law, 131072
+// nodes, N = 512: 968 / 1045).
+//
+// A workgroup of 16 waves in step where B's slice exceeds the L2 (K = 100000,
+// 30000 rows, N = 512: 104 / 137) and the workgroups fill their last round of
+// CUs (one workgroup per CU): a round that is mostly empty costs more
+// (power-law, 116483 nodes, N = 128, 1.8 rounds: 139 one wave / 165).
+//
+// Chunks are pinned to XCDs (an XCD's rows in flight are then all rows of its
+// chunk) except for 32-column chunks of so many rows that one XCD's eighth of
+// them fills it: then all XCDs take a chunk at the same time and share its B
+// rows in the memory-side cache (524288 nodes, N = 256: 1820 / 1940).
+constexpr int64_t kSyncBytes = 6 << 20;     // B slice above which waves keep step (4 MB of L2 hold the hot rows)
+constexpr int64_t kSweptRows = 200000;
+
+static void pick_launch(int64_t rows, int RL, const StreamArgs& a, int64_t K, int& cols, int& wv, int& swept) {
+  const int64_t chunks32 = (a.N + 31) / 32;
+  const bool sync = K * 128 > kSyncBytes;
+  cols = a.N % 32 || a.ldb % 32 || K <= 16384 || (sync && chunks32 == kNumXcd && rows < kSweptRows) ? 64 : 32;
+  const int64_t waves = rows / (8 * RL) * chunks32;
+  const int64_t wgs = waves / 16, rounds = (wgs + 255) / 256;
+  wv = sync && RL == 8 && waves >= 3500 && (rounds > 3 || 10 * wgs >= 9 * 256 * rounds) ? 16 : 1;
+  swept = cols == 32 && rows >= kSweptRows;
+}
+
+int colsweep_rows_per_list(int64_t rows, int N) {
+  const int64_t chunks32 = (N + 31) / 32;
+  int RL = 8;
+  while (RL > 1 && rows / (8 * RL) * chunks32 < 2000) RL /= 2;
+  return RL;
+}
+
+hipError_t launch_colsweep(const ColSweep& s, const StreamArgs& a, int64_t K, unsigned long long token,
+                           unsigned long long* flag, hipStream_t st) {
+  int cols, wv, swept;
+  pick_launch((int64_t)s.n_lists * s.RL, s.RL, a, K, cols, wv, swept);
+#define SRBCRS_SWEEP(C, RL, WV) return launch_t<C, RL, WV>(s, a, K, swept, token, flag, st)
+#define SRBCRS_SWEEP_RL(C)                  \
+  switch (s.RL) {                           \
+    case 8:                                 \
+      if (wv == 16) SRBCRS_SWEEP(C, 8, 16); \
+      SRBCRS_SWEEP(C, 8, 1);                \
+    case 4: SRBCRS_SWEEP(C, 4, 1);          \
+    case 2: SRBCRS_SWEEP(C, 2, 1);          \
+    default: SRBCRS_SWEEP(C, 1, 1);         \
+  }
+  if (cols == 32) SRBCRS_SWEEP_RL(32)
+  SRBCRS_SWEEP_RL(64)
+#undef SRBCRS_SWEEP_RL
+#undef SRBCRS_SWEEP
+}
+
+static SweepTasks sweep_tasks(const ColSweepTasks& t) { return SweepTasks{t.begin, t.end, t.window, t.slot, t.n}; }
+
+hipError_t launch_colsweep_repair(const ColSweepTasks& t, const StreamArgs& a, unsigned long long token,
+                                  const unsigned long long* flag, hipStream_t st) {
+  const int64_t work = (int64_t)t.n * ((a.N + 63) / 64);
+  if (work == 0) return hipSuccess;
+  const unsigned grid = work < 4096 ? (unsigned)work : 4096u;
+  hipLaunchKernelGGL(k_sweep_repair, dim3(grid), dim3(64), 0, st, flag, token, sweep_tasks(t), a.a_words, a.sidx,
+                     a.a_packed, a.B, a.C, a.partial, a.rowmap, a.M, a.N, a.ldb, a.ldc, a.relu);
+  return hipGetLastError();
+}
+
+hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc, DeviceFree dfree, void* ctx,
+                          hipStream_t st) {
+  const SweepTasks t = sweep_tasks(in.tasks);
+  const int64_t rows = (int64_t)t.n * 16;
+  const int RL = out.RL;
+  const int64_t n_lists = (rows + 8 * RL - 1) / (8 * RL) * 8, slots = n_lists * RL;
+  if (rows == 0 || slots > INT32_MAX) return hipErrorInvalidValue;
+  out.n_lists = (int)n_lists;
+  // rows over the lists' average, and over 128 values, are long (power-law
+  // graph of 8000 nodes, N = 64, us: 88 none, 28 over 256, 21 over 128; of
+  // 232965 nodes, N = 256: 1378 over twice the average, 1297 over it)
+  constexpr int64_t kLongMin = 128;
+  const int64_t long_len = std::max<int64_t>(kLongMin, in.n_values / n_lists);
+  const int long_bin = sweep_bin((int)long_len);
+  // stored values, and room for explicit zeros (k_sweep_len counts them)
+  const int64_t most = in.n_values + in.n_values / 16 + 4096;
+  const int64_t long_cap = most / kLongMin + 1;
+  const int64_t cap = most + kSweepBatch * n_lists + kSweepLongBatch * long_cap;
+  if (cap > INT32_MAX) return hipErrorInvalidValue;
+  int *len = nullptr, *hist = nullptr, *vrow = nullptr, *list_len = nullptr, *lvrow = nullptr;
+  unsigned long long* total = nullptr;
+  auto drop = [&](auto*& p) {
+    if (p) dfree(ctx, (void*)p);
+    p = nullptr;
+  };
+  auto cleanup = [&](hipError_t e) {
+    drop(len);
+    drop(hist);
+    drop(vrow);
+    drop(list_len);
+    drop(lvrow);
+    drop(total);
+    if (e != hipSuccess) {
+      drop(out.entries);
+      drop(out.start);
+      drop(out.nblk);
+      drop(out.wblk8);
+      drop(out.wblk4);
+      drop(out.dest);
+      drop(out.lstart);
+      drop(out.lnblk);
+      drop(out.ldest);
+    }
+    return e;
+  };
+  len = (int*)alloc(ctx, (size_t)rows * 4);
+  hist = (int*)alloc(ctx, 2 * kSweepBins * 4);
+  vrow = (int*)alloc(ctx, (size_t)slots * 4);
+  list_len = (int*)alloc(ctx, (size_t)n_lists * 4);
+  lvrow = (int*)alloc(ctx, (size_t)long_cap * 4);
+  total = (unsigned long long*)alloc(ctx, 16);   // entries taken, long rows
+  out.entries = (uint2*)alloc(ctx, (size_t)(cap + 8) * 8);
+  out.start = (int*)alloc(ctx, (size_t)n_lists * 4);
+  out.nblk = (int*)alloc(ctx, (size_t)n_lists * 4);
+  out.wblk8 = (int*)alloc(ctx, (size_t)n_lists / 8 * 4);
+  out.wblk4 = (int*)alloc(ctx, (size_t)n_lists / 4 * 4);
+  out.dest = (int*)alloc(ctx, (size_t)slots * 4);
+  out.lstart = (int*)alloc(ctx, (size_t)long_cap * 4);
+  out.lnblk = (int*)alloc(ctx, (size_t)long_cap * 4);
+  out.ldest = (int*)alloc(ctx, (size_t)long_cap * 4);
+  if (!len || !hist || !vrow || !list_len || !total || !out.entries || !out.start || !out.nblk || !out.wblk8 ||
+      !out.wblk4 || !out.dest || !lvrow || !out.lstart || !out.lnblk || !out.ldest)
+    return cleanup(hipErrorOutOfMemory);
+#define SRBCRS_STEP(x)                          \
+  do {                                          \
+    const hipError_t e_ = (x);                  \
+    if (e_ != hipSuccess) return cleanup(e_);   \
+  } while (0)
+  SRBCRS_STEP(hipMemsetAsync(hist, 0, 2 * kSweepBins * 4, st));
+  SRBCRS_STEP(hipMemsetAsync(vrow, 0xff, (size_t)slots * 4, st));
+  SRBCRS_STEP(hipMemsetAsync(out.dest, 0xff, (size_t)slots * 4, st));
+  SRBCRS_STEP(hipMemsetAsync(list_len, 0, (size_t)n_lists * 4, st));
+  SRBCRS_STEP(hipMemsetAsync(total, 0, 16, st));
+  int64_t g = (rows + 31) / 32;
+  hipLaunchKernelGGL(k_sweep_len, dim3((unsigned)(g > 8192 ? 8192 : g)), dim3(256), 0, st, t, in.words, in.sidx, len,
+                     hist);
+  SRBCRS_STEP(hipGetLastError());
+  g = (rows + 256 * kSweepRankRows - 1) / (256 * kSweepRankRows);
+  int* n_long = reinterpret_cast<int*>(total + 1);
+  hipLaunchKernelGGL(k_sweep_rank, dim3((unsigned)g), dim3(256), 0, st, t, len, hist, hist + kSweepBins, (int)n_lists,
+                     RL, long_bin, in.rowmap, in.M, vrow, out.dest, list_len, lvrow, out.ldest, (int)long_cap, n_long);
+  SRBCRS_STEP(hipGetLastError());
+  const int n8 = (int)(n_lists / 8);
+  hipLaunchKernelGGL(k_sweep_place, dim3((unsigned)((n8 + 63) / 64)), dim3(64), 0, st, list_len, n8, cap, out.start,
+                     out.nblk, out.wblk8, out.wblk4, total);
+  SRBCRS_STEP(hipGetLastError());
+  hipLaunchKernelGGL(k_sweep_place_long, dim3((unsigned)((long_cap + 63) / 64)), dim3(64), 0, st, len, lvrow, n_long,
+                     (int)long_cap, cap, out.lstart, out.lnblk, total);
+  SRBCRS_STEP(hipGetLastError());
+  hipLaunchKernelGGL(k_sweep_fill, dim3((unsigned)((slots + 7) / 8 + (long_cap + 7) / 8)), dim3(64),
+                     32 * out.phases * 4, st, t, in.words, in.sidx, in.packed, vrow, slots, RL, list_len, out.start,
+                     out.nblk, out.phases, out.shift, lvrow, len, out.lstart, out.lnblk, n_long, (int)long_cap,
+                     out.entries);
+  SRBCRS_STEP(hipGetLastError());
+  unsigned long long h_total[2] = {0, 0};
+  SRBCRS_STEP(hipMemcpyAsync(h_total, total, 16, hipMemcpyDeviceToHost, st));
+  SRBCRS_STEP(hipStreamSynchronize(st));
+#undef SRBCRS_STEP
+  out.n_entries = (int64_t)h_total[0];
+  out.n_long = (int)(h_total[1] & 0xffffffffu);
+  return cleanup(out.n_entries <= cap && out.n_long <= long_cap ? hipSuccess : hipErrorInvalidValue);
+}
+
+}  // namespace srbcrs

@@ -4,6 +4,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "srbcrs_kernels.h"
+
 namespace srbcrs {
 
 struct DeviceConvertIn {
@@ -48,5 +50,20 @@ struct CompactOut {
 
 hipError_t device_compact(const float* val, int64_t n_blocks, int blk_h, int blk_w, DeviceAlloc alloc,
                           DeviceFree dfree, void* ctx, hipStream_t st, CompactOut& out);
+
+// Entry stream of the column sweep (srbcrs_colsweep.hip): out's RL, phases and
+// shift are the caller's choice, the rest is filled in; its arrays are allocated through the callback and the caller's to free.
+// hipErrorInvalidValue: the matrix does not fit the stream's 32-bit offsets.
+struct ColSweepIn {
+  ColSweepTasks tasks;
+  const uint2* words;    // compact A
+  const int* sidx;
+  const float* packed;
+  int64_t n_values;      // stored values
+  const int* rowmap;     // packed row -> output row (null = identity)
+  int M;                 // packed rows
+};
+hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc, DeviceFree dfree, void* ctx,
+                          hipStream_t st);
 
 }  // namespace srbcrs

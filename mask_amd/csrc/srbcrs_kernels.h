@@ -112,6 +112,30 @@ int64_t merged_grid(int64_t n_groups, int n_chunks);
 // a.N / 64 column chunks (XCD-pinned when merged_chunks_ok accepts the count).
 hipError_t launch_nzsweep(const NzArgs& z, const StreamArgs& a, int U, int D, hipStream_t st);
 bool nz_setting_ok(int W, int U, int D);
+// The column sweep (srbcrs_colsweep.hpp): its entry stream for one schedule,
+// lists of RL (1, 2, 4 or 8) rows and phases of 2^shift columns.
+struct ColSweep {
+  int RL = 8, phases = 1, shift = 24;
+  int n_lists = 0;        // a multiple of 8
+  int64_t n_entries = 0;
+  uint2* entries = nullptr;
+  int *start = nullptr, *nblk = nullptr, *dest = nullptr;
+  int *wblk8 = nullptr, *wblk4 = nullptr;   // batches per 8 and per 4 lists
+  int n_long = 0;                           // rows outside the lists
+  int *lstart = nullptr, *lnblk = nullptr, *ldest = nullptr;
+};
+struct ColSweepTasks {   // block ranges; window null = window t, slot null = no partial tiles
+  const int *begin, *end, *window, *slot;
+  int n;
+};
+// Rows per list for a launch of N columns over this many task rows: the most
+// that leave 2000 waves (256 CUs hold 5120; below that the lists' chains set
+// the time: 16384 rows of 20, N = 64: 27 us at 8 rows, 22 at 4 or 2).
+int colsweep_rows_per_list(int64_t rows, int N);
+hipError_t launch_colsweep(const ColSweep& s, const StreamArgs& a, int64_t K, unsigned long long token,
+                           unsigned long long* flag, hipStream_t st);
+hipError_t launch_colsweep_repair(const ColSweepTasks& t, const StreamArgs& a, unsigned long long token,
+                                  const unsigned long long* flag, hipStream_t st);
 hipError_t launch_reduce(const ReduceArgs& a, int vec, hipStream_t st);
 hipError_t launch_csr(const CsrArgs& a, int vec, hipStream_t st);
 hipError_t launch_zero_rows(float* C, const int* rows, int n_rows, int N, int64_t ldc, hipStream_t st);

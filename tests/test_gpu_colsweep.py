@@ -1,0 +1,164 @@
+"""The column sweep (the default launch at low block fill, from a plan's
+second run on): the block kernels' bits on every schedule, width and row
+order, infinities and NaNs included, under graph capture and on two streams."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tests.helpers import assert_gate, gate, random_csr
+
+pytestmark = pytest.mark.gpu
+
+# (M, K, columns per row, heavy rows): lists shorter than a wave, one row past a window, several list
+# heights, one and many column phases, rows long enough to leave the lists
+SHAPES = [(1, 300, 200, 0), (17, 3000, 16, 0), (129, 5000, 20, 2), (1025, 20000, 14, 3), (5003, 40011, 13, 5)]
+WIDTHS = [16, 48, 64, 112, 256]
+
+
+def _csr(M, K, per_row, heavy, seed):
+    rng = np.random.default_rng(seed)
+    rows = [np.sort(rng.choice(K, min(K, 2000 if r < heavy else int(rng.integers(per_row // 2, 2 * per_row))),
+                               replace=False)) for r in range(M)]
+    rowptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    colind = np.concatenate(rows).astype(np.int32)
+    return rowptr, colind, rng.uniform(-1, 1, colind.size).astype(np.float32)
+
+
+def _plan(csr, M, **kw):
+    import torch
+    from mask_amd.SRBCRSSpMM import Plan
+    return Plan(*(torch.from_numpy(np.asarray(a)).cuda() for a in csr), M, **kw)
+
+
+def _same(a, b):
+    """Equal bits of value: NaN where NaN, else equal."""
+    import torch
+    na, nb = torch.isnan(a), torch.isnan(b)
+    return torch.equal(na, nb) and torch.equal(a[~na], b[~nb])
+
+
+def _check(plan, B, what, **kw):
+    ref = plan.run(B, grid_order=1, depth=2, wg_cols=128, **kw)
+    for i in range(3):   # the first run may take the block kernel, the later ones the sweep
+        assert _same(plan.run(B, **kw), ref), (what, i)
+    return ref
+
+
+@pytest.mark.parametrize("policy", [("row", 0), ("auto", 0), ("split", 7), ("strict_lb", 9), ("multi_bind", 0)])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_bits_of_the_block_kernels(gpu, shape, policy):
+    import torch
+    M, K, per_row, heavy = shape
+    csr = _csr(M, K, per_row, heavy, M)
+    plan = _plan(csr, M)
+    plan.set_schedule(*policy)
+    for N in WIDTHS:
+        print("[case] colsweep", shape, policy, N, flush=True)
+        B = torch.from_numpy(np.random.default_rng(N).uniform(-1, 1, (K, N)).astype(np.float32)).cuda()
+        C = _check(plan, B, (shape, policy, N))
+        _check(plan, B, (shape, policy, N, "relu"), relu=True)
+    assert_gate(gate(C.cpu().numpy(), *csr, B.cpu().numpy(), M))
+
+
+def test_second_run_builds_the_stream(gpu):
+    """The stream (8 bytes per stored value) is allocated by the second run."""
+    import torch
+    M = K = 60000
+    rng = np.random.default_rng(1)
+    cols = np.sort(rng.integers(0, K // 16, (M, 16)) * 16 + np.arange(16), axis=1)
+    csr = (np.arange(M + 1, dtype=np.int32) * 16, cols.ravel().astype(np.int32),
+           rng.uniform(-1, 1, M * 16).astype(np.float32))
+    plan = _plan(csr, M)
+    B, out = torch.ones((K, 64), device="cuda"), torch.empty((M, 64), device="cuda")
+    free = []
+    for _ in range(3):
+        print("[case] stream build", flush=True)
+        plan.run(B, out)
+        torch.cuda.synchronize()
+        free.append(torch.cuda.mem_get_info()[0])
+    assert free[0] - free[1] >= 8 * M * 16 and free[2] == free[1]
+
+
+@pytest.mark.parametrize("policy", [("row", 0), ("split", 7)])
+def test_non_finite_dense_values(gpu, policy):
+    """An infinity or NaN of B poisons every row of the windows whose blocks
+    hold its column, as in the block kernels: also a column whose only entry
+    is an explicit zero, and one past a list's end; a later finite run is not
+    affected."""
+    import torch
+    M, K, N = 1025, 20000, 64
+    rowptr, colind, values = _csr(M, K, 14, 2, 3)
+    values[5:400:7] = 0.0                     # explicit zeros, dropped from the compact values
+    zero_col = int(colind[5])
+    plan = _plan((rowptr, colind, values), M)
+    plan.set_schedule(*policy)
+    fine = torch.from_numpy(np.random.default_rng(2).uniform(-1, 1, (K, N)).astype(np.float32)).cuda()
+    for cols, v in (((int(colind[700]), zero_col), float("inf")), ((int(colind[-1]),), float("nan")),
+                    ((zero_col,), float("-inf"))):
+        B = fine.clone()
+        B[list(cols), 3] = v
+        B[list(cols), 63] = -v
+        print("[case] non-finite", policy, cols, v, flush=True)
+        ref = _check(plan, B, (cols, v))
+        assert bool(torch.isnan(ref).any())
+        _check(plan, B, (cols, v, "relu"), relu=True)
+        _check(plan, fine, "finite again")
+
+
+@pytest.mark.parametrize("order", ["first_col_sort", "sparse_rows"])
+def test_row_orders_and_strides(gpu, order):
+    import torch
+    M, K, N = 700, 9000, 96
+    csr = random_csr(M, K, 0.002, seed=5, empty_rows=0.2, heavy_rows=2, heavy_len=900)
+    plan = _plan(csr, M, row_order=order, K=K)
+    wide = torch.from_numpy(np.random.default_rng(5).uniform(-1, 1, (K, 131)).astype(np.float32)).cuda()
+    for ldb, ldc in ((96, 96), (100, 104), (131, 96), (96, 101)):   # the last two: the block kernels
+        B = torch.as_strided(wide.flatten()[: K * ldb].clone(), (K, N), (ldb, 1))
+        print("[case] order", order, ldb, ldc, flush=True)
+        ref = plan.run(B, grid_order=1, depth=2, wg_cols=128)
+        for _ in range(3):
+            C = torch.full((M, ldc), 7.0, device="cuda")
+            plan.run(B, C[:, :N])
+            assert torch.equal(C[:, :N], ref) and bool((C[:, N:] == 7.0).all())
+
+
+def test_capture_and_two_streams(gpu):
+    """Captured before and after the stream is built, replays equal the eager
+    results; two streams share one plan, one of them with NaNs."""
+    import torch
+    M, K, N = 3000, 30000, 128
+    csr = _csr(M, K, 15, 3, 9)
+    rng = np.random.default_rng(9)
+    mk = lambda: torch.from_numpy(rng.uniform(-1, 1, (K, N)).astype(np.float32)).cuda()
+    for eager in (1, 2):
+        plan = _plan(csr, M)
+        B, C = mk(), torch.empty((M, N), device="cuda")
+        for _ in range(eager):
+            plan.run(B, C)
+        torch.cuda.synchronize()
+        print("[case] capture after", eager, flush=True)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            plan.run(B, C)
+        for i in range(4):
+            B.copy_(mk())
+            if i == 2:
+                B[int(csr[1][40])] = float("nan")
+            C.fill_(7.0)
+            g.replay()
+            torch.cuda.synchronize()
+            assert _same(C, plan.run(B, grid_order=1, depth=2, wg_cols=128)), (eager, i)
+    B1, B2 = mk(), mk()
+    B2[int(csr[1][40])] = float("nan")
+    r1, r2 = (plan.run(b, grid_order=1, depth=2, wg_cols=128) for b in (B1, B2))
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    print("[case] two streams", flush=True)
+    outs = []
+    for _ in range(20):
+        for s, b in ((s1, B1), (s2, B2)):
+            with torch.cuda.stream(s):
+                outs.append(plan.run(b))
+    torch.cuda.synchronize()
+    assert all(_same(o, (r1, r2)[i % 2]) for i, o in enumerate(outs))
