@@ -217,8 +217,9 @@ int srbcrs_plan_set_schedule(srbcrs_plan *plan, const char *policy, int32_t para
  * K * ldb * 4 < 2^32, and runs from a width's second run on, which builds its
  * entry stream (it allocates 8 bytes per stored value, kept until the plan is
  * destroyed): capture after two eager runs to capture it.  Elsewhere, under
- * capture before that, and on small products, the block kernels run.  A call that is refused (a negative status)
- * has launched nothing and left C untouched. */
+ * capture before that, and on small products, the block kernels run.  A call
+ * that is refused (a negative status) has launched nothing and left C
+ * untouched. */
 int srbcrs_run(srbcrs_plan *plan, const float *d_B, int64_t K, int64_t N, int64_t ldb,
                float *d_C, int64_t ldc, int64_t c_rows, void *stream);
 
@@ -227,8 +228,10 @@ int srbcrs_run(srbcrs_plan *plan, const float *d_B, int64_t K, int64_t N, int64_
  * Retired buffers are what graphs captured on earlier runs may still
  * address: call this only when no such graph will be replayed again and no
  * launch that used them is in flight on another stream.  Without it they
- * are freed with the plan.  No reference counterpart (the reference keeps
- * one global cache entry). */
+ * are freed with the plan.  Also gives back to the driver the device memory
+ * that destroyed plans and conversions have left (kept, up to 4 GiB a
+ * process, for the next ones).  No reference counterpart (the reference
+ * keeps one global cache entry). */
 int srbcrs_plan_trim(srbcrs_plan *plan, void *stream);
 
 /* Launch knobs of the SR-BCRS kernels (template parameters; each maps a

@@ -23,6 +23,7 @@
 #include "srbcrs_kernels.h"
 #include "srbcrs_convert.h"
 #include "srbcrs_pack.h"
+#include "srbcrs_pool.h"
 #include "srbcrs_probe.h"
 
 namespace {
@@ -379,19 +380,16 @@ Schedule* build_schedule(const int32_t* soff, int32_t Mo, const char* policy_c, 
 
 template <class T>
 T* dev_alloc(size_t n) {
-  void* p = nullptr;
   if (n == 0) n = 1;
-  hipError_t e = hipMalloc(&p, n * sizeof(T));
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    fail(SRBCRS_ENOMEM, "hipMalloc(%zu bytes) failed: %s", n * sizeof(T), hipGetErrorString(e));
-  }
+  void* p = srbcrs::pool_alloc(n * sizeof(T));
+  if (!p) fail(SRBCRS_ENOMEM, "allocation of %zu bytes of device memory failed", n * sizeof(T));
   return static_cast<T*>(p);
 }
 
+// no queued work may use p any more
 template <class T>
 void dev_free(T*& p) {
-  if (p) (void)hipFree(p);
+  srbcrs::pool_free(p);
   p = nullptr;
 }
 
@@ -501,7 +499,18 @@ struct srbcrs_plan {
     if (hipGetDevice(&cur) == hipSuccess && cur != device) switched = hipSetDevice(device) == hipSuccess;
     retire_schedule();
     retire(d_partial);
-    for (void* p : retired) (void)hipFree(p);
+    // the memory may be handed to another plan, thread or stream at once:
+    // wait for everything that could still use it (hipFree waits as well)
+    const bool idle = hipDeviceSynchronize() == hipSuccess;
+    if (!idle) (void)hipGetLastError();
+    auto dev_free = [&](auto*& p) {
+      if (idle)
+        srbcrs::pool_free(p);
+      else
+        srbcrs::pool_drop(p);
+      p = nullptr;
+    };
+    for (void* p : retired) dev_free(p);
     dev_free(d_soff);
     dev_free(d_sidx);
     dev_free(d_val);
@@ -635,18 +644,11 @@ void create_packed(srbcrs_plan& plan, const int32_t* rp, const int32_t* ci, cons
   plan.sched.policy = "row";
 }
 
-void* conv_alloc(void*, size_t bytes) {
-  void* p = nullptr;
-  if (hipMalloc(&p, bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  return p;
-}
+void* conv_alloc(void*, size_t bytes) { return srbcrs::pool_alloc(bytes); }
+void conv_free(void*, void* p) { srbcrs::pool_free(p); }
 
-void conv_free(void*, void* p) { (void)hipFree(p); }
-
-// Canonical conversion of a device CSR on the device (srbcrs_convert.hip).
+// Canonical conversion of a device CSR on the device (srbcrs_convert.hip),
+// with the compact copy of the block values where there is room for it.
 void create_on_device(srbcrs_plan& plan, const int32_t* rowptr, const int32_t* colind,
                       const float* values, hipStream_t st) {
   const int32_t Mo = (plan.num_nodes + plan.blk_h - 1) / plan.blk_h;
@@ -655,26 +657,23 @@ void create_on_device(srbcrs_plan& plan, const int32_t* rowptr, const int32_t* c
   plan.d_e2r = dev_alloc<int32_t>((size_t)plan.nnz);
   plan.d_e2c = dev_alloc<int32_t>((size_t)plan.nnz);
   plan.d_bp = dev_alloc<int32_t>((size_t)Mo);
-  if (plan.nnz) {
-    hip_check(hipMemsetAsync(plan.d_e2r, 0, (size_t)plan.nnz * 4, st), "hipMemsetAsync");
-    hip_check(hipMemsetAsync(plan.d_e2c, 0, (size_t)plan.nnz * 4, st), "hipMemsetAsync");
-  }
+  plan.h_soff.resize((size_t)Mo + 1);
   srbcrs::DeviceConvertIn in{rowptr, colind, values, plan.num_nodes, plan.nnz, plan.blk_h, plan.blk_w,
                              plan.d_e2r, plan.d_e2c, plan.d_bp};
   srbcrs::DeviceConvertOut out;
   out.soff = plan.d_soff;
+  out.h_soff = plan.h_soff.data();
   const hipError_t e = srbcrs::device_convert(in, out, conv_alloc, conv_free, nullptr, st);
   plan.d_sidx = out.sidx;   // owned by the plan from here on, even on failure
   plan.d_val = out.val;
+  plan.d_awords = out.compact.words;
+  plan.d_apacked = out.compact.packed;
+  plan.n_apacked = out.compact.n_packed;
   hip_check(e, "device conversion");
   if (out.bad == 1) fail(SRBCRS_EINVAL, "rowptr must be non-decreasing and within [0, nnz]");
   if (out.bad == 2) fail(SRBCRS_EINVAL, "colind holds a negative column index");
   plan.total = out.total;
   plan.max_col = out.max_col;
-  plan.h_soff.resize((size_t)Mo + 1);
-  hip_check(hipMemcpyAsync(plan.h_soff.data(), plan.d_soff, plan.h_soff.size() * 4, hipMemcpyDeviceToHost, st),
-            "copy soff");
-  hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
   plan.sched.policy = "row";
 }
 
@@ -817,8 +816,8 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
   s.phases = (plan.max_col >> s.shift) + 1;
   hipError_t e = hipSuccess;
   if (!plan.d_sweep_flags) {
-    e = hipMalloc(reinterpret_cast<void**>(&plan.d_sweep_flags), kSweepFlags * 8);
-    if (e == hipSuccess) e = hipMemsetAsync(plan.d_sweep_flags, 0, kSweepFlags * 8, st);
+    plan.d_sweep_flags = static_cast<unsigned long long*>(srbcrs::pool_alloc(kSweepFlags * 8));
+    e = plan.d_sweep_flags ? hipMemsetAsync(plan.d_sweep_flags, 0, kSweepFlags * 8, st) : hipErrorOutOfMemory;
   }
   srbcrs::ColSweepIn in{t, plan.d_awords, plan.d_sidx, plan.d_apacked, plan.n_apacked, plan.d_rowmap,
                         (int)plan.packed_rows};
@@ -1092,7 +1091,6 @@ int srbcrs_plan_create_ex(const int32_t* rowptr, const int32_t* colind, const fl
       plan->canonical = true;
       plan->packed_rows = num_nodes;
       create_on_device(*plan, rowptr, colind, values, st);
-      build_compact(*plan, st);
       *out = plan.release();
       return;
     }
@@ -1647,8 +1645,9 @@ int srbcrs_plan_trim(srbcrs_plan* plan, void* stream) {
     // every launch that could still read a retired buffer was queued on this
     // stream (or on work the caller has already waited for)
     hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream)), "hipStreamSynchronize");
-    for (void* p : plan->retired) (void)hipFree(p);
+    for (void* p : plan->retired) srbcrs::pool_drop(p);
     plan->retired.clear();
+    srbcrs::pool_release(plan->device);
   });
 }
 

@@ -135,6 +135,7 @@ hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc
     p = nullptr;
   };
   auto cleanup = [&](hipError_t e) {
+    if (e != hipSuccess) (void)hipStreamSynchronize(st);   // queued kernels may use what is given back
     drop(len);
     drop(hist);
     drop(vrow);

@@ -91,6 +91,7 @@ hipError_t device_compact(const float* val, int64_t n_blocks, int blk_h, int blk
     if (tail) dfree(ctx, tail);
   };
   auto fail = [&](hipError_t e) {
+    (void)hipStreamSynchronize(st);   // queued kernels may use what is given back
     cleanup();
     if (out.words) dfree(ctx, out.words);
     if (out.packed) dfree(ctx, out.packed);

@@ -15,26 +15,10 @@ struct DeviceConvertIn {
   int num_nodes;
   int64_t nnz;
   int blk_h, blk_w;
-  int* edge_to_row;        // device, nnz (required; caller zero-fills it)
-  int* edge_to_col;        // device, nnz or null (caller zero-fills it)
+  int* edge_to_row;        // device, nnz (required)
+  int* edge_to_col;        // device, nnz or null
   int* block_partition;    // device, Mo or null
 };
-
-struct DeviceConvertOut {
-  int* soff;               // device, Mo + 1, allocated by the caller
-  int* sidx = nullptr;     // allocated through the callback
-  float* val = nullptr;    // allocated through the callback
-  int Mo = 0;
-  int64_t total = 0;
-  int max_col = -1;
-  int bad = 0;             // 1: malformed rowptr, 2: negative column (nothing else produced)
-};
-
-typedef void* (*DeviceAlloc)(void* ctx, size_t bytes);
-typedef void (*DeviceFree)(void* ctx, void* p);
-
-hipError_t device_convert(const DeviceConvertIn& in, DeviceConvertOut& out, DeviceAlloc alloc,
-                          DeviceFree dfree, void* ctx, hipStream_t st);
 
 // Compact copy of the block values (srbcrs_compact.hip): per 32 logical
 // positions of a block one {mask, base} word, and the stored values.
@@ -48,11 +32,31 @@ struct CompactOut {
   int64_t n_packed = 0;
 };
 
+struct DeviceConvertOut {
+  int* soff;               // device, Mo + 1, allocated by the caller
+  int* h_soff;             // host, Mo + 1, allocated by the caller
+  int* sidx = nullptr;     // allocated through the callback
+  float* val = nullptr;    // allocated through the callback
+  CompactOut compact;      // allocated through the callback (null: no room)
+  int Mo = 0;
+  int64_t total = 0;
+  int max_col = -1;
+  int bad = 0;             // 1: malformed rowptr, 2: negative column (nothing else produced)
+};
+
+typedef void* (*DeviceAlloc)(void* ctx, size_t bytes);
+typedef void (*DeviceFree)(void* ctx, void* p);   // called when no queued work uses p any more
+
+// Returns with the stream's work done.
+hipError_t device_convert(const DeviceConvertIn& in, DeviceConvertOut& out, DeviceAlloc alloc,
+                          DeviceFree dfree, void* ctx, hipStream_t st);
+
 hipError_t device_compact(const float* val, int64_t n_blocks, int blk_h, int blk_w, DeviceAlloc alloc,
                           DeviceFree dfree, void* ctx, hipStream_t st, CompactOut& out);
 
 // Entry stream of the column sweep (srbcrs_colsweep.hip): out's RL, phases and
-// shift are the caller's choice, the rest is filled in; its arrays are allocated through the callback and the caller's to free.
+// shift are the caller's choice, the rest is filled in; its arrays are
+// allocated through the callback and the caller's to free.
 // hipErrorInvalidValue: the matrix does not fit the stream's 32-bit offsets.
 struct ColSweepIn {
   ColSweepTasks tasks;

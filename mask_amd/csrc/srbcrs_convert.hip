@@ -4,13 +4,24 @@
 // SRBCRSSpMM_kernel.cu:226-340): per BH-row window the sorted distinct
 // columns, cut into BW-column blocks padded with the window's last column;
 // values at the swizzled block offset, the last write winning for duplicate
-// (row, column) pairs; edge_to_row / edge_to_col / block_partition.
+// (row, column) pairs; edge_to_row / edge_to_col / block_partition; and the
+// compact copy of the block values (srbcrs_compact.hip).
 //
-// The reference copies the CSR to the host and converts there.  Here the CSR
-// stays in HBM: edges are keyed (window << 32 | column), radix-sorted with
-// their edge index (stable, so duplicates keep edge order), and the distinct
-// keys are ranked with a scan.  Every write has a single owner (no atomics):
-// a duplicate run's last entry writes the value.
+// A window's edges are contiguous in the CSR, so nothing needs a sort of the
+// whole matrix: one workgroup sorts a window's (column, edge) keys in LDS,
+// ranks the distinct columns and counts the stored values; a scan over the
+// windows gives the block offsets; then 16 lanes (16x8) or a wave (32x32) per
+// block write the block whole -- indices, mask words, stored values and the
+// dense values, each byte once.  Every write has a single owner.
+//
+// Bound: the dense values, 512 bytes a block, written once (11.7 M edges of a
+// power-law graph, 232965 rows, 1.4 M blocks: 0.71 GB of 0.95 GB moved, 190 us
+// at the rate of a copy).  Measured on that graph (one MI355X): the windows 460
+// us, the sort, ranks and second scan of the 15 windows longer than LDS holds
+// 350, blocks 380, scan 21; the whole call 1.40 ms.  Sorting the whole matrix
+// by (window, column, edge) with a device-wide sort, writing the blocks entry
+// by entry over a fill, and copying the stored values out in a pass of their
+// own took 43.5 ms; on 5000 rows with a product 535 us, now 203.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 #include <stdint.h>
@@ -23,138 +34,498 @@ namespace {
 
 __device__ __forceinline__ int swz(int o) { return o ^ ((o & 0x60) >> 3); }
 
-// flag[0] = 1 when the CSR is malformed (rowptr decreasing / out of range,
-// negative column); flag[1] = max column (as int, -1 if none).
-__global__ void k_validate_rowptr(const int* __restrict__ rowptr, int num_nodes, int64_t nnz,
-                                  int* __restrict__ flag) {
-  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r <= num_nodes;
-       r += (int64_t)gridDim.x * blockDim.x) {
-    const int v = rowptr[r];
-    bool bad = v < 0 || v > nnz;
-    if (r < num_nodes && rowptr[r + 1] < v) bad = true;
-    if (bad) flag[0] = 1;   // plain store: every writer writes the same value
+// What the host needs back before it can size the arrays, and the counters of
+// the windows too long for one workgroup's LDS.
+struct Head {
+  unsigned long long totals;       // blocks | stored values << 32
+  unsigned long long big_entries;
+  int bad, negative;
+  int max_col1;                    // largest column + 1 (all zero at the start)
+  int n_list[2], n_big;            // windows listed for k_listed_windows<0 / 1>, and longer ones
+};
+
+// Per sorted entry (at its window's edge range): what the block pass reads.
+struct Sorted {
+  int* col;         // its column
+  float* val;       // its value
+  int* rank;        // rank of its column among the window's distinct ones
+  int* stored;      // stored values of the window before it
+  int* block;       // [e0 + j]: the window's first entry of block j
+  uint8_t* row;     // row in the window, bit 7: the last of its (row, column) run
+};
+
+struct ConvArgs {
+  const int* rowptr;
+  const int* colind;
+  const float* values;
+  int num_nodes;
+  int64_t nnz;
+  int bh, bw;
+  int *e2r, *e2c, *bp;   // e2c, bp may be null
+  Sorted s;
+  unsigned long long* wcount;   // per window: blocks | stored values << 32
+  int *list[2], *big;           // windows of the longer classes
+  Head* head;
+};
+
+// Entries of a window sorted in LDS: by 256, 512 and 1024 threads.
+constexpr int kClass[3] = {2048, 4096, 16384};
+
+__device__ __forceinline__ void note_max(int* p, int v) {
+  if (v > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p, v);
+}
+
+// Row of edge e in a window whose row offsets are rp[0..rows].
+__device__ __forceinline__ int row_of(const int* rp, int rows, int e) {
+  int lo = 0, hi = rows;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) / 2;
+    if (rp[mid] <= e) lo = mid; else hi = mid;
+  }
+  return lo;
+}
+
+// Inclusive scan over the workgroup; total in every thread.
+template <int T>
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* part, uint32_t& total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t x = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t y = __shfl_up(x, d);
+    if (lane >= d) x += y;
+  }
+  __syncthreads();
+  if (lane == 63) part[wave] = x;
+  __syncthreads();
+  uint32_t before = 0;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < T / 64; ++w) {
+    if (w < wave) before += part[w];
+    total += part[w];
+  }
+  return before + x;
+}
+
+// Stable sort of n <= T * IPT keys by their high word, of `bits` bits: radix
+// passes of up to 8 bits, in LDS.  A wave owns a contiguous run of keys, so
+// rank = keys of lower digits, of the same digit in earlier waves, and of the
+// same digit before it in its wave (lanes with the digit found by ballots).
+// The keys wait in registers while the counts are summed, so one copy in LDS
+// is enough.  (A bitonic sort moved each key through LDS 55 to 105 times and
+// was bound by that: on the graph above 960 us, the radix passes 460.)
+template <int T, int IPT>
+__device__ __forceinline__ void radix_sort(uint64_t* key, int n, int bits, uint32_t* hist, uint32_t* part) {
+  constexpr int W = T / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t below = (1ull << lane) - 1ull;
+  const int iters = (n + W * 64 - 1) / (W * 64);   // 64-key steps per wave
+  const int first = wave * iters * 64 + lane;
+  const int passes = (bits + 7) / 8, width = (bits + passes - 1) / passes;
+  for (int shift = 0; shift < bits; shift += width) {
+    const int digits = 1 << width;
+    for (int i = threadIdx.x; i < digits * W; i += T) hist[i] = 0;
+    __syncthreads();
+    uint64_t k[IPT];
+    uint32_t rank[IPT];
+#pragma unroll
+    for (int it = 0; it < IPT; ++it) {
+      if (it < iters) {
+        const int i = first + it * 64;
+        const bool valid = i < n;
+        k[it] = valid ? key[i] : 0;
+        const uint32_t d = (uint32_t)(k[it] >> (32 + shift)) & (uint32_t)(digits - 1);
+        uint64_t same = __ballot(valid);
+        for (int b = 0; b < width; ++b) {
+          const uint64_t ones = __ballot((d >> b) & 1u);
+          same &= ((d >> b) & 1u) ? ones : ~ones;
+        }
+        // hist is digit-major: [digit][wave]
+        const uint32_t before = valid ? hist[d * W + wave] : 0;
+        rank[it] = before + (uint32_t)__popcll(same & below);
+        __builtin_amdgcn_wave_barrier();
+        if (valid && (same & below) == 0) hist[d * W + wave] = before + (uint32_t)__popcll(same);
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+    __syncthreads();
+    // exclusive sums in (digit, wave) order
+    const int per = digits * W / T > 0 ? digits * W / T : 1;
+    uint32_t sum = 0, total;
+    const int e0 = threadIdx.x * per;
+    for (int e = e0; e < e0 + per && e < digits * W; ++e) sum += hist[e];
+    uint32_t at = block_scan<T>(sum, part, total) - sum;
+    for (int e = e0; e < e0 + per && e < digits * W; ++e) {
+      const uint32_t c = hist[e];
+      hist[e] = at;
+      at += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IPT; ++it) {
+      if (it < iters && first + it * 64 < n) {
+        const uint32_t d = (uint32_t)(k[it] >> (32 + shift)) & (uint32_t)(digits - 1);
+        key[hist[d * W + wave] + rank[it]] = k[it];
+      }
+    }
+    __syncthreads();
   }
 }
 
-// Row ids of the edges in two parallel passes (a per-row loop serialises on
-// hub rows): each non-empty row marks its first edge (one writer per edge:
-// rows with the same start are empty but the last), then an inclusive max
-// scan over the zero-filled edge range carries each mark forward.
-__global__ void k_row_starts(const int* __restrict__ rowptr, int num_nodes, int* __restrict__ e2r) {
-  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < num_nodes;
-       r += (int64_t)gridDim.x * blockDim.x)
-    if (rowptr[r + 1] > rowptr[r]) e2r[rowptr[r]] = (int)r;
+// Tile of sorted keys -> ranks, stored counts and the per-entry outputs.
+// col(i) / edge(i): sorted entry i of the window; first and stored carry the
+// window's counts over the tiles before this one.
+template <int T, class Col, class Edge>
+__device__ __forceinline__ void rank_tile(const ConvArgs& a, const int* rp, int rows, int n, int i0,
+                                          uint32_t& firsts, uint32_t& stored, uint32_t* part, Col col, Edge edge) {
+  const int e0 = rp[0];
+  const int i = i0 + (int)threadIdx.x;
+  uint32_t flag = 0;
+  int c = 0, e = 0, row = 0;
+  float v = 0.f;
+  bool last = false;
+  if (i < n) {
+    c = col(i);
+    e = edge(i);
+    row = row_of(rp, rows, e);
+    const bool first = i == 0 || col(i - 1) != c;
+    last = i + 1 == n || col(i + 1) != c || row_of(rp, rows, edge(i + 1)) != row;
+    v = a.values[e];
+    flag = (first ? 1u : 0u) | (last && __float_as_uint(v) != 0u ? 1u << 16 : 0u);
+  }
+  uint32_t total;
+  const uint32_t incl = block_scan<T>(flag, part, total);
+  if (i < n) {
+    const int p = (int)(firsts + (incl & 0xffffu)) - 1;
+    const int64_t at = (int64_t)e0 + i;
+    a.s.col[at] = c;
+    a.s.val[at] = v;
+    a.s.rank[at] = p;
+    a.s.stored[at] = (int)(stored + ((incl - flag) >> 16));
+    a.s.row[at] = (uint8_t)(row | (last ? 0x80 : 0));
+    if ((flag & 1u) && p % a.bw == 0) a.s.block[(int64_t)e0 + p / a.bw] = i;
+    if (a.e2c) a.e2c[e] = p;
+  }
+  firsts += total & 0xffffu;
+  stored += total >> 16;
 }
 
-__global__ void k_make_keys(const int* __restrict__ colind, const int* __restrict__ e2r, int e0,
-                            int n, int bh, uint64_t* __restrict__ keys, int* __restrict__ idx,
-                            int* __restrict__ neg) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int e = e0 + (int)i;
-    const int c = colind[e];
-    if (c < 0) neg[0] = 1;
-    keys[i] = ((uint64_t)(uint32_t)(e2r[e] / bh) << 32) | (uint32_t)c;
-    idx[i] = e;
+__device__ __forceinline__ void put_count(const ConvArgs& a, int w, uint32_t firsts, uint32_t stored) {
+  const uint32_t nb = (firsts + (uint32_t)a.bw - 1) / (uint32_t)a.bw;
+  a.wcount[w] = (unsigned long long)nb | ((unsigned long long)stored << 32);
+  if (a.bp) a.bp[w] = (int)nb;
+}
+
+// The window's row offsets into LDS; false (and head->bad) if they are not
+// non-decreasing within [0, nnz].  Nothing of such a window is read.
+__device__ __forceinline__ bool window_rows(const ConvArgs& a, int w, int* rp, int& rows) {
+  const int64_t r0 = (int64_t)w * a.bh;
+  rows = (int)(r0 + a.bh < a.num_nodes ? a.bh : a.num_nodes - r0);
+  __syncthreads();   // rp may still be read for the workgroup's previous window
+  bool bad = false;
+  if ((int)threadIdx.x <= rows) {
+    const int v = a.rowptr[r0 + threadIdx.x];
+    rp[threadIdx.x] = v;
+    bad = v < 0 || v > a.nnz || ((int)threadIdx.x < rows && a.rowptr[r0 + threadIdx.x + 1] < v);
+  }
+  if (__syncthreads_or(bad)) {
+    if (threadIdx.x == 0) {
+      a.head->bad = 1;   // every writer writes the same value
+      a.wcount[w] = 0;
+    }
+    return false;
+  }
+  return true;
+}
+
+// Sort and rank one window of n <= T * IPT entries.
+template <int T, int IPT>
+__device__ __forceinline__ void sort_window(const ConvArgs& a, int w, const int* rp, int rows, int n, uint64_t* key,
+                                            uint32_t* hist, uint32_t* part, int* most) {
+  const int e0 = rp[0];
+  if (threadIdx.x == 0) *most = 0;
+  __syncthreads();
+  int mx = 0;
+  for (int i = threadIdx.x; i < n; i += T) {
+    const int c = a.colind[e0 + i];
+    mx = max(mx, c < 0 ? INT32_MAX : c);   // a negative column sorts past the others
+    if (c < 0) a.head->negative = 1;
+    key[i] = ((uint64_t)(uint32_t)c << 32) | (uint32_t)i;
+    a.e2r[e0 + i] = w * a.bh + row_of(rp, rows, e0 + i);
+  }
+#pragma unroll
+  for (int d = 32; d; d >>= 1) mx = max(mx, __shfl_xor(mx, d));
+  if ((threadIdx.x & 63) == 0) atomicMax(most, mx);
+  __syncthreads();
+  radix_sort<T, IPT>(key, n, 32 - __builtin_clz(*most | 1), hist, part);
+  uint32_t firsts = 0, stored = 0;
+  for (int i0 = 0; i0 < n; i0 += T)
+    rank_tile<T>(a, rp, rows, n, i0, firsts, stored, part, [&](int i) { return (int)(key[i] >> 32); },
+                 [&](int i) { return e0 + (int)(uint32_t)key[i]; });
+  if (threadIdx.x == 0) {
+    put_count(a, w, firsts, stored);
+    note_max(&a.head->max_col1, *most < INT32_MAX ? *most + 1 : INT32_MAX);
   }
 }
 
-__global__ void k_flags(const uint64_t* __restrict__ keys, int n, int* __restrict__ flags) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    flags[i] = (i == 0 || keys[i] != keys[i - 1]) ? 1 : 0;
-}
-
-// rank[i] = inclusive count of distinct keys up to i (1-based)
-__global__ void k_unique(const uint64_t* __restrict__ keys, const int* __restrict__ rank, int n,
-                         int* __restrict__ ucol, int* __restrict__ uwin) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    if (i == 0 || keys[i] != keys[i - 1]) {
-      const int u = rank[i] - 1;
-      ucol[u] = (int)(uint32_t)keys[i];
-      uwin[u] = (int)(keys[i] >> 32);
+// One window per workgroup; the longer ones are listed for the other passes.
+__global__ __launch_bounds__(256) void k_windows(ConvArgs a) {
+  __shared__ uint64_t key[kClass[0]];
+  __shared__ uint32_t hist[256 * 4], part[4];
+  __shared__ int rp[33], most;
+  const int w = blockIdx.x;
+  int rows;
+  if (!window_rows(a, w, rp, rows)) return;
+  const int n = rp[rows] - rp[0];
+  if (n == 0) {
+    if (threadIdx.x == 0) put_count(a, w, 0, 0);
+  } else if (n <= kClass[0]) {
+    sort_window<256, kClass[0] / 256>(a, w, rp, rows, n, key, hist, part, &most);
+  } else if (threadIdx.x == 0) {
+    a.wcount[w] = 0;
+    if (n <= kClass[2]) {
+      const int q = n <= kClass[1] ? 0 : 1;
+      a.list[q][atomicAdd(&a.head->n_list[q], 1)] = w;
+    } else {
+      a.big[atomicAdd(&a.head->n_big, 1)] = w;
+      atomicAdd(&a.head->big_entries, (unsigned long long)n);
     }
   }
 }
 
-// ufirst[w] = first distinct-key index of window w (lower bound), w in [0, Mo]
-__global__ void k_window_first(const int* __restrict__ uwin, int nu, int Mo, int* __restrict__ ufirst) {
-  for (int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; w <= Mo;
-       w += (int64_t)gridDim.x * blockDim.x) {
-    int lo = 0, hi = nu;
-    while (lo < hi) {
-      const int mid = lo + (hi - lo) / 2;
-      if (uwin[mid] < w) lo = mid + 1; else hi = mid;
+template <int Q>
+__global__ __launch_bounds__(Q ? 1024 : 512) void k_listed_windows(ConvArgs a) {
+  constexpr int T = Q ? 1024 : 512, CAP = kClass[Q + 1];
+  __shared__ uint64_t key[CAP];
+  __shared__ uint32_t hist[256 * (T / 64)], part[T / 64];
+  __shared__ int rp[33], most;
+  for (int i = blockIdx.x; i < a.head->n_list[Q]; i += gridDim.x) {
+    const int w = a.list[Q][i];
+    int rows;
+    if (!window_rows(a, w, rp, rows)) continue;
+    sort_window<T, CAP / T>(a, w, rp, rows, rp[rows] - rp[0], key, hist, part, &most);
+    __syncthreads();
+  }
+}
+
+// First key of each of the longest windows in the concatenation of theirs.
+__global__ __launch_bounds__(64) void k_big_offsets(ConvArgs a, int64_t* __restrict__ off) {
+  const int lane = threadIdx.x, n_big = a.head->n_big;
+  int64_t at = 0;
+  for (int b0 = 0; b0 < n_big; b0 += 64) {
+    const int b = b0 + lane;
+    int64_t n = 0;
+    if (b < n_big) {
+      const int64_t r0 = (int64_t)a.big[b] * a.bh;
+      n = a.rowptr[r0 + a.bh < a.num_nodes ? r0 + a.bh : a.num_nodes] - a.rowptr[r0];
     }
-    ufirst[w] = lo;
+    int64_t incl = n;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t x = __shfl_up(incl, d);
+      if (lane >= d) incl += x;
+    }
+    if (b < n_big) off[b] = at + incl - n;
+    at += __shfl(incl, 63);
   }
 }
 
-__global__ void k_block_counts(const int* __restrict__ ufirst, int Mo, int bw, int* __restrict__ nb,
-                               int* __restrict__ bp) {
-  for (int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; w <= Mo;
-       w += (int64_t)gridDim.x * blockDim.x) {
-    const int c = w < Mo ? (ufirst[w + 1] - ufirst[w] + bw - 1) / bw : 0;
-    nb[w] = c;
-    if (bp && w < Mo) bp[w] = c;
-  }
-}
-
-// sidx slot s (block b = s / bw): window by upper bound in soff, then the
-// window's distinct column at min(position, count - 1)
-__global__ void k_fill_sidx(const int* __restrict__ soff, const int* __restrict__ ufirst,
-                            const int* __restrict__ ucol, int Mo, int bw, int64_t nslots,
-                            int* __restrict__ sidx) {
-  for (int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; s < nslots;
-       s += (int64_t)gridDim.x * blockDim.x) {
-    const int b = (int)(s / bw);
-    int lo = 0, hi = Mo;   // last w with soff[w] <= b
+// Windows too long for LDS: (index in a.big << 32 | column) keys of all of
+// them, one after the other, for one device-wide stable sort.
+__global__ __launch_bounds__(256) void k_big_keys(ConvArgs a, const int64_t* __restrict__ off,
+                                                  uint64_t* __restrict__ keys, int* __restrict__ edges) {
+  const int b = blockIdx.y, w = a.big[b];
+  const int64_t r0 = (int64_t)w * a.bh;
+  const int64_t r1 = r0 + a.bh < a.num_nodes ? r0 + a.bh : a.num_nodes;
+  const int e0 = a.rowptr[r0], n = a.rowptr[r1] - e0;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+    const int c = a.colind[e0 + i];
+    if (c < 0) a.head->negative = 1;
+    keys[off[b] + i] = ((uint64_t)(uint32_t)b << 32) | (uint32_t)c;
+    edges[off[b] + i] = e0 + i;
+    int lo = 0, hi = (int)(r1 - r0);
     while (hi - lo > 1) {
-      const int mid = lo + (hi - lo) / 2;
-      if (soff[mid] <= b) lo = mid; else hi = mid;
+      const int mid = (lo + hi) / 2;
+      if (a.rowptr[r0 + mid] <= e0 + i) lo = mid; else hi = mid;
     }
-    const int w = lo;   // the window holding block b (empty windows have soff[w] == soff[w+1])
-    const int64_t pos = s - (int64_t)soff[w] * bw;
-    const int cnt = ufirst[w + 1] - ufirst[w];
-    sidx[s] = ucol[ufirst[w] + (pos < cnt ? (int)pos : cnt - 1)];
+    a.e2r[e0 + i] = (int)r0 + lo;
   }
 }
 
-__global__ void k_zero(float* __restrict__ p, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = 0.f;
+__global__ __launch_bounds__(1024) void k_big_rank(ConvArgs a, const int64_t* __restrict__ off,
+                                                   const uint64_t* __restrict__ keys, const int* __restrict__ edges) {
+  __shared__ uint32_t part[16];
+  __shared__ int rp[33];
+  const int b = blockIdx.x, w = a.big[b];
+  int rows;
+  if (!window_rows(a, w, rp, rows)) return;
+  const int n = rp[rows] - rp[0];
+  const uint64_t* k = keys + off[b];
+  const int* ed = edges + off[b];
+  uint32_t firsts = 0, stored = 0;
+  for (int i0 = 0; i0 < n; i0 += 1024)
+    rank_tile<1024>(a, rp, rows, n, i0, firsts, stored, part, [&](int i) { return (int)(uint32_t)k[i]; },
+                    [&](int i) { return ed[i]; });
+  if (threadIdx.x == 0) {
+    put_count(a, w, firsts, stored);
+    const int c = (int)(uint32_t)k[n - 1];
+    note_max(&a.head->max_col1, c < INT32_MAX ? c + 1 : c);
+  }
 }
 
-__global__ void k_scatter(const uint64_t* __restrict__ keys, const int* __restrict__ idx,
-                          const int* __restrict__ rank, int n, const int* __restrict__ e2r,
-                          const float* __restrict__ values, const int* __restrict__ ufirst,
-                          const int* __restrict__ soff, int bh, int bw, float* __restrict__ val,
-                          int* __restrict__ e2c) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int e = idx[i];
-    const int w = (int)(keys[i] >> 32);
-    const int p = rank[i] - 1 - ufirst[w];
-    if (e2c) e2c[e] = p;
-    const int row = e2r[e];
-    // last entry of its (row, column) run: entries of one key are in edge
-    // order and a row's edges are contiguous, so the run ends where the key
-    // or the row changes
-    const bool last = i + 1 == n || keys[i + 1] != keys[i] || e2r[idx[i + 1]] != row;
-    if (last) {
-      const int lr = row - w * bh;
-      val[((int64_t)soff[w] + p / bw) * bh * bw + swz(lr * bw + p % bw)] = values[e];
+// Exclusive sums over the windows (one workgroup): block offsets and the
+// index of each window's first stored value.  Also zeroes the edge maps of
+// edges outside rows [0, num_nodes).
+__global__ __launch_bounds__(1024) void k_window_scan(ConvArgs a, int Mo, int* __restrict__ soff,
+                                                      unsigned* __restrict__ vbase) {
+  __shared__ unsigned long long part[16];
+  constexpr int PER = 8;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  unsigned long long carry = 0;
+  for (int64_t base = 0; base < Mo; base += 1024 * PER) {
+    unsigned long long v[PER], sum = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int64_t w = base + (int64_t)threadIdx.x * PER + i;
+      v[i] = w < Mo ? a.wcount[w] : 0;
+      sum += v[i];
+    }
+    unsigned long long x = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const unsigned long long y = __shfl_up(x, d);
+      if (lane >= d) x += y;
+    }
+    __syncthreads();
+    if (lane == 63) part[wave] = x;
+    __syncthreads();
+    unsigned long long at = carry + x - sum;
+    for (int q = 0; q < 16; ++q) {
+      if (q < wave) at += part[q];
+      carry += part[q];
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int64_t w = base + (int64_t)threadIdx.x * PER + i;
+      if (w < Mo) {
+        soff[w] = (int)(at & 0xffffffffu);
+        vbase[w] = (unsigned)(at >> 32);
+      }
+      at += v[i];
+    }
+  }
+  if (threadIdx.x == 0) {
+    soff[Mo] = (int)(carry & 0xffffffffu);
+    a.head->totals = carry;
+  }
+  if (!a.head->bad) {
+    const int64_t lo = a.rowptr[0], hi = a.rowptr[a.num_nodes];
+    for (int64_t e = threadIdx.x; e < lo + (a.nnz - hi); e += 1024) {
+      const int64_t q = e < lo ? e : hi + (e - lo);
+      a.e2r[q] = 0;
+      if (a.e2c) a.e2c[q] = 0;
     }
   }
 }
 
-inline unsigned grid_for(int64_t n) {
-  int64_t b = (n + 255) / 256;
-  if (b < 1) b = 1;
-  if (b > 65536) b = 65536;
-  return (unsigned)b;
+// The blocks: G lanes each, kBlockSteps * 256 / G per workgroup.  Entries of
+// one block are contiguous in the sorted order; the lanes drop their values
+// into an LDS copy of the block, which then goes out whole.  The workgroup
+// finds the window of its first block by a 256-way search (two dependent
+// loads; with a binary search per block, 14 of them, 1.4 M blocks took 574 us,
+// now 381: 2.2 TB/s, the latency of the entries' loads).
+constexpr int kBlockSteps = 4;
+template <int BH, int BW, int G>
+__global__ __launch_bounds__(256) void k_blocks(ConvArgs a, int Mo, const int* __restrict__ soff,
+                                                const unsigned* __restrict__ vbase, int64_t n_blocks,
+                                                int* __restrict__ sidx, float* __restrict__ val,
+                                                uint2* __restrict__ words, float* __restrict__ packed) {
+  constexpr int SIZE = BH * BW, WORDS = SIZE / 32, PER_WG = 256 / G, PER = SIZE / G;
+  __shared__ __attribute__((aligned(16))) float tile[PER_WG][SIZE];
+  __shared__ uint32_t mask[PER_WG][WORDS];
+  __shared__ int cols[PER_WG][BW];
+  __shared__ int off[257];   // soff from the first block's window on
+  const int g = threadIdx.x / G, lane = threadIdx.x % G;
+  const int64_t first = (int64_t)blockIdx.x * (PER_WG * kBlockSteps);
+  int w0 = 0, len = Mo;   // last w with soff[w] <= first, in [w0, w0 + len)
+  while (len > 1) {
+    const int step = (len + 255) / 256, i = (int)threadIdx.x * step;
+    const int hit = __syncthreads_count(i < len && soff[w0 + i] <= first) - 1;
+    w0 += hit * step;
+    len = len - hit * step < step ? len - hit * step : step;
+  }
+  for (int i = threadIdx.x; i < 257; i += 256) off[i] = soff[w0 + i < Mo ? w0 + i : Mo];
+  __syncthreads();
+  for (int stp = 0; stp < kBlockSteps; ++stp) {
+    const int64_t b = first + stp * PER_WG + g;
+    const bool have = b < n_blocks;
+    int w = 0, s0 = 0, s1 = 0, p0 = 0;
+    int64_t e0 = 0;
+    if (have) {
+      int lo = 0, hi = 256, so, sn;   // last w with soff[w] <= b: the window holding block b
+      if (b < off[256] || w0 + 256 >= Mo) {
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) / 2;
+          if (off[mid] <= b) lo = mid; else hi = mid;
+        }
+        w = w0 + lo < Mo ? w0 + lo : Mo - 1;
+      } else {   // many empty windows in between
+        lo = w0 + 256;
+        hi = Mo;
+        while (hi - lo > 1) {
+          const int mid = lo + (hi - lo) / 2;
+          if (soff[mid] <= b) lo = mid; else hi = mid;
+        }
+        w = lo;
+      }
+      so = soff[w];
+      sn = soff[w + 1];
+      const int j = (int)(b - so);
+      const int64_t r0 = (int64_t)w * BH, r1 = r0 + BH < a.num_nodes ? r0 + BH : a.num_nodes;
+      e0 = a.rowptr[r0];
+      p0 = j * BW;
+      s0 = a.s.block[e0 + j];
+      s1 = b + 1 < sn ? a.s.block[e0 + j + 1] : a.rowptr[r1] - (int)e0;
+    }
+#pragma unroll
+    for (int q = 0; q < PER; ++q) tile[g][q * G + lane] = 0.f;
+    for (int q = lane; q < WORDS; q += G) mask[g][q] = 0;
+    __syncthreads();
+    for (int q = s0 + lane; q < s1; q += G) {
+      const int c = a.s.rank[e0 + q] - p0;
+      const uint8_t r = a.s.row[e0 + q];
+      const float v = a.s.val[e0 + q];
+      cols[g][c] = a.s.col[e0 + q];
+      if (r & 0x80) {
+        const int pos = BW * (r & 0x7f) + c;
+        tile[g][swz(pos)] = v;
+        if (__float_as_uint(v) != 0u) atomicOr(&mask[g][pos >> 5], 1u << (pos & 31));
+      }
+    }
+    const int ncols = have ? a.s.rank[e0 + s1 - 1] - p0 + 1 : 0;
+    __syncthreads();
+    if (have) {
+      for (int q = lane; q < BW; q += G) sidx[b * BW + q] = cols[g][q < ncols ? q : ncols - 1];
+#pragma unroll
+      for (int q = 0; q < PER / 4; ++q)
+        reinterpret_cast<float4*>(val + b * SIZE)[q * G + lane] =
+            reinterpret_cast<const float4*>(tile[g])[q * G + lane];
+      if (words) {
+        uint32_t base = vbase[w] + (uint32_t)a.s.stored[e0 + s0];
+        // the lane's positions [lane * PER, lane * PER + PER) lie in one word (PER 8 or 16)
+        const int wd = lane * PER / 32;
+        for (int q = 0; q < wd; ++q) base += (uint32_t)__builtin_popcount(mask[g][q]);
+        const uint32_t m = mask[g][wd];
+        const int bit0 = lane * PER % 32;
+        if (bit0 == 0) words[b * WORDS + wd] = uint2{m, base};
+        uint32_t at = base + (uint32_t)__builtin_popcount(m & ((1u << bit0) - 1u));
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+          if ((m >> (bit0 + q)) & 1u) packed[at++] = tile[g][swz(lane * PER + q)];
+      }
+    }
+    __syncthreads();
+  }
 }
 
 int bits_for(int64_t v) {
@@ -163,204 +534,140 @@ int bits_for(int64_t v) {
   return b < 1 ? 1 : b;
 }
 
-}  // namespace
+// Allocations of one conversion: given back together, after the stream has
+// finished with them.
+struct Temps {
+  DeviceAlloc alloc;
+  DeviceFree dfree;
+  void* ctx;
+  hipStream_t st;
+  void* p[24];
+  int n = 0;
+  template <class T>
+  T* get(size_t count) {
+    void* q = n < 24 ? alloc(ctx, (count ? count : 1) * sizeof(T)) : nullptr;
+    if (q) p[n++] = q;
+    return static_cast<T*>(q);
+  }
+  ~Temps() {
+    (void)hipStreamSynchronize(st);
+    for (int i = 0; i < n; ++i) dfree(ctx, p[i]);
+  }
+};
 
-#define SRBCRS_TRY(x)                        \
-  do {                                       \
-    hipError_t e__ = (x);                    \
-    if (e__ != hipSuccess) return e__;       \
-  } while (0)
+}  // namespace
 
 hipError_t device_convert(const DeviceConvertIn& in, DeviceConvertOut& out, DeviceAlloc alloc,
                           DeviceFree dfree, void* ctx, hipStream_t st) {
+#define SRBCRS_TRY(x)                        \
+  do {                                       \
+    const hipError_t e_ = (x);               \
+    if (e_ != hipSuccess) return e_;         \
+  } while (0)
   const int bh = in.blk_h, bw = in.blk_w;
   const int Mo = (in.num_nodes + bh - 1) / bh;
+  const size_t nnz = (size_t)in.nnz;
   out.Mo = Mo;
   out.total = 0;
   out.bad = 0;
   out.max_col = -1;
-  // 1. validate rowptr before trusting it for any edge access
-  int* d_flag = (int*)alloc(ctx, 2 * sizeof(int));
-  if (!d_flag) return hipErrorOutOfMemory;
-  int h_flag[2] = {0, -1};
-  SRBCRS_TRY(hipMemcpyAsync(d_flag, h_flag, sizeof(h_flag), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_validate_rowptr, dim3(grid_for(in.num_nodes + 1)), dim3(256), 0, st, in.rowptr,
-                     in.num_nodes, in.nnz, d_flag);
-  SRBCRS_TRY(hipGetLastError());
-  int h_rp[2];
-  SRBCRS_TRY(hipMemcpyAsync(h_flag, d_flag, sizeof(h_flag), hipMemcpyDeviceToHost, st));
-  SRBCRS_TRY(hipMemcpyAsync(&h_rp[0], in.rowptr, sizeof(int), hipMemcpyDeviceToHost, st));
-  SRBCRS_TRY(hipMemcpyAsync(&h_rp[1], in.rowptr + in.num_nodes, sizeof(int), hipMemcpyDeviceToHost, st));
-  SRBCRS_TRY(hipStreamSynchronize(st));
-  if (h_flag[0]) {
-    out.bad = 1;
-    dfree(ctx, d_flag);
-    return hipSuccess;
-  }
-  const int e0 = h_rp[0];
-  const int n = h_rp[1] - h_rp[0];
-  // 2. row ids (also edge_to_row), keys
-  int* e2r = in.edge_to_row;
-  SRBCRS_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_row_starts, dim3(grid_for(in.num_nodes)), dim3(256), 0, st, in.rowptr, in.num_nodes, e2r);
-  SRBCRS_TRY(hipGetLastError());
-  if (n > 0) {   // carry the marks over [e0, e0 + n) (the caller zero-filled edge_to_row)
-    int* scanned = (int*)alloc(ctx, (size_t)n * 4);
-    void* scan_tmp = nullptr;
-    size_t scan_bytes = 0;
-    hipError_t e = scanned ? hipSuccess : hipErrorOutOfMemory;
-    if (e == hipSuccess)
-      e = hipcub::DeviceScan::InclusiveScan(nullptr, scan_bytes, e2r + e0, scanned, hipcub::Max(), n, st);
-    if (e == hipSuccess) {
-      scan_tmp = alloc(ctx, scan_bytes ? scan_bytes : 1);
-      if (!scan_tmp) e = hipErrorOutOfMemory;
-    }
-    if (e == hipSuccess)
-      e = hipcub::DeviceScan::InclusiveScan(scan_tmp, scan_bytes, e2r + e0, scanned, hipcub::Max(), n, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(e2r + e0, scanned, (size_t)n * 4, hipMemcpyDeviceToDevice, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (scanned) dfree(ctx, scanned);
-    if (scan_tmp) dfree(ctx, scan_tmp);
-    if (e != hipSuccess) {
-      dfree(ctx, d_flag);
-      return e;
-    }
-  }
-  uint64_t *k0 = nullptr, *k1 = nullptr;
-  int *i0 = nullptr, *i1 = nullptr, *flags = nullptr, *rank = nullptr;
-  int *ucol = nullptr, *uwin = nullptr, *ufirst = nullptr, *nb = nullptr;
-  void* tmp = nullptr;
-  const size_t N = (size_t)(n > 0 ? n : 1);
-  k0 = (uint64_t*)alloc(ctx, N * 8);
-  k1 = (uint64_t*)alloc(ctx, N * 8);
-  i0 = (int*)alloc(ctx, N * 4);
-  i1 = (int*)alloc(ctx, N * 4);
-  flags = (int*)alloc(ctx, N * 4);
-  rank = (int*)alloc(ctx, N * 4);
-  ucol = (int*)alloc(ctx, N * 4);
-  uwin = (int*)alloc(ctx, N * 4);
-  ufirst = (int*)alloc(ctx, ((size_t)Mo + 1) * 4);
-  nb = (int*)alloc(ctx, ((size_t)Mo + 1) * 4);
-  hipError_t err = hipSuccess;
-  auto cleanup = [&] {
-    for (void* p : {(void*)k0, (void*)k1, (void*)i0, (void*)i1, (void*)flags, (void*)rank, (void*)ucol,
-                    (void*)uwin, (void*)ufirst, (void*)nb, tmp, (void*)d_flag})
-      if (p) dfree(ctx, p);
-  };
-  if (!k0 || !k1 || !i0 || !i1 || !flags || !rank || !ucol || !uwin || !ufirst || !nb) {
-    cleanup();
+  Temps t{alloc, dfree, ctx, st};
+  ConvArgs a{in.rowptr, in.colind, in.values, in.num_nodes, in.nnz, bh, bw, in.edge_to_row, in.edge_to_col,
+             in.block_partition, {}, nullptr, {nullptr, nullptr}, nullptr, nullptr};
+  a.s.col = t.get<int>(nnz);
+  a.s.val = t.get<float>(nnz);
+  a.s.rank = t.get<int>(nnz);
+  a.s.stored = t.get<int>(nnz);
+  a.s.block = t.get<int>(nnz);
+  a.s.row = t.get<uint8_t>(nnz);
+  a.wcount = t.get<unsigned long long>((size_t)Mo);
+  a.list[0] = t.get<int>((size_t)Mo);
+  a.list[1] = t.get<int>((size_t)Mo);
+  a.big = t.get<int>((size_t)Mo);
+  a.head = t.get<Head>(1);
+  unsigned* vbase = t.get<unsigned>((size_t)Mo);
+  if (!a.s.col || !a.s.val || !a.s.rank || !a.s.stored || !a.s.block || !a.s.row || !a.wcount || !a.list[0] ||
+      !a.list[1] || !a.big || !a.head || !vbase)
     return hipErrorOutOfMemory;
-  }
-#define SRBCRS_STEP(x)        \
-  do {                        \
-    err = (x);                \
-    if (err != hipSuccess) {  \
-      cleanup();              \
-      return err;             \
-    }                         \
-  } while (0)
-  int nu = 0;
-  if (n > 0) {
-    hipLaunchKernelGGL(k_make_keys, dim3(grid_for(n)), dim3(256), 0, st, in.colind, e2r, e0, n, bh, k0, i0,
-                       d_flag);
-    SRBCRS_STEP(hipGetLastError());
-    // 3. stable radix sort of (window, column) keys with their edge index
+  Head h{};
+  SRBCRS_TRY(hipMemsetAsync(a.head, 0, sizeof(h), st));
+  hipLaunchKernelGGL(k_windows, dim3((unsigned)Mo), dim3(256), 0, st, a);
+  SRBCRS_TRY(hipGetLastError());
+  // (a window longer than a class is impossible where the matrix has no more entries than that)
+  if (in.nnz > kClass[0])
+    hipLaunchKernelGGL(k_listed_windows<0>, dim3((unsigned)(Mo < 1024 ? Mo : 1024)), dim3(512), 0, st, a);
+  SRBCRS_TRY(hipGetLastError());
+  if (in.nnz > kClass[1])
+    hipLaunchKernelGGL(k_listed_windows<1>, dim3((unsigned)(Mo < 256 ? Mo : 256)), dim3(1024), 0, st, a);
+  SRBCRS_TRY(hipGetLastError());
+  auto scan = [&]() -> hipError_t {
+    hipLaunchKernelGGL(k_window_scan, dim3(1), dim3(1024), 0, st, a, Mo, out.soff, vbase);
+    SRBCRS_TRY(hipGetLastError());
+    SRBCRS_TRY(hipMemcpyAsync(&h, a.head, sizeof(h), hipMemcpyDeviceToHost, st));
+    SRBCRS_TRY(hipMemcpyAsync(out.h_soff, out.soff, ((size_t)Mo + 1) * 4, hipMemcpyDeviceToHost, st));
+    return hipStreamSynchronize(st);
+  };
+  SRBCRS_TRY(scan());
+  if (h.n_big && !h.bad) {
+    // windows too long for LDS: one stable device-wide sort of all of theirs
+    const size_t n = (size_t)h.big_entries;
+    uint64_t *k0 = t.get<uint64_t>(n), *k1 = t.get<uint64_t>(n);
+    int *i0 = t.get<int>(n), *i1 = t.get<int>(n);
+    int64_t* d_off = t.get<int64_t>((size_t)h.n_big);
+    if (!k0 || !k1 || !i0 || !i1 || !d_off) return hipErrorOutOfMemory;
+    hipLaunchKernelGGL(k_big_offsets, dim3(1), dim3(64), 0, st, a, d_off);
+    SRBCRS_TRY(hipGetLastError());
+    for (int b = 0; b < h.n_big; b += 32768) {   // grid y limit
+      const int m = h.n_big - b < 32768 ? h.n_big - b : 32768;
+      ConvArgs ab = a;
+      ab.big = a.big + b;
+      hipLaunchKernelGGL(k_big_keys, dim3(16, (unsigned)m), dim3(256), 0, st, ab, d_off + b, k0, i0);
+      SRBCRS_TRY(hipGetLastError());
+    }
     hipcub::DoubleBuffer<uint64_t> kb(k0, k1);
     hipcub::DoubleBuffer<int> ib(i0, i1);
-    const int end_bit = 32 + bits_for(Mo);
-    size_t tmp_bytes = 0;
-    SRBCRS_STEP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, kb, ib, n, 0, end_bit, st));
-    size_t scan_bytes = 0;
-    SRBCRS_STEP(hipcub::DeviceScan::InclusiveSum(nullptr, scan_bytes, flags, rank, n, st));
-    size_t ex_bytes = 0;
-    SRBCRS_STEP(hipcub::DeviceScan::ExclusiveSum(nullptr, ex_bytes, nb, out.soff, Mo + 1, st));
-    size_t need = tmp_bytes > scan_bytes ? tmp_bytes : scan_bytes;
-    if (ex_bytes > need) need = ex_bytes;
-    tmp = alloc(ctx, need ? need : 1);
-    if (!tmp) {
-      cleanup();
-      return hipErrorOutOfMemory;
-    }
-    SRBCRS_STEP(hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, kb, ib, n, 0, end_bit, st));
-    const uint64_t* keys = kb.Current();
-    const int* idx = ib.Current();
-    hipLaunchKernelGGL(k_flags, dim3(grid_for(n)), dim3(256), 0, st, keys, n, flags);
-    SRBCRS_STEP(hipGetLastError());
-    SRBCRS_STEP(hipcub::DeviceScan::InclusiveSum(tmp, scan_bytes, flags, rank, n, st));
-    hipLaunchKernelGGL(k_unique, dim3(grid_for(n)), dim3(256), 0, st, keys, rank, n, ucol, uwin);
-    SRBCRS_STEP(hipGetLastError());
-    SRBCRS_STEP(hipMemcpyAsync(&nu, rank + (n - 1), sizeof(int), hipMemcpyDeviceToHost, st));
-    SRBCRS_STEP(hipStreamSynchronize(st));
-    // negative column seen?
-    SRBCRS_STEP(hipMemcpyAsync(h_flag, d_flag, sizeof(int), hipMemcpyDeviceToHost, st));
-    SRBCRS_STEP(hipStreamSynchronize(st));
-    if (h_flag[0]) {
-      out.bad = 2;
-      cleanup();
-      return hipSuccess;
-    }
-    // max column: the largest column among the distinct keys
-    int* d_max = flags;   // reuse
-    size_t mx_bytes = 0;
-    SRBCRS_STEP(hipcub::DeviceReduce::Max(nullptr, mx_bytes, ucol, d_max, nu, st));
-    if (mx_bytes > need) {
-      dfree(ctx, tmp);
-      tmp = alloc(ctx, mx_bytes);
-      need = mx_bytes;
-      if (!tmp) {
-        cleanup();
-        return hipErrorOutOfMemory;
-      }
-    }
-    SRBCRS_STEP(hipcub::DeviceReduce::Max(tmp, mx_bytes, ucol, d_max, nu, st));
-    SRBCRS_STEP(hipMemcpyAsync(&out.max_col, d_max, sizeof(int), hipMemcpyDeviceToHost, st));
-    // 4. windows: first distinct key, block counts, offsets
-    hipLaunchKernelGGL(k_window_first, dim3(grid_for(Mo + 1)), dim3(256), 0, st, uwin, nu, Mo, ufirst);
-    SRBCRS_STEP(hipGetLastError());
-    hipLaunchKernelGGL(k_block_counts, dim3(grid_for(Mo + 1)), dim3(256), 0, st, ufirst, Mo, bw, nb,
-                       in.block_partition);
-    SRBCRS_STEP(hipGetLastError());
-    SRBCRS_STEP(hipcub::DeviceScan::ExclusiveSum(tmp, ex_bytes, nb, out.soff, Mo + 1, st));
-    int total = 0;
-    SRBCRS_STEP(hipMemcpyAsync(&total, out.soff + Mo, sizeof(int), hipMemcpyDeviceToHost, st));
-    SRBCRS_STEP(hipStreamSynchronize(st));
-    out.total = total;
-    // 5. arrays sized by the total
-    const int64_t nslots = (int64_t)total * bw, nval = (int64_t)total * bh * bw;
-    out.sidx = (int*)alloc(ctx, (size_t)(nslots > 0 ? nslots : 1) * 4);
-    out.val = (float*)alloc(ctx, (size_t)(nval > 0 ? nval : 1) * 4);
-    if (!out.sidx || !out.val) {
-      cleanup();
-      return hipErrorOutOfMemory;
-    }
-    if (nslots) {
-      hipLaunchKernelGGL(k_fill_sidx, dim3(grid_for(nslots)), dim3(256), 0, st, out.soff, ufirst, ucol, Mo, bw,
-                         nslots, out.sidx);
-      SRBCRS_STEP(hipGetLastError());
-      hipLaunchKernelGGL(k_zero, dim3(grid_for(nval)), dim3(256), 0, st, out.val, nval);
-      SRBCRS_STEP(hipGetLastError());
-      hipLaunchKernelGGL(k_scatter, dim3(grid_for(n)), dim3(256), 0, st, keys, idx, rank, n, e2r, in.values,
-                         ufirst, out.soff, bh, bw, out.val, in.edge_to_col);
-      SRBCRS_STEP(hipGetLastError());
-    }
-  } else {
-    // no edges: all windows empty
-    hipLaunchKernelGGL(k_window_first, dim3(grid_for(Mo + 1)), dim3(256), 0, st, uwin, 0, Mo, ufirst);
-    SRBCRS_STEP(hipGetLastError());
-    hipLaunchKernelGGL(k_block_counts, dim3(grid_for(Mo + 1)), dim3(256), 0, st, ufirst, Mo, bw, nb,
-                       in.block_partition);
-    SRBCRS_STEP(hipGetLastError());
-    size_t ex_bytes = 0;
-    SRBCRS_STEP(hipcub::DeviceScan::ExclusiveSum(nullptr, ex_bytes, nb, out.soff, Mo + 1, st));
-    tmp = alloc(ctx, ex_bytes ? ex_bytes : 1);
-    SRBCRS_STEP(hipcub::DeviceScan::ExclusiveSum(tmp, ex_bytes, nb, out.soff, Mo + 1, st));
-    out.sidx = (int*)alloc(ctx, 4);
-    out.val = (float*)alloc(ctx, 4);
+    size_t bytes = 0;
+    const int end_bit = 32 + bits_for(h.n_big);
+    SRBCRS_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, kb, ib, (int)n, 0, end_bit, st));
+    void* tmp = t.get<char>(bytes);
+    if (!tmp) return hipErrorOutOfMemory;
+    SRBCRS_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, bytes, kb, ib, (int)n, 0, end_bit, st));
+    hipLaunchKernelGGL(k_big_rank, dim3((unsigned)h.n_big), dim3(1024), 0, st, a, d_off, kb.Current(), ib.Current());
+    SRBCRS_TRY(hipGetLastError());
+    SRBCRS_TRY(scan());
   }
-  SRBCRS_STEP(hipStreamSynchronize(st));
-#undef SRBCRS_STEP
-  cleanup();
-  return hipSuccess;
+  if (h.bad || h.negative) {
+    out.bad = h.bad ? 1 : 2;
+    return hipSuccess;
+  }
+  out.max_col = h.max_col1 - 1;
+  out.total = (int64_t)(h.totals & 0xffffffffu);
+  const int64_t n_packed = (int64_t)(h.totals >> 32);
+  const int64_t n_words = out.total * bh * bw / 32;
+  auto need = [&](size_t n) { return alloc(ctx, (n ? n : 1) * 4); };
+  out.sidx = (int*)need((size_t)out.total * bw);
+  out.val = (float*)need((size_t)out.total * bh * bw);
+  if (!out.sidx || !out.val) return hipErrorOutOfMemory;
+  if (out.total == 0) return hipSuccess;
+  // without room for the compact copy the plan keeps reading val
+  out.compact.words = (uint2*)need(2 * (size_t)n_words);
+  out.compact.packed = (float*)need((size_t)(n_packed + kPackedPad));
+  if (!out.compact.words || !out.compact.packed) {
+    if (out.compact.words) dfree(ctx, out.compact.words);
+    if (out.compact.packed) dfree(ctx, out.compact.packed);
+    out.compact = CompactOut{};
+  } else {
+    out.compact.n_packed = n_packed;
+    SRBCRS_TRY(hipMemsetAsync(out.compact.packed + n_packed, 0, kPackedPad * 4, st));
+  }
+  if (bh == 16)
+    hipLaunchKernelGGL((k_blocks<16, 8, 16>), dim3((unsigned)((out.total + 63) / 64)), dim3(256), 0, st, a, Mo,
+                       out.soff, vbase, out.total, out.sidx, out.val, out.compact.words, out.compact.packed);
+  else
+    hipLaunchKernelGGL((k_blocks<32, 32, 64>), dim3((unsigned)((out.total + 15) / 16)), dim3(256), 0, st, a, Mo,
+                       out.soff, vbase, out.total, out.sidx, out.val, out.compact.words, out.compact.packed);
+  return hipGetLastError();   // the temporaries' release waits for the stream
+#undef SRBCRS_TRY
 }
 
 }  // namespace srbcrs

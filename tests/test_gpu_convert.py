@@ -79,6 +79,31 @@ def test_device_conversion_workloads(gpu, name):
     _same(_arrays(Plan(t(m.rowptr), t(m.colind), t(m.values), m.M)), oracle.convert(m.rowptr, m.colind, m.values, m.M))
 
 
+@pytest.mark.parametrize("blk,K", [((16, 8), 300), ((16, 8), 3_000_000), ((32, 32), 70_000)])
+def test_device_conversion_window_lengths(gpu, blk, K):
+    """Windows at the edges of the converter's length classes, several past the last one."""
+    import torch
+    from mask_amd.SRBCRSSpMM import Plan
+    rng = np.random.default_rng(K)
+    lens = [0, 1, 63, 257, 2047, 2048, 2049, 4095, 4096, 4097, 16383, 16384, 16385, 20000, 0, 50000, 16390]
+    lens += [0] * 300 + [9]
+    M = len(lens) * blk[0] - 5
+    counts = []
+    for w, n in enumerate(lens):   # edges over the window's rows: some empty, duplicates and unsorted columns
+        rows = min(blk[0], M - w * blk[0])
+        counts.append(np.bincount(rng.integers(0, rows, n) // 2 * 2 % rows, minlength=rows))
+    rp = np.concatenate([[0], np.cumsum(np.concatenate(counts))]).astype(np.int32)
+    ci = rng.integers(0, K, rp[-1]).astype(np.int32)
+    vv = np.where(rng.random(rp[-1]) < 0.1, 0.0, rng.uniform(-1, 1, rp[-1])).astype(np.float32)
+    _say("convert window lengths", blk, K, M, ci.size)
+    t = lambda a: torch.from_numpy(a).cuda()
+    o = oracle.convert(rp, ci, vv, M, blk[0], blk[1])
+    for _ in range(2):   # the second conversion works in memory that the first one has used
+        plan = Plan(t(rp), t(ci), t(vv), M, blk[0], blk[1])
+        _same(_arrays(plan), o)
+        del plan
+
+
 def test_device_conversion_rejects_malformed(gpu):
     import torch
     from mask_amd._capi import SrbcrsError
