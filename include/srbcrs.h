@@ -215,8 +215,8 @@ int srbcrs_plan_set_schedule(srbcrs_plan *plan, const char *policy, int32_t para
  * stored values that gives the block kernels' bits (infinities and NaNs of B
  * included); it needs ldb, ldc multiples of 4, 16-byte aligned B and C and
  * K * ldb * 4 < 2^32, and runs from a width's second run on, which builds its
- * entry stream (it allocates 8 bytes per stored value, kept until the plan is
- * destroyed): capture after two eager runs to capture it.  Elsewhere, under
+ * entry stream (it allocates 8 to 12 bytes per stored value, kept until the plan
+ * is destroyed): capture after two eager runs to capture it.  Elsewhere, under
  * capture before that, and on small products, the block kernels run.  A call
  * that is refused (a negative status) has launched nothing and left C
  * untouched. */

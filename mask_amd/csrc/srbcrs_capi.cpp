@@ -525,7 +525,9 @@ struct srbcrs_plan {
     for (auto& kv : sweeps) {
       srbcrs::ColSweep& w = kv.second.s;
       dev_free(w.entries);
-      for (int** p : {&w.start, &w.nblk, &w.dest, &w.wblk8, &w.wblk4, &w.lstart, &w.lnblk, &w.ldest}) dev_free(*p);
+      for (int** p : {&w.start, &w.nblk, &w.dest, &w.wblk8, &w.wblk4, &w.lstart, &w.lnblk, &w.ldest, &w.uoff,
+                      &w.pend})
+        dev_free(*p);
     }
     for (auto& kv : merged) {
       dev_free(kv.second.d_moff);
@@ -788,49 +790,64 @@ bool sweep_wanted(const srbcrs_plan& plan) {
 // caller that may not allocate.
 const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_build, hipStream_t st) {
   const srbcrs::ColSweepTasks t = sweep_tasks(plan);
-  const int RL = srbcrs::colsweep_rows_per_list((int64_t)t.n * 16, (int)N);
+  const int64_t rows = (int64_t)t.n * 16;
+  // the layouts to try: the phase sweep's, where it is the faster one, and the
+  // lists' (keyed by minus the rows per half, and the rows per list)
+  const int layouts[2] = {-srbcrs::phasesweep_rows(rows, (int)N, (int64_t)plan.max_col + 1),
+                          srbcrs::colsweep_rows_per_list(rows, (int)N)};
   std::lock_guard<std::mutex> lock(plan.sweep_mu);
-  srbcrs_plan::Sweep& w = plan.sweeps[{plan.sched.policy, plan.sched.param, RL}];
-  if (!w.longest)
-    for (int32_t i = 0; i < plan.Mo; ++i) w.longest = std::max(w.longest, plan.h_soff[i + 1] - plan.h_soff[i]);
-  // Small products stay with the block kernel's one launch (the sweep's repair
-  // pass is a second one, 4 us of host time): under 64 MB of gathers both take
-  // less than their launches, unless long windows make the block kernel a
-  // chain (about 0.4 us a block: 40 blocks 17.9 us, sweep 8 + 1.5).
-  if (plan.n_apacked * N < (16 << 20) && w.longest < 24) return nullptr;
-  if (w.built) return &w.s;
-  if (w.failed || !may_build) return nullptr;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
-    return nullptr;
+  bool again = false;   // not the first run of this width
+  for (int layout : layouts) {
+    if (!layout) continue;
+    srbcrs_plan::Sweep& w = plan.sweeps[{plan.sched.policy, plan.sched.param, layout}];
+    if (!w.longest)
+      for (int32_t i = 0; i < plan.Mo; ++i) w.longest = std::max(w.longest, plan.h_soff[i + 1] - plan.h_soff[i]);
+    // Small products stay with the block kernel's one launch (the sweep's repair
+    // pass is a second one, 4 us of host time): under 64 MB of gathers both take
+    // less than their launches, unless long windows make the block kernel a
+    // chain (about 0.4 us a block: 40 blocks 17.9 us, sweep 8 + 1.5).
+    if (plan.n_apacked * N < (16 << 20) && w.longest < 24) return nullptr;
+    if (w.built) return &w.s;
+    if (w.failed) continue;
+    if (!may_build) return nullptr;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    if (!again && w.seen.insert(N).second) return nullptr;
+    again = true;
+    srbcrs::ColSweep s;
+    if (layout < 0) {
+      s.rows = -layout;
+    } else {
+      s.RL = layout;
+      // phases of 4096 columns (512 KB of a 32-column slice; 2048 to 16384 ran
+      // within 3 % of it), one phase where B's slice fits the L2
+      s.shift = 12;
+      while ((plan.max_col >> s.shift) >= 128) ++s.shift;
+      if (plan.max_col < 16384) s.shift = 24;
+      s.phases = (plan.max_col >> s.shift) + 1;
+    }
+    hipError_t e = hipSuccess;
+    if (!plan.d_sweep_flags) {
+      plan.d_sweep_flags = static_cast<unsigned long long*>(srbcrs::pool_alloc(kSweepFlags * 8));
+      e = plan.d_sweep_flags ? hipMemsetAsync(plan.d_sweep_flags, 0, kSweepFlags * 8, st) : hipErrorOutOfMemory;
+    }
+    srbcrs::ColSweepIn in{t, plan.d_awords, plan.d_sidx, plan.d_apacked, plan.n_apacked, plan.d_rowmap,
+                          (int)plan.packed_rows, plan.total, plan.max_col};
+    if (e == hipSuccess) e = srbcrs::build_colsweep(in, s, conv_alloc, conv_free, nullptr, st);
+    if (e == hipErrorOutOfMemory || e == hipErrorInvalidValue) {
+      (void)hipGetLastError();
+      w.failed = true;
+      continue;
+    }
+    hip_check(e, "column sweep stream");
+    w.s = s;
+    w.built = true;
+    return &w.s;
   }
-  if (w.seen.insert(N).second) return nullptr;
-  srbcrs::ColSweep s;
-  s.RL = RL;
-  // phases of 4096 columns (512 KB of a 32-column slice; 2048 to 16384 ran
-  // within 3 % of it), one phase where B's slice fits the L2
-  s.shift = 12;
-  while ((plan.max_col >> s.shift) >= 128) ++s.shift;
-  if (plan.max_col < 16384) s.shift = 24;
-  s.phases = (plan.max_col >> s.shift) + 1;
-  hipError_t e = hipSuccess;
-  if (!plan.d_sweep_flags) {
-    plan.d_sweep_flags = static_cast<unsigned long long*>(srbcrs::pool_alloc(kSweepFlags * 8));
-    e = plan.d_sweep_flags ? hipMemsetAsync(plan.d_sweep_flags, 0, kSweepFlags * 8, st) : hipErrorOutOfMemory;
-  }
-  srbcrs::ColSweepIn in{t, plan.d_awords, plan.d_sidx, plan.d_apacked, plan.n_apacked, plan.d_rowmap,
-                        (int)plan.packed_rows};
-  if (e == hipSuccess) e = srbcrs::build_colsweep(in, s, conv_alloc, conv_free, nullptr, st);
-  if (e == hipErrorOutOfMemory || e == hipErrorInvalidValue) {
-    (void)hipGetLastError();
-    w.failed = true;
-    return nullptr;
-  }
-  hip_check(e, "column sweep stream");
-  w.s = s;
-  w.built = true;
-  return &w.s;
+  return nullptr;
 }
 
 int64_t nz_key(int W, int U, int D) { return ((int64_t)W << 16) | ((int64_t)U << 8) | (int64_t)D; }

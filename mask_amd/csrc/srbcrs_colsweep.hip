@@ -4,12 +4,21 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <vector>
 
 #include "srbcrs_colsweep.hpp"
 #include "srbcrs_convert.h"
 #include "srbcrs_kernels.h"
+#include "srbcrs_phasesweep.hpp"
 
 namespace srbcrs {
+
+// Workgroups for sweep_chunk.
+static int64_t sweep_grid(int64_t n_wg, int n_chunks, int swept) {
+  if (swept || n_chunks > kNumXcd || kNumXcd % n_chunks) return n_wg * n_chunks;
+  const int per = kNumXcd / n_chunks;
+  return (n_wg + per - 1) / per * kNumXcd;
+}
 
 template <int C, int RL, int WV>
 static hipError_t launch_t(const ColSweep& s, const StreamArgs& a, int64_t K, int swept, unsigned long long token,
@@ -17,11 +26,7 @@ static hipError_t launch_t(const ColSweep& s, const StreamArgs& a, int64_t K, in
   const int n_chunks = (a.N + C - 1) / C;
   const int n_waves = s.n_lists / (256 / C);
   const int64_t n_wg = (n_waves + WV - 1) / WV;
-  int64_t grid = n_wg * n_chunks;
-  if (!swept && n_chunks <= kNumXcd && kNumXcd % n_chunks == 0) {
-    const int per = kNumXcd / n_chunks;
-    grid = (n_wg + per - 1) / per * kNumXcd;
-  }
+  int64_t grid = sweep_grid(n_wg, n_chunks, swept);
   const int64_t long_waves = (int64_t)s.n_long * ((a.N + 63) / 64);
   const int64_t long_wgs = ((long_waves + WV - 1) / WV + kNumXcd - 1) / kNumXcd * kNumXcd;
   grid += long_wgs;
@@ -31,7 +36,8 @@ static hipError_t launch_t(const ColSweep& s, const StreamArgs& a, int64_t K, in
   const SweepStream ss{s.entries, s.start, s.nblk, C == 32 ? s.wblk8 : s.wblk4, s.dest, n_waves,
                        s.lstart, s.lnblk, s.ldest, s.n_long};
   hipLaunchKernelGGL((spmm_colsweep<C, RL, WV>), dim3((unsigned)grid), dim3(64 * WV), 0, st, ss, a.B, (uint32_t)bytes,
-                     a.C, a.partial, a.N, (uint32_t)(a.ldb * 4), a.ldc, n_chunks, swept, a.relu, token, flag, (int)long_wgs);
+                     a.C, a.partial, a.N, (uint32_t)(a.ldb * 4), a.ldc, n_chunks, swept, a.relu, token, flag,
+                     (int)long_wgs);
   return hipGetLastError();
 }
 
@@ -51,7 +57,9 @@ static hipError_t launch_t(const ColSweep& s, const StreamArgs& a, int64_t K, in
 // A workgroup of 16 waves in step where B's slice exceeds the L2 (K = 100000,
 // 30000 rows, N = 512: 104 / 137) and the workgroups fill their last round of
 // CUs (one workgroup per CU): a round that is mostly empty costs more
-// (power-law, 116483 nodes, N = 128, 1.8 rounds: 139 one wave / 165).
+// (power-law, 116483 nodes, N = 128, 1.8 rounds: 139 one wave / 165).  These
+// launches are the phase sweep's unless it cannot take the matrix (more than
+// 2^21 columns, or padding of half the values and more).
 //
 // Chunks are pinned to XCDs (an XCD's rows in flight are then all rows of its
 // chunk) except for 32-column chunks of so many rows that one XCD's eighth of
@@ -59,6 +67,7 @@ static hipError_t launch_t(const ColSweep& s, const StreamArgs& a, int64_t K, in
 // rows in the memory-side cache (524288 nodes, N = 256: 1820 / 1940).
 constexpr int64_t kSyncBytes = 6 << 20;     // B slice above which waves keep step (4 MB of L2 hold the hot rows)
 constexpr int64_t kSweptRows = 200000;
+constexpr int64_t kMemCacheBytes = 256 << 20;
 
 static void pick_launch(int64_t rows, int RL, const StreamArgs& a, int64_t K, int& cols, int& wv, int& swept) {
   const int64_t chunks32 = (a.N + 31) / 32;
@@ -77,8 +86,62 @@ int colsweep_rows_per_list(int64_t rows, int N) {
   return RL;
 }
 
+// Where the phase sweep runs: B's 32-column slice exceeds an XCD's L2 by so
+// much that phases pay (40000 rows of a power-law graph, K = 40000, N = 256:
+// lists 152 us, phases 204; 58241: 226 / 214) and its workgroups, one per CU,
+// fill three quarters of the chip (65536 rows of 16, N = 64, half of it: 24 /
+// 30; N = 128: 46 / 41; power-law, 116483 nodes, N = 48: 77 / 72).
+//
+// Rows per half: as many as make the last round of workgroups a full one.
+int phasesweep_rows(int64_t rows, int N, int64_t K) {
+  const int64_t chunks = ((int64_t)N + 31) / 32;
+  if (K * 128 <= kSyncBytes || K > (int64_t(1) << kPhaseRowShift) || rows / 64 * chunks < 3000) return 0;
+  for (int64_t rounds = 1;; ++rounds) {
+    const int64_t units = 256 * rounds / chunks;
+    if (units == 0) continue;
+    const int64_t r = (rows + 2 * units - 1) / (2 * units);
+    if (r <= kPhaseMaxRows) return (int)((r + 7) / 8 * 8);
+  }
+}
+
+template <int C>
+static hipError_t launch_phase_t(const ColSweep& s, const StreamArgs& a, int64_t K, int swept,
+                                 unsigned long long token, unsigned long long* flag, hipStream_t st) {
+  const int n_chunks = (a.N + C - 1) / C;
+  const int64_t n_wg = s.n_lists / (C == 32 ? 2 : 1);
+  int64_t grid = sweep_grid(n_wg, n_chunks, swept);
+  const int64_t long_waves = (int64_t)s.n_long * ((a.N + 63) / 64);
+  const int64_t long_wgs = ((long_waves + 15) / 16 + kNumXcd - 1) / kNumXcd * kNumXcd;
+  grid += long_wgs;
+  if (long_waves > INT32_MAX || grid > INT32_MAX) return hipErrorInvalidConfiguration;
+  const uint64_t bytes = ((uint64_t)(K - 1) * (uint64_t)a.ldb + (uint64_t)a.N) * 4u;
+  const PhaseStream ps{s.entries, s.uoff, s.pend, s.dest, s.n_lists / 2, s.phases, s.rows,
+                       {s.entries, nullptr, nullptr, nullptr, nullptr, 0, s.lstart, s.lnblk, s.ldest, s.n_long}};
+  hipLaunchKernelGGL((spmm_phasesweep<C>), dim3((unsigned)grid), dim3(1024), 0, st, ps, a.B, (uint32_t)bytes, a.C,
+                     a.partial, a.N, (uint32_t)(a.ldb * 4), a.ldc, n_chunks, swept, a.relu, token, flag,
+                     (int)long_wgs);
+  return hipGetLastError();
+}
+
+// 32 or 64 columns, chunks pinned to XCDs or all XCDs on one (us, over 23
+// matrices and widths; as for the lists, narrow slices put more rows in
+// flight, but a slice of rows 1 or 2 KB apart uses few of an L2's channels):
+// 64 pinned below kSweptRows rows (uniform, 100000 rows of 30, N = 256: 32
+// pinned 264, 32 swept 248, 64 pinned 221; 65536 of 16, N = 512: 186, 214,
+// 183), above it 32 (power-law, 524288 nodes, N = 256: 64 pinned 1220, 32
+// swept 1101), swept while the memory-side cache holds a slice and the stream,
+// which every chunk reads again (2^20 nodes, N = 512, 134 + 340 MB: swept 9930,
+// pinned 8980; 232965 nodes, N = 256, 30 + 118 MB: 1033, 1194).
+static hipError_t launch_phasesweep(const ColSweep& s, const StreamArgs& a, int64_t K, unsigned long long token,
+                                    unsigned long long* flag, hipStream_t st) {
+  const int64_t rows = (int64_t)s.n_lists * s.rows;
+  if (a.N % 32 || a.ldb % 32 || rows < kSweptRows) return launch_phase_t<64>(s, a, K, 0, token, flag, st);
+  return launch_phase_t<32>(s, a, K, K * 128 + s.n_entries * 8 <= kMemCacheBytes, token, flag, st);
+}
+
 hipError_t launch_colsweep(const ColSweep& s, const StreamArgs& a, int64_t K, unsigned long long token,
                            unsigned long long* flag, hipStream_t st) {
+  if (s.rows) return launch_phasesweep(s, a, K, token, flag, st);
   int cols, wv, swept;
   pick_launch((int64_t)s.n_lists * s.RL, s.RL, a, K, cols, wv, swept);
 #define SRBCRS_SWEEP(C, RL, WV) return launch_t<C, RL, WV>(s, a, K, swept, token, flag, st)
@@ -109,8 +172,138 @@ hipError_t launch_colsweep_repair(const ColSweepTasks& t, const StreamArgs& a, u
   return hipGetLastError();
 }
 
+static hipError_t build_phasesweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc, DeviceFree dfree,
+                                   void* ctx, hipStream_t st) {
+  const SweepTasks t = sweep_tasks(in.tasks);
+  const int64_t rows = (int64_t)t.n * 16;
+  const int64_t halves = (rows + 2 * out.rows - 1) / (2 * out.rows) * 2, slots = halves * out.rows;
+  const int64_t per_list = in.n_values / (halves * 64);
+  const int64_t long_len = std::max<int64_t>(128, per_list);   // as for the lists above
+  if (rows == 0 || slots > INT32_MAX || long_len > 30000) return hipErrorInvalidValue;
+  const int long_bin = sweep_bin((int)long_len);
+  const int64_t long_cap = (in.n_values + in.n_values / 16 + 4096) / 128 + 1;
+  out.phases = (int)std::min<int64_t>(kPhaseMax, std::max<int64_t>(1, per_list / kPhaseLoad));
+  const int cap = (int)std::max<int64_t>(kPhaseLoad, (long_len + out.phases - 1) / out.phases);
+  out.n_lists = (int)halves;
+  int bin_shift = 0;
+  while ((in.max_col >> bin_shift) >= kPhaseBins) ++bin_shift;
+  const int64_t hp = halves * out.phases;
+  std::vector<void*> temps;
+  hipError_t err = hipSuccess;
+  auto temp = [&](size_t bytes) {
+    void* p = err == hipSuccess ? alloc(ctx, bytes) : nullptr;
+    if (p)
+      temps.push_back(p);
+    else
+      err = hipErrorOutOfMemory;
+    return p;
+  };
+  auto keep = [&](size_t n) {
+    void* p = err == hipSuccess ? alloc(ctx, n) : nullptr;
+    if (!p) err = hipErrorOutOfMemory;
+    return p;
+  };
+  auto cleanup = [&](hipError_t e) {
+    if (e != hipSuccess) (void)hipStreamSynchronize(st);   // queued kernels may use what is given back
+    for (void* p : temps) dfree(ctx, p);
+    if (e != hipSuccess) {
+      auto drop = [&](auto*& p) {
+        if (p) dfree(ctx, (void*)p);
+        p = nullptr;
+      };
+      drop(out.entries);
+      for (int** p : {&out.dest, &out.uoff, &out.pend, &out.lstart, &out.lnblk, &out.ldest}) drop(*p);
+    }
+    return e;
+  };
+  int* len = (int*)temp((size_t)rows * 4);
+  int* hist = (int*)temp(2 * kSweepBins * 4);
+  int* col_hist = (int*)temp(kPhaseBins * 4);
+  uint8_t* phase_of = (uint8_t*)temp(kPhaseBins);
+  int* vrow = (int*)temp((size_t)slots * 4);
+  int* half_len = (int*)temp((size_t)halves * 4);
+  int* lvrow = (int*)temp((size_t)long_cap * 4);
+  // all entries, long rows, entries of the halves, values of the halves
+  unsigned long long* total = (unsigned long long*)temp(32);
+  uint16_t* cnt = (uint16_t*)temp((size_t)(slots * out.phases) * 2);
+  uint32_t* place = (uint32_t*)temp((size_t)(slots * out.phases) * 4);
+  uint16_t* load = (uint16_t*)temp((size_t)hp * 64 * 2);
+  int* batches = (int*)temp((size_t)hp * 4);
+  out.dest = (int*)keep((size_t)slots * 4);
+  out.uoff = (int*)keep((size_t)(halves / 2 + 1) * 4);
+  out.pend = (int*)keep((size_t)(halves / 2 * out.phases) * 4);
+  out.lstart = (int*)keep((size_t)long_cap * 4);
+  out.lnblk = (int*)keep((size_t)long_cap * 4);
+  out.ldest = (int*)keep((size_t)long_cap * 4);
+  if (err != hipSuccess) return cleanup(err);
+#define SRBCRS_STEP(x)                          \
+  do {                                          \
+    const hipError_t e_ = (x);                  \
+    if (e_ != hipSuccess) return cleanup(e_);   \
+  } while (0)
+  SRBCRS_STEP(hipMemsetAsync(hist, 0, 2 * kSweepBins * 4, st));
+  SRBCRS_STEP(hipMemsetAsync(col_hist, 0, kPhaseBins * 4, st));
+  SRBCRS_STEP(hipMemsetAsync(vrow, 0xff, (size_t)slots * 4, st));
+  SRBCRS_STEP(hipMemsetAsync(out.dest, 0xff, (size_t)slots * 4, st));
+  SRBCRS_STEP(hipMemsetAsync(half_len, 0, (size_t)halves * 4, st));
+  SRBCRS_STEP(hipMemsetAsync(total, 0, 32, st));
+  int64_t g = (rows + 31) / 32;
+  hipLaunchKernelGGL(k_sweep_len, dim3((unsigned)(g > 8192 ? 8192 : g)), dim3(256), 0, st, t, in.words, in.sidx, len,
+                     hist);
+  SRBCRS_STEP(hipGetLastError());
+  g = (rows + 256 * kSweepRankRows - 1) / (256 * kSweepRankRows);
+  int* n_long = reinterpret_cast<int*>(total + 1);
+  hipLaunchKernelGGL(k_sweep_rank, dim3((unsigned)g), dim3(256), 0, st, t, len, hist, hist + kSweepBins, (int)halves,
+                     out.rows, long_bin, in.rowmap, in.M, vrow, out.dest, half_len, lvrow, out.ldest, (int)long_cap,
+                     n_long);
+  SRBCRS_STEP(hipGetLastError());
+  g = (in.n_blocks + 256 * 16 - 1) / (256 * 16);
+  hipLaunchKernelGGL(k_phase_hist, dim3((unsigned)(g > 1024 ? 1024 : g < 1 ? 1 : g)), dim3(256), 0, st, in.words,
+                     in.sidx, in.n_blocks, bin_shift, col_hist);
+  SRBCRS_STEP(hipGetLastError());
+  hipLaunchKernelGGL(k_phase_cuts, dim3(1), dim3(1024), 0, st, col_hist, out.phases, phase_of);
+  SRBCRS_STEP(hipGetLastError());
+  hipLaunchKernelGGL(k_phase_count, dim3((unsigned)(slots / 8)), dim3(64), 0, st, t, in.words, in.sidx, vrow, out.rows,
+                     out.phases, bin_shift, cap, phase_of, cnt);
+  SRBCRS_STEP(hipGetLastError());
+  hipLaunchKernelGGL(k_phase_assign, dim3((unsigned)hp), dim3(64), 0, st, cnt, out.rows, place, load, batches);
+  SRBCRS_STEP(hipGetLastError());
+  hipLaunchKernelGGL(k_phase_offsets, dim3(1), dim3(1024), 0, st, batches, half_len, (int)(halves / 2), out.phases,
+                     out.pend, out.uoff, total);
+  SRBCRS_STEP(hipGetLastError());
+  hipLaunchKernelGGL(k_sweep_place_long, dim3((unsigned)((long_cap + 63) / 64)), dim3(64), 0, st, len, lvrow, n_long,
+                     (int)long_cap, (int64_t)INT32_MAX, out.lstart, out.lnblk, total);
+  SRBCRS_STEP(hipGetLastError());
+  unsigned long long h[4] = {0, 0, 0, 0};
+  SRBCRS_STEP(hipMemcpyAsync(h, total, 32, hipMemcpyDeviceToHost, st));
+  SRBCRS_STEP(hipStreamSynchronize(st));
+  out.n_long = (int)(h[1] & 0xffffffffu);
+  out.n_entries = (int64_t)h[0];
+  if (h[0] > (unsigned long long)INT32_MAX - 64 || out.n_long > long_cap || h[2] > h[3] + h[3] / 2 + 65536)
+    return cleanup(hipErrorInvalidValue);
+  out.entries = (uint2*)alloc(ctx, ((size_t)h[0] + 8) * 8);
+  if (!out.entries) return cleanup(hipErrorOutOfMemory);
+  const PhaseFill f{cnt, place, load, out.uoff, out.pend, out.rows, out.phases};
+  hipLaunchKernelGGL(k_phase_fill, dim3((unsigned)(slots / 8)), dim3(64), 0, st, t, in.words, in.sidx, in.packed, vrow,
+                     f, out.entries);
+  SRBCRS_STEP(hipGetLastError());
+  hipLaunchKernelGGL(k_phase_pad, dim3((unsigned)(halves / 2 * out.phases)), dim3(128), 0, st, f, in.max_col,
+                     out.entries);
+  SRBCRS_STEP(hipGetLastError());
+  if (out.n_long) {
+    hipLaunchKernelGGL(k_sweep_fill, dim3((unsigned)((out.n_long + 7) / 8)), dim3(64), 32 * 4, st, t, in.words,
+                       in.sidx, in.packed, vrow, (int64_t)0, 1, half_len, out.uoff, out.uoff, 1, 31, lvrow, len,
+                       out.lstart, out.lnblk, n_long, (int)long_cap, out.entries);
+    SRBCRS_STEP(hipGetLastError());
+  }
+  SRBCRS_STEP(hipStreamSynchronize(st));
+#undef SRBCRS_STEP
+  return cleanup(hipSuccess);
+}
+
 hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc, DeviceFree dfree, void* ctx,
                           hipStream_t st) {
+  if (out.rows) return build_phasesweep(in, out, alloc, dfree, ctx, st);
   const SweepTasks t = sweep_tasks(in.tasks);
   const int64_t rows = (int64_t)t.n * 16;
   const int RL = out.RL;

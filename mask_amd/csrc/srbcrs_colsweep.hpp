@@ -145,10 +145,24 @@ __device__ __forceinline__ void sweep_long_row(const SweepStream& s, int r, int 
   if (__any(bad) && lane == 0) atomicMax(flag, token);
 }
 
-// One workgroup = WV waves of LG lists on one chunk of C columns.  swept = 0:
-// column chunks pinned to XCDs (xcd_remap over chunk-major ids, or chunk =
-// XCD % n_chunks where the chunks divide the 8 XCDs); 1: every XCD on the
-// same chunk at a time.
+// Workgroup id of n_ids to row part wg (>= n_wg: none) and column chunk c.
+// swept = 0: chunks pinned to XCDs (xcd_remap over chunk-major ids, or chunk =
+// XCD % n_chunks where the chunks divide the 8 XCDs); 1: every XCD on the same
+// chunk at a time.
+__device__ __forceinline__ void sweep_chunk(int id, int n_ids, int n_wg, int n_chunks, int swept, int& wg, int& c) {
+  if (!swept && n_chunks <= kNumXcd && kNumXcd % n_chunks == 0) {
+    const int per = kNumXcd / n_chunks;
+    const int x = id % kNumXcd;
+    c = x % n_chunks;
+    wg = id / kNumXcd * per + x / n_chunks;
+  } else {
+    const int lid = swept ? id : (int)xcd_remap(id, n_ids);
+    c = lid / n_wg;
+    wg = lid % n_wg;
+  }
+}
+
+// One workgroup = WV waves of LG lists on one chunk of C columns.
 template <int C, int RL, int WV>
 __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(WV == 1 ? 5 : 4))) void spmm_colsweep(
     SweepStream s, const float* __restrict__ B, uint32_t b_bytes, float* __restrict__ Cout,
@@ -157,7 +171,7 @@ __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(WV == 1
   constexpr int LPG = C / 4, LG = 64 / LPG;
   __shared__ __attribute__((aligned(16))) float tile[WV * LG * RL * C];
   const int n_wg = (s.n_waves + WV - 1) / WV;
-  int bid = (int)blockIdx.x;
+  const int bid = (int)blockIdx.x;
   const int wave = WV == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (bid < long_wgs) {   // whole workgroups: the barriers below are not theirs
@@ -166,18 +180,8 @@ __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(WV == 1
       sweep_long_row(s, i % s.n_long, i / s.n_long, B, b_bytes, Cout, partial, N, ldb4, ldc, relu, token, flag, lane);
     return;
   }
-  bid -= long_wgs;   // a multiple of the XCD count: the chunk mapping below still sees XCD = id % 8
-  int wg, c;
-  if (!swept && n_chunks <= kNumXcd && kNumXcd % n_chunks == 0) {
-    const int per = kNumXcd / n_chunks;
-    const int x = bid % kNumXcd;
-    c = x % n_chunks;
-    wg = bid / kNumXcd * per + x / n_chunks;
-  } else {
-    const int lid = swept ? bid : (int)xcd_remap(bid, gridDim.x - long_wgs);
-    c = lid / n_wg;
-    wg = lid % n_wg;
-  }
+  int wg, c;   // long_wgs is a multiple of the XCD count: XCD = id % 8 still
+  sweep_chunk(bid - long_wgs, gridDim.x - long_wgs, n_wg, n_chunks, swept, wg, c);
   if (wg >= n_wg) return;
   const int grp = lane / LPG, sub = lane % LPG;
   int w = wg * WV + wave;
@@ -529,7 +533,8 @@ static __global__ __launch_bounds__(64) void k_sweep_place(const int* __restrict
 static __global__ __launch_bounds__(64) void k_sweep_place_long(const int* __restrict__ len,
                                                                 const int* __restrict__ lvrow,
                                                                 const int* __restrict__ n_long, int long_cap,
-                                                                int64_t cap, int* __restrict__ lstart, int* __restrict__ lnblk,
+                                                                int64_t cap, int* __restrict__ lstart,
+                                                                int* __restrict__ lnblk,
                                                                 unsigned long long* __restrict__ total) {
   const int r = blockIdx.x * 64 + threadIdx.x;
   if (r >= *n_long || r >= long_cap) return;

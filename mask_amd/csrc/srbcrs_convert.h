@@ -55,9 +55,9 @@ hipError_t device_compact(const float* val, int64_t n_blocks, int blk_h, int blk
                           DeviceFree dfree, void* ctx, hipStream_t st, CompactOut& out);
 
 // Entry stream of the column sweep (srbcrs_colsweep.hip): out's RL, phases and
-// shift are the caller's choice, the rest is filled in; its arrays are
-// allocated through the callback and the caller's to free.
-// hipErrorInvalidValue: the matrix does not fit the stream's 32-bit offsets.
+// shift, or its rows (the phase sweep), are the caller's choice, the rest is
+// filled in; its arrays are allocated through the callback and the caller's to
+// free.  hipErrorInvalidValue: the matrix does not fit the stream.
 struct ColSweepIn {
   ColSweepTasks tasks;
   const uint2* words;    // compact A
@@ -66,6 +66,8 @@ struct ColSweepIn {
   int64_t n_values;      // stored values
   const int* rowmap;     // packed row -> output row (null = identity)
   int M;                 // packed rows
+  int64_t n_blocks;
+  int max_col;
 };
 hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc, DeviceFree dfree, void* ctx,
                           hipStream_t st);

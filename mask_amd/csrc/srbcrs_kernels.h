@@ -123,6 +123,8 @@ struct ColSweep {
   int *wblk8 = nullptr, *wblk4 = nullptr;   // batches per 8 and per 4 lists
   int n_long = 0;                           // rows outside the lists
   int *lstart = nullptr, *lnblk = nullptr, *ldest = nullptr;
+  int rows = 0;           // phase sweep: rows per half (of n_lists halves); 0: the lists above
+  int *uoff = nullptr, *pend = nullptr;
 };
 struct ColSweepTasks {   // block ranges; window null = window t, slot null = no partial tiles
   const int *begin, *end, *window, *slot;
@@ -132,6 +134,8 @@ struct ColSweepTasks {   // block ranges; window null = window t, slot null = no
 // that leave 2000 waves (256 CUs hold 5120; below that the lists' chains set
 // the time: 16384 rows of 20, N = 64: 27 us at 8 rows, 22 at 4 or 2).
 int colsweep_rows_per_list(int64_t rows, int N);
+// Rows per half for the phase sweep (srbcrs_phasesweep.hpp); 0: the launch takes the lists.
+int phasesweep_rows(int64_t rows, int N, int64_t K);
 hipError_t launch_colsweep(const ColSweep& s, const StreamArgs& a, int64_t K, unsigned long long token,
                            unsigned long long* flag, hipStream_t st);
 hipError_t launch_colsweep_repair(const ColSweepTasks& t, const StreamArgs& a, unsigned long long token,

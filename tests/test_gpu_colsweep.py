@@ -81,6 +81,34 @@ def test_second_run_builds_the_stream(gpu):
     assert free[0] - free[1] >= 8 * M * 16 and free[2] == free[1]
 
 
+# (M, K, columns per row, N, band): 64 columns with a ragged last chunk; 32 columns, all XCDs on one chunk
+# and chunks pinned; rows whose columns all lie in one phase; fewer columns than phases have bins
+@pytest.mark.parametrize("policy", [("row", 0), ("split", 5)])
+@pytest.mark.parametrize("shape", [(6100, 50000, 9, 1008, 0), (210001, 49999, 4, 32, 0), (210000, 1990000, 4, 32, 0),
+                                   (70003, 70003, 20, 128, 200), (150000, 49160, 1, 128, 0)])
+def test_phase_sweep(gpu, shape, policy):
+    """Widths and sizes at which the workgroups' rows are pooled."""
+    import torch
+    M, K, per_row, N, band = shape
+    rng = np.random.default_rng(M + per_row)
+    lens = rng.integers(0, 2 * per_row + 1, M)
+    lens[[5, M // 2]] = 3000    # longer than a list
+    lens[17:40] = 130           # more than a phase's share
+    row = np.repeat(np.arange(M), lens)
+    cols = rng.integers(0, K, row.size) if not band else np.clip(row + rng.integers(-band, band, row.size), 0, K - 1)
+    cols = cols[np.lexsort((cols, row))].astype(np.int32)
+    csr = (np.concatenate([[0], np.cumsum(lens)]).astype(np.int32), cols,
+           rng.uniform(-1, 1, row.size).astype(np.float32))
+    print("[case] phase sweep", shape, policy, row.size, flush=True)
+    plan = _plan(csr, M)
+    plan.set_schedule(*policy)
+    B = torch.rand((K, N), device="cuda") - 0.5
+    _check(plan, B, shape)
+    _check(plan, B, (shape, "relu"), relu=True)
+    B[int(cols[777]), 7] = float("inf")
+    assert not bool(torch.isfinite(_check(plan, B, (shape, "inf"))).all())
+
+
 @pytest.mark.parametrize("policy", [("row", 0), ("split", 7)])
 def test_non_finite_dense_values(gpu, policy):
     """An infinity or NaN of B poisons every row of the windows whose blocks
