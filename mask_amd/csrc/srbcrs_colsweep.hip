@@ -95,7 +95,7 @@ int colsweep_rows_per_list(int64_t rows, int N) {
 // Rows per half: as many as make the last round of workgroups a full one.
 int phasesweep_rows(int64_t rows, int N, int64_t K) {
   const int64_t chunks = ((int64_t)N + 31) / 32;
-  if (K * 128 <= kSyncBytes || K > (int64_t(1) << kPhaseRowShift) || rows / 64 * chunks < 3000) return 0;
+  if (K * 128 <= kSyncBytes || K > (int64_t)kPhaseNull || rows / 64 * chunks < 3000) return 0;
   for (int64_t rounds = 1;; ++rounds) {
     const int64_t units = 256 * rounds / chunks;
     if (units == 0) continue;
@@ -104,39 +104,52 @@ int phasesweep_rows(int64_t rows, int N, int64_t K) {
   }
 }
 
-template <int C>
+template <int C, int WV>
 static hipError_t launch_phase_t(const ColSweep& s, const StreamArgs& a, int64_t K, int swept,
                                  unsigned long long token, unsigned long long* flag, hipStream_t st) {
   const int n_chunks = (a.N + C - 1) / C;
-  const int64_t n_wg = s.n_lists / (C == 32 ? 2 : 1);
-  int64_t grid = sweep_grid(n_wg, n_chunks, swept);
+  const int64_t n_wg = s.n_lists / (C == 32 ? WV / 8 : 1);
+  const int64_t n_ids = sweep_grid(n_wg, n_chunks, swept);
   const int64_t long_waves = (int64_t)s.n_long * ((a.N + 63) / 64);
-  const int64_t long_wgs = ((long_waves + 15) / 16 + kNumXcd - 1) / kNumXcd * kNumXcd;
-  grid += long_wgs;
-  if (long_waves > INT32_MAX || grid > INT32_MAX) return hipErrorInvalidConfiguration;
+  const int64_t total = n_ids + (long_waves + WV - 1) / WV;
+  if (long_waves > INT32_MAX || total > INT32_MAX) return hipErrorInvalidConfiguration;
   const uint64_t bytes = ((uint64_t)(K - 1) * (uint64_t)a.ldb + (uint64_t)a.N) * 4u;
   const PhaseStream ps{s.entries, s.uoff, s.pend, s.dest, s.n_lists / 2, s.phases, s.rows,
                        {s.entries, nullptr, nullptr, nullptr, nullptr, 0, s.lstart, s.lnblk, s.ldest, s.n_long}};
-  hipLaunchKernelGGL((spmm_phasesweep<C>), dim3((unsigned)grid), dim3(1024), 0, st, ps, a.B, (uint32_t)bytes, a.C,
-                     a.partial, a.N, (uint32_t)(a.ldb * 4), a.ldc, n_chunks, swept, a.relu, token, flag,
-                     (int)long_wgs);
+  if (total == 0) return hipSuccess;
+  hipLaunchKernelGGL((spmm_phasesweep<C, WV>), dim3((unsigned)total), dim3(64 * WV), 0, st, ps, a.B, (uint32_t)bytes,
+                     a.C, a.partial, a.N, (uint32_t)(a.ldb * 4), a.ldc, n_chunks, swept, a.relu, token, flag,
+                     (int)n_ids);
   return hipGetLastError();
 }
 
-// 32 or 64 columns, chunks pinned to XCDs or all XCDs on one (us, over 23
-// matrices and widths; as for the lists, narrow slices put more rows in
-// flight, but a slice of rows 1 or 2 KB apart uses few of an L2's channels):
-// 64 pinned below kSweptRows rows (uniform, 100000 rows of 30, N = 256: 32
-// pinned 264, 32 swept 248, 64 pinned 221; 65536 of 16, N = 512: 186, 214,
-// 183), above it 32 (power-law, 524288 nodes, N = 256: 64 pinned 1220, 32
-// swept 1101), swept while the memory-side cache holds a slice and the stream,
-// which every chunk reads again (2^20 nodes, N = 512, 134 + 340 MB: swept 9930,
-// pinned 8980; 232965 nodes, N = 256, 30 + 118 MB: 1033, 1194).
+// Columns, waves per workgroup and mapping, from all of them on 26 matrices
+// and widths (us; 32 columns put twice the rows in flight of 64, but a slice
+// of B rows 1 or 2 KB apart uses few of an L2's channels; two workgroups of 8
+// waves on a CU overlap one's phase start, where the misses are, with the
+// other's, but keep two phases of B in the L2):
+//   64 columns, pinned     few rows: uniform, 100000 of 30, N = 256: 221, 32
+//                          columns of 8 / 16 waves 237 / 246; 30000 of 20: 62,
+//                          73 / 73
+//   32, 8 waves, swept     graphs with hubs (rows past the lists' average) and
+//                          20 values a row: power-law, 116483 nodes, N = 256:
+//                          245, 261 of 16 waves, 263 at 64; 58241: 190, 216,
+//                          209; 232965: 988, 1055, 1005
+//   32, 16 waves, swept    many rows, fewer values: 524288 nodes of 16, N = 256:
+//                          1124, 8 waves 1188, 64 columns 1174; uniform, 300000
+//                          of 8, N = 128: 119, 133, 135
+//   32, 16 waves, pinned   where the memory-side cache does not hold a slice and
+//                          the stream, which every chunk reads again (2^20
+//                          nodes, N = 512, 134 + 340 MB: 8680, swept 9760)
 static hipError_t launch_phasesweep(const ColSweep& s, const StreamArgs& a, int64_t K, unsigned long long token,
                                     unsigned long long* flag, hipStream_t st) {
   const int64_t rows = (int64_t)s.n_lists * s.rows;
-  if (a.N % 32 || a.ldb % 32 || rows < kSweptRows) return launch_phase_t<64>(s, a, K, 0, token, flag, st);
-  return launch_phase_t<32>(s, a, K, K * 128 + s.n_entries * 8 <= kMemCacheBytes, token, flag, st);
+  const bool cached = K * 128 + s.n_entries * 8 <= kMemCacheBytes;
+  const bool hubs = s.n_long > 0 && s.n_entries >= 20 * rows;
+  if (a.N % 32 || a.ldb % 32 || (rows < kSweptRows && !(cached && hubs)))
+    return launch_phase_t<64, 16>(s, a, K, 0, token, flag, st);
+  if (cached && hubs) return launch_phase_t<32, 8>(s, a, K, 1, token, flag, st);
+  return launch_phase_t<32, 16>(s, a, K, cached, token, flag, st);
 }
 
 hipError_t launch_colsweep(const ColSweep& s, const StreamArgs& a, int64_t K, unsigned long long token,
@@ -287,8 +300,7 @@ static hipError_t build_phasesweep(const ColSweepIn& in, ColSweep& out, DeviceAl
   hipLaunchKernelGGL(k_phase_fill, dim3((unsigned)(slots / 8)), dim3(64), 0, st, t, in.words, in.sidx, in.packed, vrow,
                      f, out.entries);
   SRBCRS_STEP(hipGetLastError());
-  hipLaunchKernelGGL(k_phase_pad, dim3((unsigned)(halves / 2 * out.phases)), dim3(128), 0, st, f, in.max_col,
-                     out.entries);
+  hipLaunchKernelGGL(k_phase_pad, dim3((unsigned)(halves / 2 * out.phases)), dim3(128), 0, st, f, out.entries);
   SRBCRS_STEP(hipGetLastError());
   if (out.n_long) {
     hipLaunchKernelGGL(k_sweep_fill, dim3((unsigned)((out.n_long + 7) / 8)), dim3(64), 32 * 4, st, t, in.words,

@@ -5,13 +5,14 @@
 // rows favour other columns drift apart: on a power-law graph of 232965 nodes
 // the rows in flight on an XCD touch a tenth as many B rows as they have
 // values, yet 58 % of the gathers missed the L2.  Here B is cut into phases of
-// equally many values.  A unit is two halves of up to 640 rows, whose sums are
-// all in LDS (160 KB with both halves at 32 columns, or one half at 64), and
-// any lane group may add to any of them: per phase the rows' runs of values
-// are dealt, longest first, to the half's 64 lists, so that they come out
-// within a value of each other, and a barrier ends the phase (the next one may
-// give a row to another list).  Lists are padded to the phase's longest in
-// whole batches; a mean of 13 values a list nearly always takes two, so all
+// equally many values.  A unit is two halves of up to 640 rows; a workgroup
+// holds the sums of one half (16 waves at 64 columns, 8 at 32) or of both (16
+// waves at 32) in LDS, and any lane group may add to any row of its half: per
+// phase the rows' runs of values are dealt, longest first, to the half's 64
+// lists, so that they come out within a value of each other, and a barrier
+// ends the phase (the next one may give a row to another list).  Lists are
+// padded to the phase's longest in whole batches (the null entries' gathers
+// lie past B's end and fetch nothing); a mean of 13 values a list nearly always takes two, so all
 // workgroups of the chip run the same number of batches in every phase and
 // keep step without any of them waiting (means of 20 in three batches, 28 in
 // four: 2-5 % slower on power-law graphs; means that spill over in some units:
@@ -23,13 +24,19 @@
 // follow each other on a list, both happen in one step.
 //
 // Measured against the column sweep (one MI355X, three B in turn, us): the
-// 232965-node graph, N = 256 1284 -> 1033 (misses 58 % -> 30 %), N = 384
-// 1879 -> 1537, N = 128 666 -> 527; 2^20 nodes, 34.4 M values, N = 512 10570 ->
-// 8980; uniform 100000 x 100000, 30 per row, N = 256 276 -> 221; 65536 x 65536,
-// 16 per row, N = 512 189 -> 183.  The bound: a B row 1 or 2 KB from the next
-// one keeps to a few of the L2's channels (with 32 floats of padding 1033 ->
-// 927, but padding B costs a copy of it).  A third batch of gathers in flight
-// changed nothing.
+// 232965-node graph, N = 256 1284 -> 988 (misses 58 % -> 30 %), N = 128 666 ->
+// 482; 2^20 nodes, 34.4 M values, N = 512 10570 -> 8680; 116483 nodes, N = 256
+// 292 -> 245; uniform 100000 x 100000, 30 per row, N = 256 276 -> 221; 65536 x
+// 65536, 16 per row, N = 512 189 -> 182.
+//
+// What bounds it: with B small enough that every gather hits the L2, 475 us
+// for the first graph's values at N = 256 (25 TB/s into the CUs), whatever the
+// runs' lengths; above that the misses, and that a B row 1 or 2 KB from the
+// next keeps to a few of the L2's channels (32 floats of padding gain 6-11 %,
+// less than a padded copy of B costs).  Without effect: a third batch of
+// gathers in flight; launches of a round or four each, which start the
+// workgroups together (up to 5 % slower).  Slower: reading a batch's eight
+// sums ahead of it (4-12 %).
 #pragma once
 #include "srbcrs_colsweep.hpp"
 
@@ -38,6 +45,7 @@ namespace srbcrs {
 // Stream entry: kPhaseLast | row of the half << kPhaseRowShift | B row, value.
 constexpr uint32_t kPhaseLast = 0x80000000u;
 constexpr int kPhaseRowShift = 21;
+constexpr uint32_t kPhaseNull = (1u << kPhaseRowShift) - 1u;   // B row of null entries, and the field's mask
 constexpr int kPhaseMaxRows = 640;   // rows of a half; two halves of 32 columns fill 160 KB
 constexpr int kPhaseLists = 128;     // lists of a unit
 constexpr int kPhaseBins = 4096;     // of the column histogram
@@ -53,34 +61,34 @@ struct PhaseStream {
   SweepStream longs;      // the long rows
 };
 
-template <int C>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void spmm_phasesweep(
+template <int C, int WV>
+__global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(4))) void spmm_phasesweep(
     PhaseStream s, const float* __restrict__ B, uint32_t b_bytes, float* __restrict__ Cout,
     float* __restrict__ partial, int N, uint32_t ldb4, int64_t ldc, int n_chunks, int swept, int relu,
-    unsigned long long token, unsigned long long* __restrict__ flag, int long_wgs) {
-  constexpr int LPG = C / 4, LG = 64 / LPG, SH = C == 32 ? 7 : 8, HALVES = C == 32 ? 2 : 1;
+    unsigned long long token, unsigned long long* __restrict__ flag, int n_ids) {
+  constexpr int LPG = C / 4, LG = 64 / LPG, SH = C == 32 ? 7 : 8, HALVES = WV * LG / 64;
   __shared__ __attribute__((aligned(16))) float tile[HALVES * kPhaseMaxRows * C];
   const int n_wg = s.n_units * (2 / HALVES);
-  const int bid = (int)blockIdx.x;
+  const int id = (int)blockIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  if (bid < long_wgs) {   // whole workgroups: the barriers below are not theirs
-    const int i = bid * 16 + wave;
+  if (id >= n_ids) {   // whole workgroups: the barriers below are not theirs
+    const int i = (id - n_ids) * WV + wave;
     if (i < s.longs.n_long * ((N + 63) / 64))
       sweep_long_row(s.longs, i % s.longs.n_long, i / s.longs.n_long, B, b_bytes, Cout, partial, N, ldb4, ldc, relu,
                      token, flag, lane);
     return;
   }
   int wg, c;
-  sweep_chunk(bid - long_wgs, gridDim.x - long_wgs, n_wg, n_chunks, swept, wg, c);
+  sweep_chunk(id, n_ids, n_wg, n_chunks, swept, wg, c);
   if (wg >= n_wg) return;
   const int grp = lane / LPG, sub = lane % LPG;
-  const int unit = C == 32 ? wg : wg >> 1;
-  const int rows = HALVES * s.rows;                       // of this workgroup
-  const int list = C == 32 ? wave * LG + grp : (wg & 1) * 64 + wave * LG + grp;
-  const uint32_t row0 = C == 32 && wave >= 8 ? (uint32_t)s.rows : 0u;
+  const int unit = HALVES == 2 ? wg : wg >> 1;
+  const int rows = HALVES * s.rows;   // of this workgroup
+  const int list = (HALVES == 2 ? 0 : (wg & 1) * 64) + wave * LG + grp;
+  const uint32_t row0 = HALVES == 2 && wave >= WV / 2 ? (uint32_t)s.rows : 0u;
   f4* tile4 = reinterpret_cast<f4*>(tile);
-  for (int i = threadIdx.x; i < rows * LPG; i += 1024) tile4[i] = f4{0.f, 0.f, 0.f, 0.f};
+  for (int i = threadIdx.x; i < rows * LPG; i += 64 * WV) tile4[i] = f4{0.f, 0.f, 0.f, 0.f};
   const int col = c * C + 4 * sub;
   const int u0 = uniform_load(s.uoff, unit), nb = uniform_load(s.uoff, unit + 1) - u0;
   auto barrier = [] {   // the sums are in LDS: only its operations are waited for
@@ -97,7 +105,9 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
     auto fetch = [&](int j) { return ep[(int64_t)(j < nb ? j : nb - 1) * (kPhaseLists * kSweepBatch)]; };
     f4 b[2][kSweepBatch];
     auto issue = [&](f4(&d)[kSweepBatch], uint2 m) {
-      const uint32_t off = __umul24(m.x & ((1u << kPhaseRowShift) - 1u), ldb4);
+      const uint32_t row = m.x & kPhaseNull;
+      // (with more than 4 KB of columns or B near 4 GB a null entry may land inside B: harmless)
+      const uint32_t off = row == kPhaseNull ? 0u - 4096u : __umul24(row, ldb4);
 #define SRBCRS_ISSUE(q)                                                \
   d[q] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128( \
                                     rs, group_bcast<LPG, q>(off) + boff, 0, 0))
@@ -174,7 +184,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
   barrier();
   bool bad = false;
   const int* dest = s.dest + (int64_t)wg * rows;
-  for (int r = wave * LG + grp; r < rows; r += 16 * LG) {
+  for (int r = wave * LG + grp; r < rows; r += WV * LG) {
     const int d = dest[r];
     f4 v = tile4[r * LPG + sub];
     if (d != -1 && col < N) {
@@ -453,9 +463,10 @@ static __global__ __launch_bounds__(64) void k_phase_fill(SweepTasks t, const ui
   }
 }
 
-// Null entries where a list's phase is shorter than its unit's: the B row
-// before it again (a cache hit), value 0, never stored.
-static __global__ __launch_bounds__(128) void k_phase_pad(PhaseFill f, int max_col, uint2* __restrict__ entries) {
+// Null entries where a list's phase is shorter than its unit's: a B row past
+// the end (the buffer load returns 0 and fetches nothing), value 0, never
+// stored.
+static __global__ __launch_bounds__(128) void k_phase_pad(PhaseFill f, uint2* __restrict__ entries) {
   const int64_t unit = blockIdx.x / f.phases;
   const int p = (int)(blockIdx.x % f.phases), list = threadIdx.x;
   const int begin = p ? f.pend[unit * f.phases + p - 1] : 0, end = f.pend[unit * f.phases + p];
@@ -463,9 +474,7 @@ static __global__ __launch_bounds__(128) void k_phase_pad(PhaseFill f, int max_c
   const int n = f.load[((2 * unit + (list >> 6)) * f.phases + p) * 64 + (list & 63)];
   const int room = (end - begin) * kSweepBatch;
   if (n >= room) return;
-  uint32_t x = (uint32_t)((unit * 131 + list * 37) % ((int64_t)max_col + 1));
-  if (n) x = entries[phase_entry(batch, list, n - 1)].x & ~kPhaseLast;
-  for (int i = n; i < room; ++i) entries[phase_entry(batch, list, i)] = uint2{x, 0u};
+  for (int i = n; i < room; ++i) entries[phase_entry(batch, list, i)] = uint2{kPhaseNull, 0u};
 }
 
 }  // namespace srbcrs

@@ -81,11 +81,12 @@ def test_second_run_builds_the_stream(gpu):
     assert free[0] - free[1] >= 8 * M * 16 and free[2] == free[1]
 
 
-# (M, K, columns per row, N, band): 64 columns with a ragged last chunk; 32 columns, all XCDs on one chunk
-# and chunks pinned; rows whose columns all lie in one phase; fewer columns than phases have bins
+# (M, K, columns per row, N, band): 64 columns with a ragged last chunk; 32 columns with 16 waves, all XCDs
+# on one chunk and chunks pinned; with 8 waves; rows whose columns all lie in one phase; mostly empty rows
 @pytest.mark.parametrize("policy", [("row", 0), ("split", 5)])
 @pytest.mark.parametrize("shape", [(6100, 50000, 9, 1008, 0), (210001, 49999, 4, 32, 0), (210000, 1990000, 4, 32, 0),
-                                   (70003, 70003, 20, 128, 200), (150000, 49160, 1, 128, 0)])
+                                   (66001, 52000, 30, 128, 0), (70003, 70003, 20, 128, 200),
+                                   (150000, 49160, 1, 128, 0)])
 def test_phase_sweep(gpu, shape, policy):
     """Widths and sizes at which the workgroups' rows are pooled."""
     import torch
