@@ -1897,7 +1897,7 @@ int srbcrs_csr_spmm(const int32_t* d_rowptr, const int32_t* d_colind, const floa
                        (reinterpret_cast<uintptr_t>(d_B) % (4 * vec)) ||
                        (reinterpret_cast<uintptr_t>(d_C) % (4 * vec))))
       vec /= 2;
-    srbcrs::CsrArgs a{d_rowptr, d_colind, d_values, d_B, d_C, M, (int)N, ldb, ldc};
+    srbcrs::CsrArgs a{d_rowptr, d_colind, d_values, d_B, d_C, M, (int)N, ldb, ldc, K};
     hip_check(srbcrs::launch_csr(a, vec, static_cast<hipStream_t>(stream)), "launch csr_spmm_rowwave");
   });
 }

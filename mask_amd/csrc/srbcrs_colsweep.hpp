@@ -56,17 +56,6 @@ constexpr int kSweepSlotShift = 24;
 constexpr int kSweepBatch = 8;   // entries per list and batch
 constexpr int kSweepLongBatch = 32;   // entries per batch of a long row (lists of entries are padded for it)
 
-// Lane q's value of each lane group to the group's lanes: one DPP row
-// broadcast for groups of 16 lanes, two (the upper half of the row written by
-// the second) for groups of 8.
-template <int LPG, int Q>
-__device__ __forceinline__ uint32_t group_bcast(uint32_t v) {
-  static_assert(LPG == 8 || LPG == 16, "lane groups of 8 or 16");
-  int r = __builtin_amdgcn_mov_dpp((int)v, 0x150 + Q, 0xf, 0xf, true);
-  if constexpr (LPG == 8) r = __builtin_amdgcn_update_dpp(r, (int)v, 0x158 + Q, 0xf, 0xc, false);
-  return (uint32_t)r;
-}
-
 struct SweepStream {
   const uint2* entries;
   const int* start;   // first entry of each list
@@ -143,23 +132,6 @@ __device__ __forceinline__ void sweep_long_row(const SweepStream& s, int r, int 
     __builtin_nontemporal_store(acc, sweep_out(d, col, ldc, Cout, partial));
   }
   if (__any(bad) && lane == 0) atomicMax(flag, token);
-}
-
-// Workgroup id of n_ids to row part wg (>= n_wg: none) and column chunk c.
-// swept = 0: chunks pinned to XCDs (xcd_remap over chunk-major ids, or chunk =
-// XCD % n_chunks where the chunks divide the 8 XCDs); 1: every XCD on the same
-// chunk at a time.
-__device__ __forceinline__ void sweep_chunk(int id, int n_ids, int n_wg, int n_chunks, int swept, int& wg, int& c) {
-  if (!swept && n_chunks <= kNumXcd && kNumXcd % n_chunks == 0) {
-    const int per = kNumXcd / n_chunks;
-    const int x = id % kNumXcd;
-    c = x % n_chunks;
-    wg = id / kNumXcd * per + x / n_chunks;
-  } else {
-    const int lid = swept ? id : (int)xcd_remap(id, n_ids);
-    c = lid / n_wg;
-    wg = lid % n_wg;
-  }
 }
 
 // One workgroup = WV waves of LG lists on one chunk of C columns.

@@ -84,6 +84,7 @@ struct CsrArgs {
   float* C;
   int M, N;
   int64_t ldb, ldc;
+  int64_t K;   // rows of B
 };
 
 hipError_t launch_row(const StreamArgs& a, const int* soff, int Mo, int vec, const RunOpts& o,

@@ -39,8 +39,39 @@ hipError_t launch_reduce(const ReduceArgs& a, int vec, hipStream_t st) {
   return hipGetLastError();
 }
 
-// vec: columns per lane per pass (64*vec divides N, or 1).
+template <int C>
+static hipError_t launch_csr_t(const CsrArgs& a, uint32_t bytes, hipStream_t st) {
+  const int n_chunks = (a.N + C - 1) / C;
+  const int64_t n_wg = ((int64_t)a.M + 1024 / C - 1) / (1024 / C);
+  int64_t grid = n_wg * n_chunks;
+  if (n_chunks <= kNumXcd && kNumXcd % n_chunks == 0) {
+    const int per = kNumXcd / n_chunks;
+    grid = (n_wg + per - 1) / per * kNumXcd;
+  }
+  if (grid > INT32_MAX) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((csr_spmm_rowgroup<C>), dim3((unsigned)grid), dim3(256), 0, st, a.rowptr, a.colind, a.values, a.B,
+                     bytes, a.C, a.M, a.N, (uint32_t)(a.ldb * 4), a.ldc, n_chunks, (int)n_wg);
+  return hipGetLastError();
+}
+
+// vec: columns per lane per pass of the wave kernel (64*vec divides N, or 1).
 hipError_t launch_csr(const CsrArgs& a, int vec, hipStream_t st) {
+  if (a.M == 0) return hipSuccess;
+  const uint64_t bytes = a.K > 0 ? ((uint64_t)(a.K - 1) * (uint64_t)a.ldb + (uint64_t)a.N) * 4u : 0u;
+  const bool quads = a.N % 4 == 0 && a.ldb % 4 == 0 && a.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(a.B) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(a.C) % 16 == 0;
+  // One row per lane group wherever float4 segments and 32-bit offsets fit,
+  // but on B so tall that no cache holds any of it, where whole 1 KB segments
+  // of a row per wave gather a little faster (100000 x 400000, 12 per row, N =
+  // 256: 186 / 195 us; at 384 columns, not whole segments, 355 / 280).  32
+  // columns where their slice of B is within reach of the L2 (K = 65536: 138 us,
+  // 64 columns 153; 150000: 184 / 176), 64 where theirs is in it (K = 8000: 18,
+  // 32 columns 20) or 32-column segments straddle cache lines (N = 100: 98 / 125).
+  if (quads && !(vec == 4 && a.K > 262144) && a.K < (int64_t(1) << 32) &&
+      bytes + (uint64_t)a.N * 4 < (uint64_t(1) << 32)) {
+    if (a.N % 32 || a.ldb % 32 || a.K <= 16384 || a.K > 131072) return launch_csr_t<64>(a, (uint32_t)bytes, st);
+    return launch_csr_t<32>(a, (uint32_t)bytes, st);
+  }
   const int n_chunks = (a.N + 64 * vec - 1) / (64 * vec);
   const int64_t nwg = ((int64_t)a.M + 3) / 4 * n_chunks;
   if (nwg == 0) return hipSuccess;

@@ -72,6 +72,34 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t id, int64_t n) {
   return x * q + (x < r ? x : r) + t;
 }
 
+// Workgroup id of n_ids to row part wg (>= n_wg: none) and column chunk c.
+// swept = 0: chunks pinned to XCDs (xcd_remap over chunk-major ids, or chunk =
+// XCD % n_chunks where the chunks divide the 8 XCDs); 1: every XCD on the same
+// chunk at a time.
+__device__ __forceinline__ void sweep_chunk(int id, int n_ids, int n_wg, int n_chunks, int swept, int& wg, int& c) {
+  if (!swept && n_chunks <= kNumXcd && kNumXcd % n_chunks == 0) {
+    const int per = kNumXcd / n_chunks;
+    const int x = id % kNumXcd;
+    c = x % n_chunks;
+    wg = id / kNumXcd * per + x / n_chunks;
+  } else {
+    const int lid = swept ? id : (int)xcd_remap(id, n_ids);
+    c = lid / n_wg;
+    wg = lid % n_wg;
+  }
+}
+
+// Lane q's value of each lane group to the group's lanes: one DPP row
+// broadcast for groups of 16 lanes, two (the upper half of the row written by
+// the second) for groups of 8.
+template <int LPG, int Q>
+__device__ __forceinline__ uint32_t group_bcast(uint32_t v) {
+  static_assert(LPG == 8 || LPG == 16, "lane groups of 8 or 16");
+  int r = __builtin_amdgcn_mov_dpp((int)v, 0x150 + Q, 0xf, 0xf, true);
+  if constexpr (LPG == 8) r = __builtin_amdgcn_update_dpp(r, (int)v, 0x158 + Q, 0xf, 0xc, false);
+  return (uint32_t)r;
+}
+
 // Block geometry: BH x BW blocks, H = BH/16 row halves, Q = BW/8 units.
 template <int BH, int BW>
 struct Shape {
@@ -770,11 +798,91 @@ __global__ __launch_bounds__(256) void zero_rows(T* __restrict__ C, const int* _
   }
 }
 
-// CSR SpMM, one wave per (row, column chunk): lane owns VEC consecutive
-// columns of a 64*VEC-column chunk.  Edge-ordered fp32 accumulation, the
-// arithmetic of the reference's csr_spmm_value_kernel (examples/src_fp32/
-// sr_bcrs/testbed/SRBCRSSpMM_kernel.cu:66-87), laid out for wave64 vector
-// loads.  The grid is chunk-major (every row's first chunk before any second
+// CSR SpMM, C columns of a row on a lane group of C / 4 lanes.  Edge-ordered
+// fp32 accumulation, the arithmetic of the reference's csr_spmm_value_kernel
+// (examples/src_fp32/sr_bcrs/testbed/SRBCRSSpMM_kernel.cu:66-87).  Bound by
+// the gathers' L2 misses: narrow column chunks, each on its own XCDs, make an
+// XCD's share of B small.  Measured against a wave per row and 256-column
+// chunk (one MI355X, us): 50021 x 65536, 24 per row, N = 256 169 -> 138, N = 64
+// 48 -> 35, N = 16 40 -> 15; power-law, 200000 nodes, N = 256 925 -> 611.
+//
+// A group's lanes load 8 entries of its row at a time and broadcast them; past
+// the row's end the gather lies past B's end (it returns 0 and fetches
+// nothing) and the value is -0, which changes no sum.
+template <int C>
+__global__ __launch_bounds__(256) void csr_spmm_rowgroup(const int* __restrict__ rowptr,
+                                                         const int* __restrict__ colind,
+                                                         const float* __restrict__ values,
+                                                         const float* __restrict__ B, uint32_t b_bytes,
+                                                         float* __restrict__ Cout, int M, int N, uint32_t ldb4,
+                                                         int64_t ldc, int n_chunks, int n_wg) {
+  constexpr int LPG = C / 4, LG = 64 / LPG, U = 8;
+  int wg, c;
+  sweep_chunk((int)blockIdx.x, (int)gridDim.x, n_wg, n_chunks, 0, wg, c);
+  if (wg >= n_wg) return;
+  const int lane = threadIdx.x & 63, grp = lane / LPG, sub = lane % LPG;
+  const int64_t row = ((int64_t)wg * 4 + (threadIdx.x >> 6)) * LG + grp;
+  int e0 = 0, n = 0;
+  if (row < M) {
+    e0 = rowptr[row];
+    n = rowptr[row + 1] - e0;
+  }
+  int most = n;
+#pragma unroll
+  for (int d = LPG; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d));
+  most = __builtin_amdgcn_readfirstlane(most);
+  const int col = c * C + 4 * sub;
+  const uint32_t boff = (uint32_t)(col < N - 4 ? col : N - 4) * 4u;   // columns past N: repeat the last (not stored)
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, (int)b_bytes, 0x00020000);
+  f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+  uint32_t off, v;
+  auto fetch = [&](int i) {
+    i += lane & (U - 1);
+    off = b_bytes;
+    v = 0x80000000u;
+    if (i < n) {
+      off = (uint32_t)colind[(int64_t)e0 + i] * ldb4;
+      v = __builtin_bit_cast(uint32_t, values[(int64_t)e0 + i]);
+    }
+  };
+  fetch(0);
+  for (int i = 0; i < most; i += U) {
+    f4 b[U];
+#define SRBCRS_GATHER(q)                                               \
+  b[q] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128( \
+                                    rs, group_bcast<LPG, q>(off) + boff, 0, 0))
+    SRBCRS_GATHER(0);
+    SRBCRS_GATHER(1);
+    SRBCRS_GATHER(2);
+    SRBCRS_GATHER(3);
+    SRBCRS_GATHER(4);
+    SRBCRS_GATHER(5);
+    SRBCRS_GATHER(6);
+    SRBCRS_GATHER(7);
+#undef SRBCRS_GATHER
+    const uint32_t w = v;
+    fetch(i + U);
+#define SRBCRS_ADD(q)                                                                  \
+  {                                                                                    \
+    const float a = __builtin_bit_cast(float, group_bcast<LPG, q>(w));                 \
+    _Pragma("unroll") for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(a, b[q][e], acc[e]); \
+  }
+    SRBCRS_ADD(0);
+    SRBCRS_ADD(1);
+    SRBCRS_ADD(2);
+    SRBCRS_ADD(3);
+    SRBCRS_ADD(4);
+    SRBCRS_ADD(5);
+    SRBCRS_ADD(6);
+    SRBCRS_ADD(7);
+#undef SRBCRS_ADD
+  }
+  if (row < M && col < N) __builtin_nontemporal_store(acc, reinterpret_cast<f4*>(Cout + row * ldc + col));
+}
+
+// The same with one wave per (row, column chunk), for operands that float4
+// segments do not fit: lane owns VEC consecutive columns of a 64*VEC-column
+// chunk.  The grid is chunk-major (every row's first chunk before any second
 // chunk), which keeps the B columns in flight narrow: 17-22 % faster than
 // looping over the chunks inside the wave on the uniform and R-MAT
 // workloads.  UNROLL B rows are loaded before their FMAs.

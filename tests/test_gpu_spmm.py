@@ -168,6 +168,36 @@ def test_csr_fallback(gpu):
         assert_gate(gate(out.cpu().numpy(), rowptr, colind, values, B, M))
 
 
+# (M, K, N, ldb): one row, columns past a segment, both segment widths, row tails, operands that float4
+# segments do not fit, and B past what the narrow segments take
+@pytest.mark.parametrize("shape", [(1, 5, 4, 4), (33, 300, 36, 36), (257, 20000, 64, 96), (77, 20000, 100, 100),
+                                   (130, 140000, 32, 32), (65, 262200, 256, 256), (130, 20000, 64, 67)])
+def test_csr_row_groups(gpu, shape):
+    """Every row length around the 8 entries loaded at a time; what B holds
+    past the referenced rows does not reach the output."""
+    torch = _torch()
+    from mask_amd import _capi
+    M, K, N, ldb = shape
+    _say("csr row groups", shape)
+    rng = np.random.default_rng(M)
+    lens = np.array([0, 1, 7, 8, 9, 16, 33, 3])[np.arange(M) % 8]
+    rowptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    colind = rng.integers(1, K - 1, rowptr[-1]).astype(np.int32)
+    values = rng.uniform(-1, 1, colind.size).astype(np.float32)
+    B = rng.uniform(-1, 1, (K, ldb)).astype(np.float32)
+    B[[0, -1]] = np.nan
+    B[:, N:] = np.nan
+    out = torch.full((M + 1, N), 7.0, device="cuda")
+    dev = [torch.from_numpy(a).cuda() for a in (rowptr, colind, values, B)]
+    _capi.check(_capi.lib().srbcrs_csr_spmm(*(t.data_ptr() for t in dev[:3]), M, colind.size, int(colind.max(initial=0)),
+                                            dev[3].data_ptr(), K, N, ldb, out.data_ptr(), N,
+                                            torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert bool((out[M] == 7.0).all())
+    B[[0, -1]] = 0.0
+    assert_gate(gate(out[:M].cpu().numpy(), rowptr, colind, values, np.ascontiguousarray(B[:, :N]), M))
+
+
 @pytest.mark.parametrize("blk", [(16, 8), (32, 32)])
 def test_knobs_are_bitwise_invariant(gpu, blk):
     """Depth, tile_b, workgroup width, grid order and windows-per-wave change
