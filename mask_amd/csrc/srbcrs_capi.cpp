@@ -791,6 +791,15 @@ bool sweep_wanted(const srbcrs_plan& plan) {
 const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_build, hipStream_t st) {
   const srbcrs::ColSweepTasks t = sweep_tasks(plan);
   const int64_t rows = (int64_t)t.n * 16;
+  // Short rows whose B rows hardly any other row reads: nothing to share, and
+  // the block kernels' 64-column gathers take less than the sweep's lists and
+  // its second launch (us, sweep / block: 5710 x 141462, 9 per row, N = 512 26 /
+  // 23; 100000 x 400000, 4 per row, N = 256 98 / 81; but 3000 x 200000, 30 per
+  // row, N = 256 19 / 39, and N = 96, where the block kernels take 32 columns,
+  // 20000 x 300000, 10 per row 19 / 25).
+  if (N % 64 == 0 && plan.n_apacked <= 2 * ((int64_t)plan.max_col + 1) &&
+      plan.n_apacked <= 11 * (int64_t)plan.num_nodes)
+    return nullptr;
   // the layouts to try: the phase sweep's, where it is the faster one, and the
   // lists' (keyed by minus the rows per half, and the rows per list)
   const int layouts[2] = {-srbcrs::phasesweep_rows(rows, (int)N, (int64_t)plan.max_col + 1),

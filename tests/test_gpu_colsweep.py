@@ -110,6 +110,28 @@ def test_phase_sweep(gpu, shape, policy):
     assert not bool(torch.isfinite(_check(plan, B, (shape, "inf"))).all())
 
 
+@pytest.mark.parametrize("K,N,built", [(300000, 256, False), (300000, 224, True), (60000, 256, True)])
+def test_short_rows_without_shared_columns(gpu, K, N, built):
+    """Ten values a row and under two a column at whole 64-column chunks: the
+    block kernels stay, and no stream is built."""
+    import torch
+    M = 20000
+    rng = np.random.default_rng(K)
+    cols = np.sort(rng.integers(0, K, (M, 10)), axis=1).astype(np.int32).ravel()
+    cols[-1] = K - 1
+    plan = _plan((np.arange(M + 1, dtype=np.int32) * 10, cols, rng.uniform(-1, 1, M * 10).astype(np.float32)), M)
+    print("[case] short rows", K, N, flush=True)
+    B, out = torch.rand((K, N), device="cuda"), torch.empty((M, N), device="cuda")
+    plan.trim()
+    plan.run(B, out)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    plan.run(B, out)
+    torch.cuda.synchronize()
+    assert (torch.cuda.mem_get_info()[0] < free) == built
+    _check(plan, B, (K, N))
+
+
 @pytest.mark.parametrize("policy", [("row", 0), ("split", 7)])
 def test_non_finite_dense_values(gpu, policy):
     """An infinity or NaN of B poisons every row of the windows whose blocks
