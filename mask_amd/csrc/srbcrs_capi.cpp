@@ -378,10 +378,12 @@ Schedule* build_schedule(const int32_t* soff, int32_t Mo, const char* policy_c, 
 
 // ---- device memory helpers ------------------------------------------------
 
+// reuse: from kept memory too (conversions; what a run allocates goes through
+// hipMalloc, so that under graph capture it is refused whatever is kept)
 template <class T>
-T* dev_alloc(size_t n) {
+T* dev_alloc(size_t n, bool reuse = false) {
   if (n == 0) n = 1;
-  void* p = srbcrs::pool_alloc(n * sizeof(T));
+  void* p = srbcrs::pool_alloc(n * sizeof(T), !reuse);
   if (!p) fail(SRBCRS_ENOMEM, "allocation of %zu bytes of device memory failed", n * sizeof(T));
   return static_cast<T*>(p);
 }
@@ -655,10 +657,10 @@ void create_on_device(srbcrs_plan& plan, const int32_t* rowptr, const int32_t* c
                       const float* values, hipStream_t st) {
   const int32_t Mo = (plan.num_nodes + plan.blk_h - 1) / plan.blk_h;
   plan.Mo = Mo;
-  plan.d_soff = dev_alloc<int32_t>((size_t)Mo + 1);
-  plan.d_e2r = dev_alloc<int32_t>((size_t)plan.nnz);
-  plan.d_e2c = dev_alloc<int32_t>((size_t)plan.nnz);
-  plan.d_bp = dev_alloc<int32_t>((size_t)Mo);
+  plan.d_soff = dev_alloc<int32_t>((size_t)Mo + 1, true);
+  plan.d_e2r = dev_alloc<int32_t>((size_t)plan.nnz, true);
+  plan.d_e2c = dev_alloc<int32_t>((size_t)plan.nnz, true);
+  plan.d_bp = dev_alloc<int32_t>((size_t)Mo, true);
   plan.h_soff.resize((size_t)Mo + 1);
   srbcrs::DeviceConvertIn in{rowptr, colind, values, plan.num_nodes, plan.nnz, plan.blk_h, plan.blk_w,
                              plan.d_e2r, plan.d_e2c, plan.d_bp};

@@ -60,7 +60,7 @@ std::list<Block> take(Pool& P, int device, size_t room) {
 
 }  // namespace
 
-void* pool_alloc(size_t bytes) {
+void* pool_alloc(size_t bytes, bool fresh) {
   Pool& P = pool();
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) {
@@ -68,7 +68,7 @@ void* pool_alloc(size_t bytes) {
     return nullptr;
   }
   const size_t want = size_class(bytes);
-  {
+  if (!fresh) {
     std::lock_guard<std::mutex> lock(P.mu);
     auto best = P.kept.end();
     for (auto it = P.kept.begin(); it != P.kept.end(); ++it)
@@ -84,8 +84,10 @@ void* pool_alloc(size_t bytes) {
     }
   }
   Block b{nullptr, want, dev};
-  if (hipMalloc(&b.p, want) != hipSuccess) {
+  const hipError_t e = hipMalloc(&b.p, want);
+  if (e != hipSuccess) {
     (void)hipGetLastError();
+    if (e != hipErrorOutOfMemory) return nullptr;
     pool_release(dev);
     if (hipMalloc(&b.p, want) != hipSuccess) {
       (void)hipGetLastError();

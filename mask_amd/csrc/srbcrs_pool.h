@@ -15,8 +15,9 @@ namespace srbcrs {
 constexpr size_t kPoolBytes = size_t(4) << 30;
 
 // Device memory on the current device, at least `bytes`; null: none left.
-// A block taken from the pool is idle: no queued work uses it.
-void* pool_alloc(size_t bytes);
+// A block taken from the pool is idle: no queued work uses it.  fresh: always
+// through hipMalloc, which graph capture refuses.
+void* pool_alloc(size_t bytes, bool fresh = false);
 // Give a block back.  No queued work may still use it, on any stream.
 void pool_free(void* p);
 // hipFree of a block from pool_alloc.
