@@ -331,24 +331,28 @@ __global__ __launch_bounds__(64) void k_big_offsets(ConvArgs a, int64_t* __restr
 }
 
 // Windows too long for LDS: (index in a.big << 32 | column) keys of all of
-// them, one after the other, for one device-wide stable sort.
-__global__ __launch_bounds__(256) void k_big_keys(ConvArgs a, const int64_t* __restrict__ off,
+// them, one after the other, for one device-wide stable sort.  A row of the
+// grid takes every kBigRows-th window.
+constexpr int kBigRows = 64;   // times 16 workgroups a window: 4 per CU
+__global__ __launch_bounds__(256) void k_big_keys(ConvArgs a, int n_big, const int64_t* __restrict__ off,
                                                   uint64_t* __restrict__ keys, int* __restrict__ edges) {
-  const int b = blockIdx.y, w = a.big[b];
-  const int64_t r0 = (int64_t)w * a.bh;
-  const int64_t r1 = r0 + a.bh < a.num_nodes ? r0 + a.bh : a.num_nodes;
-  const int e0 = a.rowptr[r0], n = a.rowptr[r1] - e0;
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    const int c = a.colind[e0 + i];
-    if (c < 0) a.head->negative = 1;
-    keys[off[b] + i] = ((uint64_t)(uint32_t)b << 32) | (uint32_t)c;
-    edges[off[b] + i] = e0 + i;
-    int lo = 0, hi = (int)(r1 - r0);
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) / 2;
-      if (a.rowptr[r0 + mid] <= e0 + i) lo = mid; else hi = mid;
+  for (int b = blockIdx.y; b < n_big; b += gridDim.y) {
+    const int w = a.big[b];
+    const int64_t r0 = (int64_t)w * a.bh;
+    const int64_t r1 = r0 + a.bh < a.num_nodes ? r0 + a.bh : a.num_nodes;
+    const int e0 = a.rowptr[r0], n = a.rowptr[r1] - e0;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+      const int c = a.colind[e0 + i];
+      if (c < 0) a.head->negative = 1;
+      keys[off[b] + i] = ((uint64_t)(uint32_t)b << 32) | (uint32_t)c;
+      edges[off[b] + i] = e0 + i;
+      int lo = 0, hi = (int)(r1 - r0);
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) / 2;
+        if (a.rowptr[r0 + mid] <= e0 + i) lo = mid; else hi = mid;
+      }
+      a.e2r[e0 + i] = (int)r0 + lo;
     }
-    a.e2r[e0 + i] = (int)r0 + lo;
   }
 }
 
@@ -617,13 +621,9 @@ hipError_t device_convert(const DeviceConvertIn& in, DeviceConvertOut& out, Devi
     if (!k0 || !k1 || !i0 || !i1 || !d_off) return hipErrorOutOfMemory;
     hipLaunchKernelGGL(k_big_offsets, dim3(1), dim3(64), 0, st, a, d_off);
     SRBCRS_TRY(hipGetLastError());
-    for (int b = 0; b < h.n_big; b += 32768) {   // grid y limit
-      const int m = h.n_big - b < 32768 ? h.n_big - b : 32768;
-      ConvArgs ab = a;
-      ab.big = a.big + b;
-      hipLaunchKernelGGL(k_big_keys, dim3(16, (unsigned)m), dim3(256), 0, st, ab, d_off + b, k0, i0);
-      SRBCRS_TRY(hipGetLastError());
-    }
+    hipLaunchKernelGGL(k_big_keys, dim3(16, (unsigned)(h.n_big < kBigRows ? h.n_big : kBigRows)), dim3(256), 0, st, a,
+                       h.n_big, d_off, k0, i0);
+    SRBCRS_TRY(hipGetLastError());
     hipcub::DoubleBuffer<uint64_t> kb(k0, k1);
     hipcub::DoubleBuffer<int> ib(i0, i1);
     size_t bytes = 0;

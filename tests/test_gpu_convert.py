@@ -104,6 +104,26 @@ def test_device_conversion_window_lengths(gpu, blk, K):
         del plan
 
 
+def test_device_conversion_many_long_windows(gpu):
+    """More windows past the LDS classes than the key pass has grid rows: each
+    keeps its own entries (the columns of neighbours overlap)."""
+    import torch
+    from mask_amd.SRBCRSSpMM import Plan
+    windows, K = 131, 40_000
+    rng = np.random.default_rng(1)
+    lens = rng.integers(16385, 17000, windows)
+    M = windows * 16
+    rp = np.zeros(M + 1, np.int64)
+    for w, n in enumerate(lens):
+        rp[w * 16 + 1:w * 16 + 17] = np.bincount(rng.integers(0, 16, n), minlength=16)
+    rp = np.cumsum(rp).astype(np.int32)
+    ci = np.concatenate([np.sort(rng.choice(K, rp[r + 1] - rp[r], replace=False)) for r in range(M)]).astype(np.int32)
+    vv = rng.uniform(-1, 1, ci.size).astype(np.float32)
+    _say("convert long windows", windows, ci.size)
+    t = lambda a: torch.from_numpy(a).cuda()
+    _same(_arrays(Plan(t(rp), t(ci), t(vv), M)), oracle.convert(rp, ci, vv, M))
+
+
 def test_device_conversion_rejects_malformed(gpu):
     import torch
     from mask_amd._capi import SrbcrsError
