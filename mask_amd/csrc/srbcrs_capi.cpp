@@ -649,7 +649,12 @@ void create_packed(srbcrs_plan& plan, const int32_t* rp, const int32_t* ci, cons
 }
 
 void* conv_alloc(void*, size_t bytes) { return srbcrs::pool_alloc(bytes); }
-void conv_free(void*, void* p) { srbcrs::pool_free(p); }
+void conv_free(void*, void* p, bool idle) {
+  if (idle)
+    srbcrs::pool_free(p);
+  else
+    srbcrs::pool_drop(p);
+}
 
 // Canonical conversion of a device CSR on the device (srbcrs_convert.hip),
 // with the compact copy of the block values where there is room for it.

@@ -217,11 +217,11 @@ static hipError_t build_phasesweep(const ColSweepIn& in, ColSweep& out, DeviceAl
     return p;
   };
   auto cleanup = [&](hipError_t e) {
-    if (e != hipSuccess) (void)hipStreamSynchronize(st);   // queued kernels may use what is given back
-    for (void* p : temps) dfree(ctx, p);
+    const bool idle = e == hipSuccess || hipStreamSynchronize(st) == hipSuccess;   // queued kernels may use these
+    for (void* p : temps) dfree(ctx, p, idle);
     if (e != hipSuccess) {
       auto drop = [&](auto*& p) {
-        if (p) dfree(ctx, (void*)p);
+        if (p) dfree(ctx, (void*)p, idle);
         p = nullptr;
       };
       drop(out.entries);
@@ -335,12 +335,13 @@ hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc
   if (cap > INT32_MAX) return hipErrorInvalidValue;
   int *len = nullptr, *hist = nullptr, *vrow = nullptr, *list_len = nullptr, *lvrow = nullptr;
   unsigned long long* total = nullptr;
+  bool idle = true;
   auto drop = [&](auto*& p) {
-    if (p) dfree(ctx, (void*)p);
+    if (p) dfree(ctx, (void*)p, idle);
     p = nullptr;
   };
   auto cleanup = [&](hipError_t e) {
-    if (e != hipSuccess) (void)hipStreamSynchronize(st);   // queued kernels may use what is given back
+    idle = e == hipSuccess || hipStreamSynchronize(st) == hipSuccess;   // queued kernels may use these
     drop(len);
     drop(hist);
     drop(vrow);

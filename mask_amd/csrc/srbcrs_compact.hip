@@ -84,17 +84,17 @@ hipError_t device_compact(const float* val, int64_t n_blocks, int blk_h, int blk
   uint32_t* bases = nullptr;
   void* tmp = nullptr;
   uint32_t* tail = nullptr;
-  auto cleanup = [&] {
-    if (counts) dfree(ctx, counts);
-    if (bases) dfree(ctx, bases);
-    if (tmp) dfree(ctx, tmp);
-    if (tail) dfree(ctx, tail);
+  auto cleanup = [&](bool idle) {
+    if (counts) dfree(ctx, counts, idle);
+    if (bases) dfree(ctx, bases, idle);
+    if (tmp) dfree(ctx, tmp, idle);
+    if (tail) dfree(ctx, tail, idle);
   };
   auto fail = [&](hipError_t e) {
-    (void)hipStreamSynchronize(st);   // queued kernels may use what is given back
-    cleanup();
-    if (out.words) dfree(ctx, out.words);
-    if (out.packed) dfree(ctx, out.packed);
+    const bool idle = hipStreamSynchronize(st) == hipSuccess;   // queued kernels may use what is given back
+    cleanup(idle);
+    if (out.words) dfree(ctx, out.words, idle);
+    if (out.packed) dfree(ctx, out.packed, idle);
     out = CompactOut{};
     return e;
   };
@@ -134,7 +134,7 @@ hipError_t device_compact(const float* val, int64_t n_blocks, int blk_h, int blk
   SRBCRS_STEP(hipGetLastError());
   SRBCRS_STEP(hipStreamSynchronize(st));
 #undef SRBCRS_STEP
-  cleanup();
+  cleanup(true);
   return hipSuccess;
 }
 

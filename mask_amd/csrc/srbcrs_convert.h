@@ -45,9 +45,9 @@ struct DeviceConvertOut {
 };
 
 typedef void* (*DeviceAlloc)(void* ctx, size_t bytes);
-typedef void (*DeviceFree)(void* ctx, void* p);   // called when no queued work uses p any more
+typedef void (*DeviceFree)(void* ctx, void* p, bool idle);   // idle: no queued work uses p any more
 
-// Returns with the stream's work done.
+// Returns with the stream's work done, and its error if it failed.
 hipError_t device_convert(const DeviceConvertIn& in, DeviceConvertOut& out, DeviceAlloc alloc,
                           DeviceFree dfree, void* ctx, hipStream_t st);
 

@@ -547,15 +547,22 @@ struct Temps {
   hipStream_t st;
   void* p[24];
   int n = 0;
+  bool waited = false, idle = false;
   template <class T>
   T* get(size_t count) {
     void* q = n < 24 ? alloc(ctx, (count ? count : 1) * sizeof(T)) : nullptr;
     if (q) p[n++] = q;
     return static_cast<T*>(q);
   }
+  hipError_t wait() {
+    const hipError_t e = hipStreamSynchronize(st);
+    waited = true;
+    idle = e == hipSuccess;
+    return e;
+  }
   ~Temps() {
-    (void)hipStreamSynchronize(st);
-    for (int i = 0; i < n; ++i) dfree(ctx, p[i]);
+    if (!waited) (void)wait();
+    for (int i = 0; i < n; ++i) dfree(ctx, p[i], idle);
   }
 };
 
@@ -653,8 +660,8 @@ hipError_t device_convert(const DeviceConvertIn& in, DeviceConvertOut& out, Devi
   out.compact.words = (uint2*)need(2 * (size_t)n_words);
   out.compact.packed = (float*)need((size_t)(n_packed + kPackedPad));
   if (!out.compact.words || !out.compact.packed) {
-    if (out.compact.words) dfree(ctx, out.compact.words);
-    if (out.compact.packed) dfree(ctx, out.compact.packed);
+    if (out.compact.words) dfree(ctx, out.compact.words, true);
+    if (out.compact.packed) dfree(ctx, out.compact.packed, true);
     out.compact = CompactOut{};
   } else {
     out.compact.n_packed = n_packed;
@@ -666,7 +673,8 @@ hipError_t device_convert(const DeviceConvertIn& in, DeviceConvertOut& out, Devi
   else
     hipLaunchKernelGGL((k_blocks<32, 32, 64>), dim3((unsigned)((out.total + 15) / 16)), dim3(256), 0, st, a, Mo,
                        out.soff, vbase, out.total, out.sidx, out.val, out.compact.words, out.compact.packed);
-  return hipGetLastError();   // the temporaries' release waits for the stream
+  SRBCRS_TRY(hipGetLastError());
+  return t.wait();
 #undef SRBCRS_TRY
 }
 

@@ -1,0 +1,89 @@
+"""The library's host code against a stand-in HIP runtime (tests/c/fake_hip.c,
+no GPU): what it does when calls fail, under graph capture, and with device
+memory over many calls.  Each test is a process of its own."""
+from __future__ import annotations
+
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+
+PRELUDE = """
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)   # before the library: its HIP calls come here
+import numpy as np
+from mask_amd import _capi
+L = _capi.lib()
+fake.fake_live_bytes.restype = ctypes.c_size_t
+fake.fake_launches.argtypes = [ctypes.c_char_p]
+fake.fake_launches.restype = fake.fake_calls.restype = fake.fake_mallocs.restype = ctypes.c_long
+launches = lambda part: fake.fake_launches(part.encode())
+error = lambda: L.srbcrs_last_error().decode()
+
+def d2h(data):
+    data = np.ascontiguousarray(data)
+    fake.fake_d2h(ctypes.c_size_t(data.nbytes), ctypes.c_void_p(data.ctypes.data))
+
+def csr(M, K, per_row, seed=0):
+    cols = np.sort(np.random.default_rng(seed).integers(0, K, (M, per_row)), axis=1).astype(np.int32).ravel()
+    return (np.arange(M + 1, dtype=np.int32) * per_row, cols, np.ones(cols.size, np.float32))
+
+def create(c, M, on_device):
+    h = ctypes.c_void_p()
+    rc = L.srbcrs_plan_create(*(a.ctypes.data for a in c), M, c[1].size, 16, 8, on_device, None, ctypes.byref(h))
+    return rc, h
+
+def head(blocks, stored, max_col):
+    # what the conversion's kernels would have counted (struct Head)
+    d2h(np.array([blocks, stored, 0, 0, 0, 0, max_col + 1, 0, 0, 0], np.uint32))
+
+def sparse_plan(M, K, per_row):
+    # a plan converted on the host, whose compact copy holds all its values
+    c = csr(M, K, per_row)
+    d2h(np.array([0, c[1].size], np.uint32))
+    rc, h = create(c, M, 0)
+    assert rc == 0, error()
+    fake.fake_d2h(ctypes.c_size_t(0), None)
+    return h
+
+def run(h, M, K, N, B=np.zeros(1 << 22, np.float32), C=np.zeros(1 << 22, np.float32)):
+    assert K * N <= B.size and M * N <= C.size
+    align = lambda a: (a.ctypes.data + 15) // 16 * 16
+    return L.srbcrs_run(h, align(B), K, N, N, align(C), N, M, None)
+"""
+
+
+@pytest.fixture(scope="session")
+def fake_hip(tmp_path_factory):
+    so = tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so"
+    subprocess.run(["gcc", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-o", str(so),
+                    str(ROOT / "tests" / "c" / "fake_hip.c")], check=True)
+    return so
+
+
+def _run(fake_hip, code):
+    r = subprocess.run([sys.executable, "-c", PRELUDE + code, str(fake_hip)], cwd=ROOT, capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stdout[-1000:] + r.stderr[-2000:]
+
+
+# the conversion's synchronisations: after the window scan, and at its end
+@pytest.mark.parametrize("good_syncs", [0, 1])
+def test_conversion_reports_a_failure_of_its_kernels(fake_hip, good_syncs):
+    """An error that shows only when the stream is waited for is the call's
+    result, and none of the memory is kept for another conversion."""
+    _run(fake_hip, f"""
+c = csr(320, 500, 5)
+head(900, c[1].size, 499)
+fake.fake_fail_sync({good_syncs})
+rc, h = create(c, 320, 1)
+assert launches("k_blocks") == {good_syncs}
+assert rc == _capi.SRBCRS_EHIP and not h.value, (rc, error())
+assert fake.fake_live_blocks() == 0
+fake.fake_fail_sync(-1)
+rc, h = create(c, 320, 1)
+assert rc == 0, error()
+""")
