@@ -1115,6 +1115,12 @@ int srbcrs_plan_create_ex(const int32_t* rowptr, const int32_t* colind, const fl
     if (canonical && is_device == 1) {
       // device CSR converted in HBM (no host round trip)
       if (!rowptr || (nnz > 0 && (!colind || !values))) fail(SRBCRS_EINVAL, "NULL CSR array");
+      // its arrays may come from kept memory, which no hipMalloc refuses:
+      // nothing may be recorded into the graph before the first wait fails
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      hip_check(hipStreamIsCapturing(st, &cs), "hipStreamIsCapturing");
+      if (cs != hipStreamCaptureStatusNone)
+        fail(SRBCRS_ENOMEM, "a conversion allocates device memory, which stream capture does not permit");
       auto plan = std::make_unique<srbcrs_plan>();
       hip_check(hipGetDevice(&plan->device), "hipGetDevice");
       plan->num_nodes = num_nodes;

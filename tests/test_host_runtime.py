@@ -87,3 +87,21 @@ fake.fake_fail_sync(-1)
 rc, h = create(c, 320, 1)
 assert rc == 0, error()
 """)
+
+
+def test_conversion_under_capture_is_refused_before_any_call(fake_hip):
+    """Also with kept memory at hand: nothing is recorded into the graph."""
+    _run(fake_hip, """
+c = csr(320, 500, 5)
+head(900, c[1].size, 499)
+rc, h = create(c, 320, 1)
+assert rc == 0, error()
+L.srbcrs_plan_destroy(h)
+calls, mallocs = fake.fake_calls(), fake.fake_mallocs()
+fake.fake_capture(1)
+rc, h = create(c, 320, 1)
+assert rc == _capi.SRBCRS_ENOMEM and "capture" in error(), (rc, error())
+assert (fake.fake_calls(), fake.fake_mallocs()) == (calls, mallocs)
+fake.fake_capture(0)
+assert create(c, 320, 1)[0] == 0, error()
+""")
