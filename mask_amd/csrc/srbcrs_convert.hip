@@ -40,7 +40,7 @@ struct Head {
   unsigned long long totals;       // blocks | stored values << 32
   unsigned long long big_entries;
   int bad, negative;
-  int max_col1;                    // largest column + 1 (all zero at the start)
+  unsigned max_col1;               // largest column + 1 (all zero at the start)
   int n_list[2], n_big;            // windows listed for k_listed_windows<0 / 1>, and longer ones
 };
 
@@ -71,7 +71,7 @@ struct ConvArgs {
 // Entries of a window sorted in LDS: by 256, 512 and 1024 threads.
 constexpr int kClass[3] = {2048, 4096, 16384};
 
-__device__ __forceinline__ void note_max(int* p, int v) {
+__device__ __forceinline__ void note_max(unsigned* p, unsigned v) {
   if (v > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p, v);
 }
 
@@ -265,7 +265,7 @@ __device__ __forceinline__ void sort_window(const ConvArgs& a, int w, const int*
                  [&](int i) { return e0 + (int)(uint32_t)key[i]; });
   if (threadIdx.x == 0) {
     put_count(a, w, firsts, stored);
-    note_max(&a.head->max_col1, *most < INT32_MAX ? *most + 1 : INT32_MAX);
+    note_max(&a.head->max_col1, (unsigned)*most + 1u);
   }
 }
 
@@ -372,8 +372,7 @@ __global__ __launch_bounds__(1024) void k_big_rank(ConvArgs a, const int64_t* __
                     [&](int i) { return ed[i]; });
   if (threadIdx.x == 0) {
     put_count(a, w, firsts, stored);
-    const int c = (int)(uint32_t)k[n - 1];
-    note_max(&a.head->max_col1, c < INT32_MAX ? c + 1 : c);
+    note_max(&a.head->max_col1, (unsigned)(uint32_t)k[n - 1] + 1u);   // (negative columns refuse the matrix)
   }
 }
 
@@ -647,7 +646,7 @@ hipError_t device_convert(const DeviceConvertIn& in, DeviceConvertOut& out, Devi
     out.bad = h.bad ? 1 : 2;
     return hipSuccess;
   }
-  out.max_col = h.max_col1 - 1;
+  out.max_col = (int)(h.max_col1 - 1u);
   out.total = (int64_t)(h.totals & 0xffffffffu);
   const int64_t n_packed = (int64_t)(h.totals >> 32);
   const int64_t n_words = out.total * bh * bw / 32;

@@ -124,6 +124,19 @@ def test_device_conversion_many_long_windows(gpu):
     _same(_arrays(Plan(t(rp), t(ci), t(vv), M)), oracle.convert(rp, ci, vv, M))
 
 
+@pytest.mark.parametrize("n", [3, 3000, 17000])   # windows sorted by 256 and 512 threads, and past LDS
+def test_device_conversion_largest_column(gpu, n):
+    """max_col is exact up to the largest column index: a dense operand must
+    have more rows than it."""
+    import torch
+    from mask_amd.SRBCRSSpMM import Plan
+    ci = np.arange(n, dtype=np.int32)
+    ci[-1] = 2**31 - 1
+    _say("convert largest column", n)
+    plan = Plan(*(torch.from_numpy(a).cuda() for a in (np.array([0, n], np.int32), ci, np.ones(n, np.float32))), 1)
+    assert plan.max_col == 2**31 - 1
+
+
 def test_device_conversion_rejects_malformed(gpu):
     import torch
     from mask_amd._capi import SrbcrsError
