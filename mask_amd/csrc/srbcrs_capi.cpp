@@ -470,8 +470,9 @@ struct srbcrs_plan {
   struct Sweep {
     std::set<int64_t> seen;   // widths that have run
     int32_t longest = 0;   // blocks of the schedule's longest task
-    bool failed = false;   // cannot be built: the block kernels run, with the same bits
+    bool unfit = false;   // the matrix does not fit this layout
     bool built = false;
+    int skip = 0, backoff = 1;   // runs before the next attempt after a build that failed, and after the next failure
     srbcrs::ColSweep s;
   };
   std::mutex sweep_mu;   // runs on several threads may come first together
@@ -772,6 +773,14 @@ const srbcrs_plan::Merged& merged_stream(srbcrs_plan& plan, int W, hipStream_t s
   return plan.merged.emplace(W, m).first->second;
 }
 
+// Allocations of this thread while another stream is being captured: relaxed,
+// they neither fail nor invalidate that capture.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 constexpr int kSweepFlags = 256;
 constexpr int kSweepKeyCols = 1 << 24;   // an entry holds 24 bits of B row
 
@@ -794,7 +803,9 @@ bool sweep_wanted(const srbcrs_plan& plan) {
 // kernels, which give the same bits.  The first run of a width does that: a
 // plan run once (a sampled graph) does not pay for the stream, which takes
 // about as long as a few runs gain.  Not built under graph capture or for a
-// caller that may not allocate.
+// caller that may not allocate.  A build that fails, for want of memory say,
+// costs the run nothing but its time: the block kernels take it, and the next
+// attempts come after 1, 2, 4, ... 1024 runs more.
 const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_build, hipStream_t st) {
   const srbcrs::ColSweepTasks t = sweep_tasks(plan);
   const int64_t rows = (int64_t)t.n * 16;
@@ -824,7 +835,7 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
     // chain (about 0.4 us a block: 40 blocks 17.9 us, sweep 8 + 1.5).
     if (plan.n_apacked * N < (16 << 20) && w.longest < 24) return nullptr;
     if (w.built) return &w.s;
-    if (w.failed) continue;
+    if (w.unfit) continue;
     if (!may_build) return nullptr;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
@@ -833,6 +844,11 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
     }
     if (!again && w.seen.insert(N).second) return nullptr;
     again = true;
+    if (w.skip > 0) {
+      --w.skip;
+      return nullptr;
+    }
+    const RelaxedCapture relaxed;
     srbcrs::ColSweep s;
     if (layout < 0) {
       s.rows = -layout;
@@ -849,16 +865,25 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
     if (!plan.d_sweep_flags) {
       plan.d_sweep_flags = static_cast<unsigned long long*>(srbcrs::pool_alloc(kSweepFlags * 8));
       e = plan.d_sweep_flags ? hipMemsetAsync(plan.d_sweep_flags, 0, kSweepFlags * 8, st) : hipErrorOutOfMemory;
+      if (e == hipSuccess) e = hipStreamSynchronize(st);   // runs on other streams may use them next
+      if (e != hipSuccess) {
+        srbcrs::pool_drop(plan.d_sweep_flags);
+        plan.d_sweep_flags = nullptr;
+      }
     }
     srbcrs::ColSweepIn in{t, plan.d_awords, plan.d_sidx, plan.d_apacked, plan.n_apacked, plan.d_rowmap,
                           (int)plan.packed_rows, plan.total, plan.max_col};
     if (e == hipSuccess) e = srbcrs::build_colsweep(in, s, conv_alloc, conv_free, nullptr, st);
-    if (e == hipErrorOutOfMemory || e == hipErrorInvalidValue) {
-      (void)hipGetLastError();
-      w.failed = true;
+    if (e == hipErrorInvalidValue) {
+      w.unfit = true;
       continue;
     }
-    hip_check(e, "column sweep stream");
+    if (e != hipSuccess) {   // (an error that lasts is the launch's as well)
+      (void)hipGetLastError();
+      w.skip = w.backoff;
+      w.backoff = std::min(2 * w.backoff, 1024);
+      return nullptr;
+    }
     w.s = s;
     w.built = true;
     return &w.s;

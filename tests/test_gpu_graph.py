@@ -84,3 +84,49 @@ def test_graph_survives_partial_buffer_growth(gpu):
         torch.cuda.synchronize()
         assert torch.equal(C, ref)
     assert wide.shape == (M, 512)
+
+
+def test_run_that_builds_its_stream_during_another_capture(gpu):
+    """A default run on a stream that is not captured may allocate (its second
+    run at a width builds the column sweep's stream) while another stream is
+    captured: the capture stays valid, also where a conversion was refused in
+    it."""
+    import torch
+    from mask_amd._capi import SrbcrsError
+    from mask_amd.SRBCRSSpMM import Plan
+    rng = np.random.default_rng(3)
+    t = lambda a: torch.from_numpy(a).cuda()
+
+    def csr(M, per):
+        cols = np.sort(rng.integers(0, M, (M, per)), axis=1).astype(np.int32).ravel()
+        return t(np.arange(M + 1, dtype=np.int32) * per), t(cols), t(rng.uniform(-1, 1, cols.size).astype(np.float32))
+
+    small, large = csr(3000, 16), csr(60000, 16)
+    p, q = Plan(*small, 3000), Plan(*large, 60000)
+    B, C = torch.rand((3000, 64), device="cuda"), torch.empty((3000, 64), device="cuda")
+    B2, C2 = torch.rand((60000, 128), device="cuda"), torch.empty((60000, 128), device="cuda")
+    for _ in range(3):
+        p.run(B, C)
+    q.run(B2, C2)
+    ref, ref2 = C.clone(), C2.clone()
+    q.trim()                      # no kept memory: the stream's arrays come from hipMalloc
+    other, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    _say("stream build during a capture")
+    free = torch.cuda.mem_get_info()[0]
+    with torch.cuda.graph(g):
+        p.run(B, C)
+        with torch.cuda.stream(other):
+            q.run(B2, C2)
+        with pytest.raises(SrbcrsError, match="capture"):
+            Plan(*small, 3000)
+    other.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] >= 8 * 60000 * 16
+    assert torch.equal(C2, ref2)
+    for _ in range(3):
+        C.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C, ref)
+        q.run(B2, C2)
+        assert torch.equal(C2, ref2)

@@ -105,3 +105,26 @@ assert (fake.fake_calls(), fake.fake_mallocs()) == (calls, mallocs)
 fake.fake_capture(0)
 assert create(c, 320, 1)[0] == 0, error()
 """)
+
+
+def test_a_sweep_stream_that_could_not_be_built_is_tried_again(fake_hip):
+    """A shortage of memory sends the run to the block kernels and is not
+    remembered for good; one that lasts is not met on every run."""
+    _run(fake_hip, """
+M = K = 4096
+h = sparse_plan(M, K, 20)
+assert run(h, M, K, 64) == 0 and launches("spmm_colsweep") == 0
+fake.fake_fail_malloc(1, 2)     # the flags are allocated, the stream's arrays are not
+assert run(h, M, K, 64) == 0, error()
+assert launches("spmm_colsweep") == 0 and launches("spmm_stream") == 2
+for _ in range(3):
+    assert run(h, M, K, 64) == 0, error()
+assert launches("spmm_colsweep") >= 1
+h = sparse_plan(M, K, 20)
+assert run(h, M, K, 64) == 0
+before = fake.fake_mallocs()
+fake.fake_fail_malloc(0, 1 << 30)
+for _ in range(500):
+    assert run(h, M, K, 64) == 0, error()
+assert fake.fake_mallocs() - before < 500   # under one a run; an attempt makes 32
+""")
