@@ -215,8 +215,11 @@ int srbcrs_plan_set_schedule(srbcrs_plan *plan, const char *policy, int32_t para
  * stored values that gives the block kernels' bits (infinities and NaNs of B
  * included); it needs ldb, ldc multiples of 4, 16-byte aligned B and C and
  * K * ldb * 4 < 2^32, and runs from a width's second run on, which builds its
- * entry stream (it allocates 8 to 12 bytes per stored value, kept until the plan
- * is destroyed): capture after two eager runs to capture it.  Elsewhere, under
+ * entry stream: it allocates 8 bytes per stored value plus up to 7 entries of
+ * padding per list (16 bytes a value in all on rows of 4).  Widths share
+ * streams where their layout is the same, and always once a schedule's streams
+ * together hold as many bytes as the plan's block values.  Capture after two
+ * eager runs to capture the sweep.  Elsewhere, under
  * capture before that, and on small products, the block kernels run.  A call
  * that is refused (a negative status) has launched nothing and left C
  * untouched. */
@@ -228,7 +231,9 @@ int srbcrs_run(srbcrs_plan *plan, const float *d_B, int64_t K, int64_t N, int64_
  * Retired buffers are what graphs captured on earlier runs may still
  * address: call this only when no such graph will be replayed again and no
  * launch that used them is in flight on another stream.  Without it they
- * are freed with the plan.  Also gives back to the driver the device memory
+ * are freed with the plan.  So are, by this call, the column sweep's entry
+ * streams of schedules that the plan no longer has, unless a run recorded into
+ * a graph used them (those stay until the plan is destroyed).  Also gives back to the driver the device memory
  * that destroyed plans and conversions have left (kept, up to 4 GiB a
  * process, for the next ones).  No reference counterpart (the reference
  * keeps one global cache entry). */

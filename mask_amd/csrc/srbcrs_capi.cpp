@@ -465,18 +465,26 @@ struct srbcrs_plan {
   };
   std::map<int64_t, Nz> nz;
   // The column sweep's entry streams, per schedule (policy, parameter) and
-  // rows per list, built by the second run of a width and kept until the
-  // plan is destroyed (a HIP graph may hold their addresses).
+  // layout, built by the second run of a width.  Those of one schedule are
+  // bounded together (sweep_stream); those of the schedules before count as
+  // retired, but for the ones whose addresses a captured launch holds.
   struct Sweep {
     std::set<int64_t> seen;   // widths that have run
     int32_t longest = 0;   // blocks of the schedule's longest task
     bool unfit = false;   // the matrix does not fit this layout
     bool built = false;
+    bool captured = false;   // by a launch recorded into a graph
     int skip = 0, backoff = 1;   // runs before the next attempt after a build that failed, and after the next failure
     srbcrs::ColSweep s;
   };
   std::mutex sweep_mu;   // runs on several threads may come first together
   std::map<std::tuple<std::string, int32_t, int>, Sweep> sweeps;
+  template <class F>
+  static void free_sweep(srbcrs::ColSweep& s, F&& drop) {
+    drop(s.entries);
+    for (int** p : {&s.start, &s.nblk, &s.dest, &s.wblk8, &s.wblk4, &s.lstart, &s.lnblk, &s.ldest, &s.uoff, &s.pend})
+      drop(*p);
+  }
   // non-finite marks of the runs in flight: run i (from 1) raises slot i %
   // kSweepFlags to i, its repair pass looks whether the slot has reached i
   unsigned long long* d_sweep_flags = nullptr;
@@ -525,13 +533,7 @@ struct srbcrs_plan {
     dev_free(d_awords);
     dev_free(d_apacked);
     dev_free(d_sweep_flags);
-    for (auto& kv : sweeps) {
-      srbcrs::ColSweep& w = kv.second.s;
-      dev_free(w.entries);
-      for (int** p : {&w.start, &w.nblk, &w.dest, &w.wblk8, &w.wblk4, &w.lstart, &w.lnblk, &w.ldest, &w.uoff,
-                      &w.pend})
-        dev_free(*p);
-    }
+    for (auto& kv : sweeps) free_sweep(kv.second.s, dev_free);
     for (auto& kv : merged) {
       dev_free(kv.second.d_moff);
       dev_free(kv.second.d_sidx);
@@ -806,7 +808,17 @@ bool sweep_wanted(const srbcrs_plan& plan) {
 // caller that may not allocate.  A build that fails, for want of memory say,
 // costs the run nothing but its time: the block kernels take it, and the next
 // attempts come after 1, 2, 4, ... 1024 runs more.
+//
+// The best layout depends on the width, but any one gives the same bits: once
+// a schedule's streams hold as much as the plan's dense block values, a width
+// whose own would exceed that takes the nearest one there is.  (A stream is 8
+// bytes a stored value and its lists' padding, at under 15 values a block of
+// 512 bytes: the bound leaves room for three at least.)
 const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_build, hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  const bool known = hipStreamIsCapturing(st, &cs) == hipSuccess;
+  if (!known) (void)hipGetLastError();
+  const bool capturing = !known || cs != hipStreamCaptureStatusNone;
   const srbcrs::ColSweepTasks t = sweep_tasks(plan);
   const int64_t rows = (int64_t)t.n * 16;
   // Short rows whose B rows hardly any other row reads: nothing to share, and
@@ -823,6 +835,10 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
   const int layouts[2] = {-srbcrs::phasesweep_rows(rows, (int)N, (int64_t)plan.max_col + 1),
                           srbcrs::colsweep_rows_per_list(rows, (int)N)};
   std::lock_guard<std::mutex> lock(plan.sweep_mu);
+  auto take = [&](srbcrs_plan::Sweep& w) {
+    w.captured = w.captured || capturing;
+    return &w.s;
+  };
   bool again = false;   // not the first run of this width
   for (int layout : layouts) {
     if (!layout) continue;
@@ -834,14 +850,24 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
     // less than their launches, unless long windows make the block kernel a
     // chain (about 0.4 us a block: 40 blocks 17.9 us, sweep 8 + 1.5).
     if (plan.n_apacked * N < (16 << 20) && w.longest < 24) return nullptr;
-    if (w.built) return &w.s;
+    if (w.built) return take(w);
     if (w.unfit) continue;
-    if (!may_build) return nullptr;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-      (void)hipGetLastError();
-      return nullptr;
+    srbcrs_plan::Sweep* near = nullptr;   // built, of this schedule
+    int near_layout = 0;
+    size_t held = 0;
+    for (auto& kv : plan.sweeps) {
+      if (std::get<0>(kv.first) != plan.sched.policy || std::get<1>(kv.first) != plan.sched.param || !kv.second.built)
+        continue;
+      held += kv.second.s.bytes;
+      const int l = std::get<2>(kv.first);   // phases before lists, the larger before the smaller: as the key sorts
+      const bool same_kind = (l < 0) == (layout < 0), near_same = near && (near_layout < 0) == (layout < 0);
+      if (!near || (same_kind && (!near_same || std::abs(l - layout) < std::abs(near_layout - layout)))) {
+        near = &kv.second;
+        near_layout = l;
+      }
     }
+    if (near && held + 10 * (size_t)plan.n_apacked > (size_t)plan.total * 512) return take(*near);
+    if (!may_build || capturing) return nullptr;
     if (!again && w.seen.insert(N).second) return nullptr;
     again = true;
     if (w.skip > 0) {
@@ -886,7 +912,7 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
     }
     w.s = s;
     w.built = true;
-    return &w.s;
+    return take(w);
   }
   return nullptr;
 }
@@ -1711,6 +1737,19 @@ int srbcrs_plan_trim(srbcrs_plan* plan, void* stream) {
     hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream)), "hipStreamSynchronize");
     for (void* p : plan->retired) srbcrs::pool_drop(p);
     plan->retired.clear();
+    std::lock_guard<std::mutex> lock(plan->sweep_mu);
+    for (auto& kv : plan->sweeps) {
+      srbcrs_plan::Sweep& w = kv.second;
+      if (!w.built || w.captured || (std::get<0>(kv.first) == plan->sched.policy &&
+                                     std::get<1>(kv.first) == plan->sched.param))
+        continue;
+      srbcrs_plan::free_sweep(w.s, [](auto*& p) {
+        srbcrs::pool_drop(p);
+        p = nullptr;
+      });
+      w.s = srbcrs::ColSweep{};
+      w.built = false;
+    }
     srbcrs::pool_release(plan->device);
   });
 }

@@ -211,9 +211,11 @@ static hipError_t build_phasesweep(const ColSweepIn& in, ColSweep& out, DeviceAl
       err = hipErrorOutOfMemory;
     return p;
   };
+  out.bytes = 0;
   auto keep = [&](size_t n) {
     void* p = err == hipSuccess ? alloc(ctx, n) : nullptr;
     if (!p) err = hipErrorOutOfMemory;
+    out.bytes += n;
     return p;
   };
   auto cleanup = [&](hipError_t e) {
@@ -294,7 +296,7 @@ static hipError_t build_phasesweep(const ColSweepIn& in, ColSweep& out, DeviceAl
   out.n_entries = (int64_t)h[0];
   if (h[0] > (unsigned long long)INT32_MAX - 64 || out.n_long > long_cap || h[2] > h[3] + h[3] / 2 + 65536)
     return cleanup(hipErrorInvalidValue);
-  out.entries = (uint2*)alloc(ctx, ((size_t)h[0] + 8) * 8);
+  out.entries = (uint2*)keep(((size_t)h[0] + 8) * 8);
   if (!out.entries) return cleanup(hipErrorOutOfMemory);
   const PhaseFill f{cnt, place, load, out.uoff, out.pend, out.rows, out.phases};
   hipLaunchKernelGGL(k_phase_fill, dim3((unsigned)(slots / 8)), dim3(64), 0, st, t, in.words, in.sidx, in.packed, vrow,
@@ -328,11 +330,8 @@ hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc
   constexpr int64_t kLongMin = 128;
   const int64_t long_len = std::max<int64_t>(kLongMin, in.n_values / n_lists);
   const int long_bin = sweep_bin((int)long_len);
-  // stored values, and room for explicit zeros (k_sweep_len counts them)
-  const int64_t most = in.n_values + in.n_values / 16 + 4096;
-  const int64_t long_cap = most / kLongMin + 1;
-  const int64_t cap = most + kSweepBatch * n_lists + kSweepLongBatch * long_cap;
-  if (cap > INT32_MAX) return hipErrorInvalidValue;
+  // rows past kLongMin values; explicit zeros count (k_sweep_len)
+  const int64_t long_cap = (in.n_values + in.n_values / 16 + 4096) / kLongMin + 1;
   int *len = nullptr, *hist = nullptr, *vrow = nullptr, *list_len = nullptr, *lvrow = nullptr;
   unsigned long long* total = nullptr;
   bool idle = true;
@@ -350,35 +349,37 @@ hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc
     drop(total);
     if (e != hipSuccess) {
       drop(out.entries);
-      drop(out.start);
-      drop(out.nblk);
-      drop(out.wblk8);
-      drop(out.wblk4);
-      drop(out.dest);
-      drop(out.lstart);
-      drop(out.lnblk);
-      drop(out.ldest);
+      for (int** p : {&out.start, &out.nblk, &out.wblk8, &out.wblk4, &out.dest, &out.lstart, &out.lnblk, &out.ldest})
+        drop(*p);
     }
     return e;
   };
-  len = (int*)alloc(ctx, (size_t)rows * 4);
-  hist = (int*)alloc(ctx, 2 * kSweepBins * 4);
-  vrow = (int*)alloc(ctx, (size_t)slots * 4);
-  list_len = (int*)alloc(ctx, (size_t)n_lists * 4);
-  lvrow = (int*)alloc(ctx, (size_t)long_cap * 4);
-  total = (unsigned long long*)alloc(ctx, 16);   // entries taken, long rows
-  out.entries = (uint2*)alloc(ctx, (size_t)(cap + 8) * 8);
-  out.start = (int*)alloc(ctx, (size_t)n_lists * 4);
-  out.nblk = (int*)alloc(ctx, (size_t)n_lists * 4);
-  out.wblk8 = (int*)alloc(ctx, (size_t)n_lists / 8 * 4);
-  out.wblk4 = (int*)alloc(ctx, (size_t)n_lists / 4 * 4);
-  out.dest = (int*)alloc(ctx, (size_t)slots * 4);
-  out.lstart = (int*)alloc(ctx, (size_t)long_cap * 4);
-  out.lnblk = (int*)alloc(ctx, (size_t)long_cap * 4);
-  out.ldest = (int*)alloc(ctx, (size_t)long_cap * 4);
-  if (!len || !hist || !vrow || !list_len || !total || !out.entries || !out.start || !out.nblk || !out.wblk8 ||
-      !out.wblk4 || !out.dest || !lvrow || !out.lstart || !out.lnblk || !out.ldest)
-    return cleanup(hipErrorOutOfMemory);
+  bool room = true;
+  auto temp = [&](size_t bytes) {
+    void* p = room ? alloc(ctx, bytes) : nullptr;
+    room = p != nullptr;
+    return p;
+  };
+  out.bytes = 0;
+  auto keep = [&](size_t bytes) {
+    out.bytes += bytes;
+    return temp(bytes);
+  };
+  len = (int*)temp((size_t)rows * 4);
+  hist = (int*)temp(2 * kSweepBins * 4);
+  vrow = (int*)temp((size_t)slots * 4);
+  list_len = (int*)temp((size_t)n_lists * 4);
+  lvrow = (int*)temp((size_t)long_cap * 4);
+  total = (unsigned long long*)temp(16);   // entries taken, long rows
+  out.start = (int*)keep((size_t)n_lists * 4);
+  out.nblk = (int*)keep((size_t)n_lists * 4);
+  out.wblk8 = (int*)keep((size_t)n_lists / 8 * 4);
+  out.wblk4 = (int*)keep((size_t)n_lists / 4 * 4);
+  out.dest = (int*)keep((size_t)slots * 4);
+  out.lstart = (int*)keep((size_t)long_cap * 4);
+  out.lnblk = (int*)keep((size_t)long_cap * 4);
+  out.ldest = (int*)keep((size_t)long_cap * 4);
+  if (!room) return cleanup(hipErrorOutOfMemory);
 #define SRBCRS_STEP(x)                          \
   do {                                          \
     const hipError_t e_ = (x);                  \
@@ -399,24 +400,28 @@ hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc
                      RL, long_bin, in.rowmap, in.M, vrow, out.dest, list_len, lvrow, out.ldest, (int)long_cap, n_long);
   SRBCRS_STEP(hipGetLastError());
   const int n8 = (int)(n_lists / 8);
-  hipLaunchKernelGGL(k_sweep_place, dim3((unsigned)((n8 + 63) / 64)), dim3(64), 0, st, list_len, n8, cap, out.start,
-                     out.nblk, out.wblk8, out.wblk4, total);
+  hipLaunchKernelGGL(k_sweep_place, dim3((unsigned)((n8 + 63) / 64)), dim3(64), 0, st, list_len, n8,
+                     (int64_t)INT32_MAX, out.start, out.nblk, out.wblk8, out.wblk4, total);
   SRBCRS_STEP(hipGetLastError());
   hipLaunchKernelGGL(k_sweep_place_long, dim3((unsigned)((long_cap + 63) / 64)), dim3(64), 0, st, len, lvrow, n_long,
-                     (int)long_cap, cap, out.lstart, out.lnblk, total);
-  SRBCRS_STEP(hipGetLastError());
-  hipLaunchKernelGGL(k_sweep_fill, dim3((unsigned)((slots + 7) / 8 + (long_cap + 7) / 8)), dim3(64),
-                     32 * out.phases * 4, st, t, in.words, in.sidx, in.packed, vrow, slots, RL, list_len, out.start,
-                     out.nblk, out.phases, out.shift, lvrow, len, out.lstart, out.lnblk, n_long, (int)long_cap,
-                     out.entries);
+                     (int)long_cap, (int64_t)INT32_MAX, out.lstart, out.lnblk, total);
   SRBCRS_STEP(hipGetLastError());
   unsigned long long h_total[2] = {0, 0};
   SRBCRS_STEP(hipMemcpyAsync(h_total, total, 16, hipMemcpyDeviceToHost, st));
   SRBCRS_STEP(hipStreamSynchronize(st));
-#undef SRBCRS_STEP
-  out.n_entries = (int64_t)h_total[0];
   out.n_long = (int)(h_total[1] & 0xffffffffu);
-  return cleanup(out.n_entries <= cap && out.n_long <= long_cap ? hipSuccess : hipErrorInvalidValue);
+  out.n_entries = (int64_t)h_total[0];
+  if (h_total[0] > (unsigned long long)INT32_MAX - 64 || out.n_long > long_cap) return cleanup(hipErrorInvalidValue);
+  out.entries = (uint2*)keep((size_t)(out.n_entries + 8) * 8);
+  if (!out.entries) return cleanup(hipErrorOutOfMemory);
+  hipLaunchKernelGGL(k_sweep_fill, dim3((unsigned)((slots + 7) / 8 + (out.n_long + 7) / 8)), dim3(64),
+                     32 * out.phases * 4, st, t, in.words, in.sidx, in.packed, vrow, slots, RL, list_len, out.start,
+                     out.nblk, out.phases, out.shift, lvrow, len, out.lstart, out.lnblk, n_long, (int)long_cap,
+                     out.entries);
+  SRBCRS_STEP(hipGetLastError());
+  SRBCRS_STEP(hipStreamSynchronize(st));
+#undef SRBCRS_STEP
+  return cleanup(hipSuccess);
 }
 
 }  // namespace srbcrs

@@ -119,6 +119,7 @@ struct ColSweep {
   int RL = 8, phases = 1, shift = 24;
   int n_lists = 0;        // a multiple of 8
   int64_t n_entries = 0;
+  size_t bytes = 0;       // of all arrays below
   uint2* entries = nullptr;
   int *start = nullptr, *nblk = nullptr, *dest = nullptr;
   int *wblk8 = nullptr, *wblk4 = nullptr;   // batches per 8 and per 4 lists

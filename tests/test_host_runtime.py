@@ -128,3 +128,53 @@ for _ in range(500):
     assert run(h, M, K, 64) == 0, error()
 assert fake.fake_mallocs() - before < 500   # under one a run; an attempt makes 32
 """)
+
+
+def test_sweep_streams_are_bounded_and_trimmed(fake_hip):
+    """However many widths run, the streams of one schedule hold at most the
+    size of the block values; trim frees those of other schedules that no
+    captured run holds."""
+    _run(fake_hip, """
+M = K = 65536
+big = dict(B=np.zeros(512 * K + 8, np.float32), C=np.zeros(512 * M + 8, np.float32))
+h = sparse_plan(M, K, 16)
+d = _capi.PlanDesc()
+L.srbcrs_plan_get(h, ctypes.byref(d))
+entries = M * 16 * 5 // 4
+d2h(np.array([entries, 0], np.uint64))                              # a list stream
+d2h(np.array([entries, 0, M * 16, M * 16], np.uint64))              # a phase stream
+trim = lambda: L.srbcrs_plan_trim(h, None)
+live = lambda: (trim(), fake.fake_live_bytes())[1]
+base = live()
+for N in range(16, 513, 16):
+    for i in range(3):
+        assert run(h, M, K, N, **big) == 0, error()
+    assert launches("spmm_stream") <= 2 * N // 16
+    assert launches("spmm_colsweep") + launches("spmm_phasesweep") >= N // 16   # at least the last of the three
+    assert live() - base <= d.total_blocks * 512 + 8 * entries
+row = live()
+assert row - base > 3 * 8 * entries
+def schedule(p, q):
+    assert L.srbcrs_plan_set_schedule(h, p, q) == 0, error()
+one = 8 * entries   # and its padding and places
+def split(p):
+    schedule(b"split", p)
+    assert run(h, M, K, 512, **big) == 0, error()   # the block kernels; the partial tiles are allocated
+    base = live()
+    assert run(h, M, K, 512, **big) == 0, error()
+    assert one < live() - base < 2 * one
+    return base
+no_streams = split(7)
+fake.fake_capture(1)
+assert run(h, M, K, 512, **big) == 0, error()
+fake.fake_capture(0)
+assert one // 2 < split(9) - no_streams < 2 * one   # the stream that the capture holds
+schedule(b"row", 0)
+assert one // 2 < live() - no_streams < 2 * one     # the other is gone
+for N in (64, 512):   # built again, by the second run at the latest
+    assert run(h, M, K, N, **big) == 0, error()
+    n = launches("spmm_colsweep") + launches("spmm_phasesweep")
+    assert run(h, M, K, N, **big) == 0, error()
+    assert launches("spmm_colsweep") + launches("spmm_phasesweep") == n + 1
+L.srbcrs_plan_destroy(h)
+""")
