@@ -485,10 +485,11 @@ struct srbcrs_plan {
     for (int** p : {&s.start, &s.nblk, &s.dest, &s.wblk8, &s.wblk4, &s.lstart, &s.lnblk, &s.ldest, &s.uoff, &s.pend})
       drop(*p);
   }
-  // non-finite marks of the runs in flight: run i (from 1) raises slot i %
-  // kSweepFlags to i, its repair pass looks whether the slot has reached i
-  unsigned long long* d_sweep_flags = nullptr;
-  std::atomic<unsigned long long> sweep_runs{0};
+  // non-finite marks (mark_raise): kSweepMarks for the numbered runs in turn,
+  // then four words for each of up to kCapturedMarks runs recorded into graphs
+  // (any past those are numbered, and repair on every replay once marked)
+  unsigned long long* d_sweep_marks = nullptr;
+  std::atomic<unsigned long long> sweep_runs{0}, sweep_captures{0};
 
   template <class T>
   void retire(T*& p) {
@@ -532,7 +533,7 @@ struct srbcrs_plan {
     dev_free(d_bp);
     dev_free(d_awords);
     dev_free(d_apacked);
-    dev_free(d_sweep_flags);
+    dev_free(d_sweep_marks);
     for (auto& kv : sweeps) free_sweep(kv.second.s, dev_free);
     for (auto& kv : merged) {
       dev_free(kv.second.d_moff);
@@ -783,7 +784,8 @@ struct RelaxedCapture {
   ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
-constexpr int kSweepFlags = 256;
+constexpr int kSweepMarks = 256, kCapturedMarks = 1024;
+constexpr size_t kMarkBytes = (kSweepMarks + 4 * kCapturedMarks) * 8;
 constexpr int kSweepKeyCols = 1 << 24;   // an entry holds 24 bits of B row
 
 srbcrs::ColSweepTasks sweep_tasks(const srbcrs_plan& plan) {
@@ -814,11 +816,12 @@ bool sweep_wanted(const srbcrs_plan& plan) {
 // whose own would exceed that takes the nearest one there is.  (A stream is 8
 // bytes a stored value and its lists' padding, at under 15 values a block of
 // 512 bytes: the bound leaves room for three at least.)
-const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_build, hipStream_t st) {
+const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_build, hipStream_t st,
+                                     bool& capturing) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   const bool known = hipStreamIsCapturing(st, &cs) == hipSuccess;
   if (!known) (void)hipGetLastError();
-  const bool capturing = !known || cs != hipStreamCaptureStatusNone;
+  capturing = !known || cs != hipStreamCaptureStatusNone;
   const srbcrs::ColSweepTasks t = sweep_tasks(plan);
   const int64_t rows = (int64_t)t.n * 16;
   // Short rows whose B rows hardly any other row reads: nothing to share, and
@@ -888,13 +891,13 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
       s.phases = (plan.max_col >> s.shift) + 1;
     }
     hipError_t e = hipSuccess;
-    if (!plan.d_sweep_flags) {
-      plan.d_sweep_flags = static_cast<unsigned long long*>(srbcrs::pool_alloc(kSweepFlags * 8));
-      e = plan.d_sweep_flags ? hipMemsetAsync(plan.d_sweep_flags, 0, kSweepFlags * 8, st) : hipErrorOutOfMemory;
+    if (!plan.d_sweep_marks) {
+      plan.d_sweep_marks = static_cast<unsigned long long*>(srbcrs::pool_alloc(kMarkBytes));
+      e = plan.d_sweep_marks ? hipMemsetAsync(plan.d_sweep_marks, 0, kMarkBytes, st) : hipErrorOutOfMemory;
       if (e == hipSuccess) e = hipStreamSynchronize(st);   // runs on other streams may use them next
       if (e != hipSuccess) {
-        srbcrs::pool_drop(plan.d_sweep_flags);
-        plan.d_sweep_flags = nullptr;
+        srbcrs::pool_drop(plan.d_sweep_marks);
+        plan.d_sweep_marks = nullptr;
       }
     }
     srbcrs::ColSweepIn in{t, plan.d_awords, plan.d_sidx, plan.d_apacked, plan.n_apacked, plan.d_rowmap,
@@ -1610,17 +1613,24 @@ static void run_impl(srbcrs_plan* plan, const float* d_B, int64_t K, int64_t N, 
     // No knobs at low block fill: the column sweep, where its 32-bit offsets
     // and 16-byte accesses reach (the block kernels' bits either way).
     const srbcrs::ColSweep* sweep = nullptr;
+    bool capturing = false;
     if ((!opts || all_default(*opts)) && sweep_wanted(*plan) && ldb % 4 == 0 && ldc % 4 == 0 &&
         (reinterpret_cast<uintptr_t>(d_B) | reinterpret_cast<uintptr_t>(d_C)) % 16 == 0 &&
         (uint64_t)K * (uint64_t)ldb * 4u < (1ull << 32) && (uint64_t)ldb * 4u < (1ull << 24))
-      sweep = sweep_stream(*plan, N, !fixed_partial, st);
+      sweep = sweep_stream(*plan, N, !fixed_partial, st, capturing);
     auto launch_sweep = [&](float* partial) {
-      const unsigned long long run = ++plan->sweep_runs;
-      unsigned long long* flag = plan->d_sweep_flags + run % kSweepFlags;
+      unsigned long long token = 0, *mark = nullptr;
+      const unsigned long long own = capturing ? plan->sweep_captures++ : kCapturedMarks;
+      if (own < kCapturedMarks) {
+        mark = plan->d_sweep_marks + kSweepMarks + 4 * own;
+      } else {
+        token = ++plan->sweep_runs;
+        mark = plan->d_sweep_marks + token % kSweepMarks;
+      }
       srbcrs::StreamArgs sa = a;
       sa.partial = partial;
-      hip_check(srbcrs::launch_colsweep(*sweep, sa, K, run, flag, st), "launch spmm_colsweep");
-      hip_check(srbcrs::launch_colsweep_repair(sweep_tasks(*plan), sa, run, flag, st), "launch sweep repair");
+      hip_check(srbcrs::launch_colsweep(*sweep, sa, K, token, mark, st), "launch spmm_colsweep");
+      hip_check(srbcrs::launch_colsweep_repair(sweep_tasks(*plan), sa, token, mark, st), "launch sweep repair");
     };
     if (plan->sched.policy == "row") {
       if (plan->n_zero_rows)

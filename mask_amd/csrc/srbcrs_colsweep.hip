@@ -22,7 +22,7 @@ static int64_t sweep_grid(int64_t n_wg, int n_chunks, int swept) {
 
 template <int C, int RL, int WV>
 static hipError_t launch_t(const ColSweep& s, const StreamArgs& a, int64_t K, int swept, unsigned long long token,
-                           unsigned long long* flag, hipStream_t st) {
+                           unsigned long long* mark, hipStream_t st) {
   const int n_chunks = (a.N + C - 1) / C;
   const int n_waves = s.n_lists / (256 / C);
   const int64_t n_wg = (n_waves + WV - 1) / WV;
@@ -36,7 +36,7 @@ static hipError_t launch_t(const ColSweep& s, const StreamArgs& a, int64_t K, in
   const SweepStream ss{s.entries, s.start, s.nblk, C == 32 ? s.wblk8 : s.wblk4, s.dest, n_waves,
                        s.lstart, s.lnblk, s.ldest, s.n_long};
   hipLaunchKernelGGL((spmm_colsweep<C, RL, WV>), dim3((unsigned)grid), dim3(64 * WV), 0, st, ss, a.B, (uint32_t)bytes,
-                     a.C, a.partial, a.N, (uint32_t)(a.ldb * 4), a.ldc, n_chunks, swept, a.relu, token, flag,
+                     a.C, a.partial, a.N, (uint32_t)(a.ldb * 4), a.ldc, n_chunks, swept, a.relu, token, mark,
                      (int)long_wgs);
   return hipGetLastError();
 }
@@ -106,7 +106,7 @@ int phasesweep_rows(int64_t rows, int N, int64_t K) {
 
 template <int C, int WV>
 static hipError_t launch_phase_t(const ColSweep& s, const StreamArgs& a, int64_t K, int swept,
-                                 unsigned long long token, unsigned long long* flag, hipStream_t st) {
+                                 unsigned long long token, unsigned long long* mark, hipStream_t st) {
   const int n_chunks = (a.N + C - 1) / C;
   const int64_t n_wg = s.n_lists / (C == 32 ? WV / 8 : 1);
   const int64_t n_ids = sweep_grid(n_wg, n_chunks, swept);
@@ -118,7 +118,7 @@ static hipError_t launch_phase_t(const ColSweep& s, const StreamArgs& a, int64_t
                        {s.entries, nullptr, nullptr, nullptr, nullptr, 0, s.lstart, s.lnblk, s.ldest, s.n_long}};
   if (total == 0) return hipSuccess;
   hipLaunchKernelGGL((spmm_phasesweep<C, WV>), dim3((unsigned)total), dim3(64 * WV), 0, st, ps, a.B, (uint32_t)bytes,
-                     a.C, a.partial, a.N, (uint32_t)(a.ldb * 4), a.ldc, n_chunks, swept, a.relu, token, flag,
+                     a.C, a.partial, a.N, (uint32_t)(a.ldb * 4), a.ldc, n_chunks, swept, a.relu, token, mark,
                      (int)n_ids);
   return hipGetLastError();
 }
@@ -142,22 +142,22 @@ static hipError_t launch_phase_t(const ColSweep& s, const StreamArgs& a, int64_t
 //                          the stream, which every chunk reads again (2^20
 //                          nodes, N = 512, 134 + 340 MB: 8680, swept 9760)
 static hipError_t launch_phasesweep(const ColSweep& s, const StreamArgs& a, int64_t K, unsigned long long token,
-                                    unsigned long long* flag, hipStream_t st) {
+                                    unsigned long long* mark, hipStream_t st) {
   const int64_t rows = (int64_t)s.n_lists * s.rows;
   const bool cached = K * 128 + s.n_entries * 8 <= kMemCacheBytes;
   const bool hubs = s.n_long > 0 && s.n_entries >= 20 * rows;
   if (a.N % 32 || a.ldb % 32 || (rows < kSweptRows && !(cached && hubs)))
-    return launch_phase_t<64, 16>(s, a, K, 0, token, flag, st);
-  if (cached && hubs) return launch_phase_t<32, 8>(s, a, K, 1, token, flag, st);
-  return launch_phase_t<32, 16>(s, a, K, cached, token, flag, st);
+    return launch_phase_t<64, 16>(s, a, K, 0, token, mark, st);
+  if (cached && hubs) return launch_phase_t<32, 8>(s, a, K, 1, token, mark, st);
+  return launch_phase_t<32, 16>(s, a, K, cached, token, mark, st);
 }
 
 hipError_t launch_colsweep(const ColSweep& s, const StreamArgs& a, int64_t K, unsigned long long token,
-                           unsigned long long* flag, hipStream_t st) {
-  if (s.rows) return launch_phasesweep(s, a, K, token, flag, st);
+                           unsigned long long* mark, hipStream_t st) {
+  if (s.rows) return launch_phasesweep(s, a, K, token, mark, st);
   int cols, wv, swept;
   pick_launch((int64_t)s.n_lists * s.RL, s.RL, a, K, cols, wv, swept);
-#define SRBCRS_SWEEP(C, RL, WV) return launch_t<C, RL, WV>(s, a, K, swept, token, flag, st)
+#define SRBCRS_SWEEP(C, RL, WV) return launch_t<C, RL, WV>(s, a, K, swept, token, mark, st)
 #define SRBCRS_SWEEP_RL(C)                  \
   switch (s.RL) {                           \
     case 8:                                 \
@@ -176,11 +176,11 @@ hipError_t launch_colsweep(const ColSweep& s, const StreamArgs& a, int64_t K, un
 static SweepTasks sweep_tasks(const ColSweepTasks& t) { return SweepTasks{t.begin, t.end, t.window, t.slot, t.n}; }
 
 hipError_t launch_colsweep_repair(const ColSweepTasks& t, const StreamArgs& a, unsigned long long token,
-                                  const unsigned long long* flag, hipStream_t st) {
+                                  unsigned long long* mark, hipStream_t st) {
   const int64_t work = (int64_t)t.n * ((a.N + 63) / 64);
   if (work == 0) return hipSuccess;
   const unsigned grid = work < 4096 ? (unsigned)work : 4096u;
-  hipLaunchKernelGGL(k_sweep_repair, dim3(grid), dim3(64), 0, st, flag, token, sweep_tasks(t), a.a_words, a.sidx,
+  hipLaunchKernelGGL(k_sweep_repair, dim3(grid), dim3(64), 0, st, mark, token, sweep_tasks(t), a.a_words, a.sidx,
                      a.a_packed, a.B, a.C, a.partial, a.rowmap, a.M, a.N, a.ldb, a.ldc, a.relu);
   return hipGetLastError();
 }

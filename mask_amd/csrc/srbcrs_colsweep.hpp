@@ -11,7 +11,7 @@
 // k-steps), gives the same bits.  What differs is B's infinities and NaNs:
 // the block kernels multiply them by A's zeros and so poison every row of a
 // window whose blocks hold the column.  Each wave therefore checks the sums
-// it stores, and a non-finite one raises a flag on which k_sweep_repair
+// it stores, and a non-finite one raises a mark on which k_sweep_repair
 // (below) recomputes the product with A's zeros in it.
 //
 // Why this order.  Every gathered segment comes through the L2, and what
@@ -78,12 +78,31 @@ __device__ __forceinline__ bool non_finite(float x) {
   return (__builtin_bit_cast(uint32_t, x) & 0x7f800000u) == 0x7f800000u;
 }
 
+// The mark of a run's non-finite sums.  A run launched eagerly has a number
+// (token) and shares the mark with the runs 256 before and after it: raised to
+// its number or beyond, the run is repaired, so a later run's at most costs a
+// pass more.  A run recorded into a graph (token 0) has a mark of its own,
+// {raised, replays, this replay}, and numbers its replays on the device: the
+// sweep writes this replay's number for the repair pass and the repair pass
+// counts it, each reading only what the other one wrote.
+__device__ __forceinline__ void mark_begin(unsigned long long token, unsigned long long* __restrict__ mark) {
+  if (token == 0 && blockIdx.x == 0 && threadIdx.x == 0) mark[2] = mark[1] + 1;
+}
+__device__ __forceinline__ void mark_raise(unsigned long long token, unsigned long long* __restrict__ mark) {
+  atomicMax(mark, token ? token : mark[1] + 1);
+}
+__device__ __forceinline__ bool mark_raised(unsigned long long token, unsigned long long* __restrict__ mark) {
+  const unsigned long long run = token ? token : mark[2];
+  if (token == 0 && blockIdx.x == 0 && threadIdx.x == 0) mark[1] = run;
+  return mark[0] >= run;
+}
+
 // One long row, 64 columns (one per lane).
 __device__ __forceinline__ void sweep_long_row(const SweepStream& s, int r, int chunk, const float* __restrict__ B,
                                                uint32_t b_bytes, float* __restrict__ Cout,
                                                float* __restrict__ partial, int N, uint32_t ldb4, int64_t ldc,
                                                int relu, unsigned long long token,
-                                               unsigned long long* __restrict__ flag, int lane) {
+                                               unsigned long long* __restrict__ mark, int lane) {
   constexpr int U = kSweepLongBatch;
   const int nb = uniform_load(s.lnblk, r);
   const int col = chunk * 64 + lane;
@@ -131,7 +150,7 @@ __device__ __forceinline__ void sweep_long_row(const SweepStream& s, int r, int 
     if (relu && d >= 0) acc = relu1(acc);
     __builtin_nontemporal_store(acc, sweep_out(d, col, ldc, Cout, partial));
   }
-  if (__any(bad) && lane == 0) atomicMax(flag, token);
+  if (__any(bad) && lane == 0) mark_raise(token, mark);
 }
 
 // One workgroup = WV waves of LG lists on one chunk of C columns.
@@ -139,7 +158,8 @@ template <int C, int RL, int WV>
 __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(WV == 1 ? 5 : 4))) void spmm_colsweep(
     SweepStream s, const float* __restrict__ B, uint32_t b_bytes, float* __restrict__ Cout,
     float* __restrict__ partial, int N, uint32_t ldb4, int64_t ldc, int n_chunks, int swept, int relu,
-    unsigned long long token, unsigned long long* __restrict__ flag, int long_wgs) {
+    unsigned long long token, unsigned long long* __restrict__ mark, int long_wgs) {
+  mark_begin(token, mark);
   constexpr int LPG = C / 4, LG = 64 / LPG;
   __shared__ __attribute__((aligned(16))) float tile[WV * LG * RL * C];
   const int n_wg = (s.n_waves + WV - 1) / WV;
@@ -149,7 +169,7 @@ __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(WV == 1
   if (bid < long_wgs) {   // whole workgroups: the barriers below are not theirs
     const int i = bid * WV + wave;
     if (i < s.n_long * ((N + 63) / 64))
-      sweep_long_row(s, i % s.n_long, i / s.n_long, B, b_bytes, Cout, partial, N, ldb4, ldc, relu, token, flag, lane);
+      sweep_long_row(s, i % s.n_long, i / s.n_long, B, b_bytes, Cout, partial, N, ldb4, ldc, relu, token, mark, lane);
     return;
   }
   int wg, c;   // long_wgs is a multiple of the XCD count: XCD = id % 8 still
@@ -255,7 +275,7 @@ __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(WV == 1
       __builtin_nontemporal_store(v, reinterpret_cast<f4*>(sweep_out(d, col, ldc, Cout, partial)));
     }
   }
-  if (__any(bad) && lane == 0) atomicMax(flag, token);
+  if (__any(bad) && lane == 0) mark_raise(token, mark);
 }
 
 // The tasks of the schedule whose partial sums the stream reproduces.
@@ -268,11 +288,11 @@ struct SweepTasks {
 };
 
 // The product again with A's zeros in it, where the column sweep stored a
-// non-finite value (flag >= token): every block position's multiply-add in
+// non-finite value (its mark is raised): every block position's multiply-add in
 // the block kernels' order, so the same infinities and NaNs.  A fixed grid
 // walks all (task, 64-column chunk) pairs, one column per lane; without the
-// flag every workgroup leaves at once.
-static __global__ __launch_bounds__(64) void k_sweep_repair(const unsigned long long* __restrict__ flag,
+// mark every workgroup leaves at once.
+static __global__ __launch_bounds__(64) void k_sweep_repair(unsigned long long* __restrict__ mark,
                                                             unsigned long long token, SweepTasks t,
                                                             const uint2* __restrict__ words,
                                                             const int* __restrict__ sidx,
@@ -281,7 +301,7 @@ static __global__ __launch_bounds__(64) void k_sweep_repair(const unsigned long 
                                                             float* __restrict__ partial,
                                                             const int* __restrict__ rowmap, int M, int N,
                                                             int64_t ldb, int64_t ldc, int relu) {
-  if (*flag < token) return;
+  if (!mark_raised(token, mark)) return;
   const int n_chunks = (N + 63) / 64;
   for (int64_t i = blockIdx.x; i < (int64_t)t.n * n_chunks; i += gridDim.x) {
     const int task = (int)(i % t.n);

@@ -138,10 +138,11 @@ struct ColSweepTasks {   // block ranges; window null = window t, slot null = no
 int colsweep_rows_per_list(int64_t rows, int N);
 // Rows per half for the phase sweep (srbcrs_phasesweep.hpp); 0: the launch takes the lists.
 int phasesweep_rows(int64_t rows, int N, int64_t K);
+// token: the run's number, or 0 where the mark is its own (srbcrs_colsweep.hpp)
 hipError_t launch_colsweep(const ColSweep& s, const StreamArgs& a, int64_t K, unsigned long long token,
-                           unsigned long long* flag, hipStream_t st);
+                           unsigned long long* mark, hipStream_t st);
 hipError_t launch_colsweep_repair(const ColSweepTasks& t, const StreamArgs& a, unsigned long long token,
-                                  const unsigned long long* flag, hipStream_t st);
+                                  unsigned long long* mark, hipStream_t st);
 hipError_t launch_reduce(const ReduceArgs& a, int vec, hipStream_t st);
 hipError_t launch_csr(const CsrArgs& a, int vec, hipStream_t st);
 hipError_t launch_zero_rows(float* C, const int* rows, int n_rows, int N, int64_t ldc, hipStream_t st);

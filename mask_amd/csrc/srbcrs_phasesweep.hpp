@@ -65,7 +65,8 @@ template <int C, int WV>
 __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(4))) void spmm_phasesweep(
     PhaseStream s, const float* __restrict__ B, uint32_t b_bytes, float* __restrict__ Cout,
     float* __restrict__ partial, int N, uint32_t ldb4, int64_t ldc, int n_chunks, int swept, int relu,
-    unsigned long long token, unsigned long long* __restrict__ flag, int n_ids) {
+    unsigned long long token, unsigned long long* __restrict__ mark, int n_ids) {
+  mark_begin(token, mark);
   constexpr int LPG = C / 4, LG = 64 / LPG, SH = C == 32 ? 7 : 8, HALVES = WV * LG / 64;
   __shared__ __attribute__((aligned(16))) float tile[HALVES * kPhaseMaxRows * C];
   const int n_wg = s.n_units * (2 / HALVES);
@@ -76,7 +77,7 @@ __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(4))) vo
     const int i = (id - n_ids) * WV + wave;
     if (i < s.longs.n_long * ((N + 63) / 64))
       sweep_long_row(s.longs, i % s.longs.n_long, i / s.longs.n_long, B, b_bytes, Cout, partial, N, ldb4, ldc, relu,
-                     token, flag, lane);
+                     token, mark, lane);
     return;
   }
   int wg, c;
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(4))) vo
       __builtin_nontemporal_store(v, reinterpret_cast<f4*>(sweep_out(d, col, ldc, Cout, partial)));
     }
   }
-  if (__any(bad) && lane == 0) atomicMax(flag, token);
+  if (__any(bad) && lane == 0) mark_raise(token, mark);
 }
 
 // ---------------------------------------------------------------------------

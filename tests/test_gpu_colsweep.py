@@ -214,3 +214,47 @@ def test_capture_and_two_streams(gpu):
                 outs.append(plan.run(b))
     torch.cuda.synchronize()
     assert all(_same(o, (r1, r2)[i % 2]) for i, o in enumerate(outs))
+
+
+@pytest.mark.parametrize("M,per_row,N", [(65536, 16, 512), (20000, 20, 128)])   # a phase stream, a list stream
+def test_replay_after_a_non_finite_one(gpu, M, per_row, N):
+    """A captured run repairs the replays whose own sums are not finite and no
+    others: the ones after take as long as before."""
+    import torch
+    rng = np.random.default_rng(M)
+    cols = np.sort(rng.integers(0, M, (M, per_row)), axis=1).astype(np.int32).ravel()
+    plan = _plan((np.arange(M + 1, dtype=np.int32) * per_row, cols, rng.uniform(-1, 1, cols.size).astype(np.float32)), M)
+    fine = torch.rand((M, N), device="cuda") - 0.5
+    bad = fine.clone()
+    bad[int(cols[7])] = float("inf")
+    B, C = fine.clone(), torch.empty((M, N), device="cuda")
+    for _ in range(2):
+        plan.run(B, C)
+    refs = [plan.run(b, grid_order=1, depth=2, wg_cols=128) for b in (fine, bad)]
+    torch.cuda.synchronize()
+    print("[case] replays", M, per_row, N, flush=True)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        plan.run(B, C)
+
+    def replay(i):
+        B.copy_((fine, bad)[i])
+        C.fill_(7.0)
+        g.replay()
+        assert _same(C, refs[i])
+        best = float("inf")
+        for _ in range(10):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            g.replay()
+            e[1].record()
+            torch.cuda.synchronize()
+            best = min(best, e[0].elapsed_time(e[1]))
+        plan.run(B)   # eager work between replays
+        return best
+
+    before = replay(0)
+    for _ in range(2):
+        replay(1)
+        # the repair pass took ten times the sweep where it ran on
+        assert replay(0) < 1.5 * before + 0.01
