@@ -288,10 +288,16 @@ struct SweepTasks {
 };
 
 // The product again with A's zeros in it, where the column sweep stored a
-// non-finite value (its mark is raised): every block position's multiply-add in
-// the block kernels' order, so the same infinities and NaNs.  A fixed grid
-// walks all (task, 64-column chunk) pairs, one column per lane; without the
-// mark every workgroup leaves at once.
+// non-finite value (its mark is raised): the block kernels' matrix
+// instructions over all positions of the blocks, so the same infinities and
+// NaNs.  A fixed grid of waves walks all (task, 64-column chunk) pairs; without
+// the mark every one leaves at once.  A block's indices are fetched two blocks
+// ahead, its values and B rows one ahead.
+//
+// Bound as the block kernels are (gathers' L2 misses); one MI355X, the pass
+// alone: 65536 x 65536, 16 per row, N = 512 295 us (block kernels 275); 232965
+// of 50, N = 256 1680; 8000 of 16, N = 128 17.  One multiply-add per position
+// and column, its A values by scalar loads, took 1615, 8080 and 104.
 static __global__ __launch_bounds__(64) void k_sweep_repair(unsigned long long* __restrict__ mark,
                                                             unsigned long long token, SweepTasks t,
                                                             const uint2* __restrict__ words,
@@ -303,33 +309,59 @@ static __global__ __launch_bounds__(64) void k_sweep_repair(unsigned long long* 
                                                             int64_t ldb, int64_t ldc, int relu) {
   if (!mark_raised(token, mark)) return;
   const int n_chunks = (N + 63) / 64;
+  const int j = threadIdx.x & 15, k = threadIdx.x >> 4;   // A: row j, column 2 k + step; B: 4 columns from 4 j
   for (int64_t i = blockIdx.x; i < (int64_t)t.n * n_chunks; i += gridDim.x) {
     const int task = (int)(i % t.n);
-    const int col = (int)(i / t.n) * 64 + (int)threadIdx.x;
-    if (col >= N) continue;
-    float acc[16];
+    const int col = (int)(i / t.n) * 64 + 4 * j;
+    const float* Bc = B + (col < N ? col : N - 4);   // columns past N: the last again (not stored)
+    const int64_t b0 = t.begin[task], b1 = t.end[task];
+    f4 acc[4];   // [column of the 4][row of rows 4 k ..]
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    for (int64_t b = t.begin[task]; b < t.end[task]; ++b)
-      for (int k = 0; k < 8; ++k) {
-        const int q = ((2 * k) & 7) | (k >> 2);
-        const float bv = B[(int64_t)sidx[8 * b + q] * ldb + col];
+    for (int c = 0; c < 4; ++c) acc[c] = f4{0.f, 0.f, 0.f, 0.f};
+    int2 ix = int2{0, 0};
+    uint2 wd = uint2{0u, 0u};
+    float a0 = 0.f, a1 = 0.f;
+    f4 v0, v1;
+    auto fetch = [&](int64_t b) {
+      if (b >= b1) b = b1 - 1;
+      ix = *reinterpret_cast<const int2*>(sidx + 8 * b + 2 * k);
+      wd = words[4 * b + (j >> 2)];
+    };
+    auto load = [&] {
+      v0 = *reinterpret_cast<const f4*>(Bc + (int64_t)ix.x * ldb);
+      v1 = *reinterpret_cast<const f4*>(Bc + (int64_t)ix.y * ldb);
+      const int bit = 8 * (j & 3) + 2 * k;
+      const uint32_t n = wd.y + (uint32_t)__builtin_popcount(wd.x & ((1u << bit) - 1u)), own = (wd.x >> bit) & 3u;
+      const float p0 = packed[n], p1 = packed[n + (own & 1u)];   // (zeros follow the stored values)
+      a0 = (own & 1u) ? p0 : 0.f;
+      a1 = (own & 2u) ? p1 : 0.f;
+    };
+    if (b0 < b1) {
+      fetch(b0);
+      load();
+      fetch(b0 + 1);
+    }
+    for (int64_t b = b0; b < b1; ++b) {
+      const f4 w0 = v0, w1 = v1;
+      const float x0 = a0, x1 = a1;
+      load();
+      fetch(b + 2);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const uint2 w = words[4 * b + (r >> 2)];
-          const int bit = 8 * (r & 3) + q;
-          const float a = ((w.x >> bit) & 1u) ? packed[w.y + __builtin_popcount(w.x & ((1u << bit) - 1u))] : 0.f;
-          acc[r] = __builtin_fmaf(a, bv, acc[r]);
-        }
-      }
+      for (int c = 0; c < 4; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x0, w0[c], acc[c], 0, 0, 0);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x1, w1[c], acc[c], 0, 0, 0);
+    }
     const int slot = t.slot ? t.slot[task] : -1;
+    if (col >= N) continue;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
+    for (int r = 0; r < 4; ++r) {
+      f4 v = f4{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
       if (slot >= 0) {
-        partial[((int64_t)slot * 16 + r) * ldc + col] = acc[r];
+        *reinterpret_cast<f4*>(partial + ((int64_t)slot * 16 + 4 * k + r) * ldc + col) = v;
       } else {
-        const int64_t row = (int64_t)(t.window ? t.window[task] : task) * 16 + r;
-        if (row < M) C[(int64_t)(rowmap ? rowmap[row] : row) * ldc + col] = relu ? relu1(acc[r]) : acc[r];
+        const int64_t row = (int64_t)(t.window ? t.window[task] : task) * 16 + 4 * k + r;
+        if (relu) v = relu4(v);
+        if (row < M) *reinterpret_cast<f4*>(C + (int64_t)(rowmap ? rowmap[row] : row) * ldc + col) = v;
       }
     }
   }

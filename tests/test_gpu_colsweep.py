@@ -158,6 +158,28 @@ def test_non_finite_dense_values(gpu, policy):
         _check(plan, fine, "finite again")
 
 
+@pytest.mark.parametrize("policy", [("row", 0), ("split", 7)])
+@pytest.mark.parametrize("N", [16, 48, 112, 256])
+def test_non_finite_at_every_width(gpu, N, policy):
+    """The repair pass over chunks that end inside 64 columns, a last window
+    that is not whole, windows without a block, and a row order."""
+    import torch
+    M, K = 1501, 20000
+    rowptr, colind, values = _csr(M, K, 14, 2, N)
+    empty = np.repeat(np.arange(M) // 16 % 9 == 4, np.diff(rowptr))   # the windows 4, 13, ... hold nothing
+    lens = np.where(np.arange(M) // 16 % 9 == 4, 0, np.diff(rowptr))
+    csr = (np.concatenate([[0], np.cumsum(lens)]).astype(np.int32), colind[~empty], values[~empty])
+    B = torch.from_numpy(np.random.default_rng(N).uniform(-1, 1, (K, N)).astype(np.float32)).cuda()
+    B[csr[1][::97].astype(np.int64), N // 2] = float("inf")
+    B[csr[1][5:9].astype(np.int64), N - 1] = float("nan")
+    for kw in ({}, dict(row_order="first_col_sort", K=K)):
+        plan = _plan(csr, M, **kw)
+        plan.set_schedule(*policy)
+        print("[case] non-finite width", N, policy, kw, flush=True)
+        assert not bool(torch.isfinite(_check(plan, B, (N, policy, kw))).all())
+        _check(plan, B, (N, policy, kw, "relu"), relu=True)
+
+
 @pytest.mark.parametrize("order", ["first_col_sort", "sparse_rows"])
 def test_row_orders_and_strides(gpu, order):
     import torch
