@@ -239,6 +239,11 @@ int srbcrs_run(srbcrs_plan *plan, const float *d_B, int64_t K, int64_t N, int64_
  * keeps one global cache entry). */
 int srbcrs_plan_trim(srbcrs_plan *plan, void *stream);
 
+/* Give that kept device memory of the current device back to the driver, with
+ * or without a plan at hand: for a process whose other allocators (PyTorch's)
+ * need it.  A failing allocation of this library does so by itself. */
+int srbcrs_release_memory(void);
+
 /* Launch knobs of the SR-BCRS kernels (template parameters; each maps a
  * knob of the reference's strategy schema, strategy_agent.py:81-130):
  *   depth        blocks in flight per wave: 2, 4 or 8 (0 = 2); the

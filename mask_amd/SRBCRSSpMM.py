@@ -297,8 +297,18 @@ _cache: Dict[int, _Entry] = {}
 
 
 def clear_cache() -> None:
+    """Drop the preprocessed graphs.  Their device memory is kept for the next
+    ones (at most 4 GiB a process, beside PyTorch's own cache); release_memory
+    gives it back."""
     with _cache_mu:
         _cache.clear()
+
+
+def release_memory() -> None:
+    """Give the device memory that dropped plans have left back to the driver
+    (srbcrs_release_memory, current device), as torch.cuda.empty_cache does
+    for PyTorch's."""
+    _capi.check(_capi.lib().srbcrs_release_memory())
 
 
 def _preprocess(colind: Tensor, rowptr: Tensor, values: Tensor, num_nodes: int, blk_h: int, blk_w: int,

@@ -40,6 +40,7 @@ EXPORTS = (
     "srbcrs_row_order", "srbcrs_pack_count", "srbcrs_pack_fill", "srbcrs_plan_create_ex", "srbcrs_plan_row_order",
     "srbcrs_plan_tune", "srbcrs_plan_tune_ex", "srbcrs_shard_windows", "srbcrs_run_noalloc", "srbcrs_noalloc_scratch_floats",
     "srbcrs_plan_trim",
+    "srbcrs_release_memory",
 )
 
 _i32p = ctypes.POINTER(ctypes.c_int32)
@@ -153,6 +154,7 @@ def lib() -> ctypes.CDLL:
                                ctypes.c_int),
         "srbcrs_noalloc_scratch_floats": ([], ctypes.c_size_t),
         "srbcrs_plan_trim": ([_vp, _vp], ctypes.c_int),
+        "srbcrs_release_memory": ([], ctypes.c_int),
     }
     for name, (args, res) in sig.items():
         f = getattr(L, name)

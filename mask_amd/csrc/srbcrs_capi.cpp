@@ -383,8 +383,9 @@ Schedule* build_schedule(const int32_t* soff, int32_t Mo, const char* policy_c, 
 template <class T>
 T* dev_alloc(size_t n, bool reuse = false) {
   if (n == 0) n = 1;
-  void* p = srbcrs::pool_alloc(n * sizeof(T), !reuse);
-  if (!p) fail(SRBCRS_ENOMEM, "allocation of %zu bytes of device memory failed", n * sizeof(T));
+  hipError_t why = hipErrorOutOfMemory;
+  void* p = srbcrs::pool_alloc(n * sizeof(T), !reuse, &why);
+  if (!p) fail(SRBCRS_ENOMEM, "hipMalloc(%zu bytes) failed: %s", n * sizeof(T), hipGetErrorString(why));
   return static_cast<T*>(p);
 }
 
@@ -1761,6 +1762,14 @@ int srbcrs_plan_trim(srbcrs_plan* plan, void* stream) {
       w.built = false;
     }
     srbcrs::pool_release(plan->device);
+  });
+}
+
+int srbcrs_release_memory(void) {
+  return guarded([] {
+    int cur = 0;
+    hip_check(hipGetDevice(&cur), "hipGetDevice");
+    srbcrs::pool_release(cur);
   });
 }
 

@@ -28,11 +28,14 @@ Pool& pool() {
   return *p;
 }
 
-// 8 sizes per octave, so that arrays of similar graphs fit each other's blocks.
+// 8 sizes per octave, so that arrays of similar graphs fit each other's
+// blocks; 32 from 16 MB on, where an eighth of the size is much to leave
+// unused; blocks that are not kept as they are.
 size_t size_class(size_t n) {
   if (n <= 4096) return 4096;
+  if (n > kPoolBytes) return n;
   const int o = 63 - __builtin_clzll((unsigned long long)n);
-  const size_t step = size_t(1) << (o - 3);
+  const size_t step = size_t(1) << (o - (o < 24 ? 3 : 5));
   return (n + step - 1) / step * step;
 }
 
@@ -60,14 +63,17 @@ std::list<Block> take(Pool& P, int device, size_t room) {
 
 }  // namespace
 
-void* pool_alloc(size_t bytes, bool fresh) {
+void* pool_alloc(size_t bytes, bool fresh, hipError_t* why) {
   Pool& P = pool();
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) {
+  hipError_t e = hipGetDevice(&dev);
+  auto refused = [&] {
     (void)hipGetLastError();
+    if (why) *why = e;
     return nullptr;
-  }
-  const size_t want = size_class(bytes);
+  };
+  if (e != hipSuccess) return refused();
+  const size_t want = fresh ? bytes : size_class(bytes);
   if (!fresh) {
     std::lock_guard<std::mutex> lock(P.mu);
     auto best = P.kept.end();
@@ -84,16 +90,13 @@ void* pool_alloc(size_t bytes, bool fresh) {
     }
   }
   Block b{nullptr, want, dev};
-  const hipError_t e = hipMalloc(&b.p, want);
-  if (e != hipSuccess) {
+  e = hipMalloc(&b.p, want);
+  if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
-    if (e != hipErrorOutOfMemory) return nullptr;
     pool_release(dev);
-    if (hipMalloc(&b.p, want) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
+    e = hipMalloc(&b.p, want);
   }
+  if (e != hipSuccess) return refused();
   std::lock_guard<std::mutex> lock(P.mu);
   P.live.emplace(b.p, b);
   return b.p;

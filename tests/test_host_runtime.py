@@ -178,3 +178,29 @@ for N in (64, 512):   # built again, by the second run at the latest
     assert launches("spmm_colsweep") + launches("spmm_phasesweep") == n + 1
 L.srbcrs_plan_destroy(h)
 """)
+
+
+def test_kept_memory_is_bounded_in_waste_and_given_back(fake_hip):
+    """A large block is at most a thirty-second more than asked for, what a run
+    allocates is just that, and with no plan left all memory can be released."""
+    _run(fake_hip, """
+M, N = 300000, 512
+c = csr(M, 20000, 1)
+blocks = 131073
+head(blocks, c[1].size, 19999)
+calls = []
+rc, h = create(c, M, 1)
+assert rc == 0, error()
+d = _capi.PlanDesc()
+L.srbcrs_plan_get(h, ctypes.byref(d))
+assert d.total_blocks == blocks
+L.srbcrs_plan_trim(h, None)
+own = 4 * (M // 16 + 2) + 8 * c[1].size + 4 * M // 16 + blocks * (512 + 32 + 32) + 4 * c[1].size
+assert own <= fake.fake_live_bytes() < own * 33 // 32 + (1 << 20)
+L.srbcrs_plan_destroy(h)
+assert fake.fake_live_bytes() >= own
+assert L.srbcrs_release_memory() == 0 and fake.fake_live_bytes() == 0
+fake.fake_fail_malloc(0, 1 << 30)
+rc, h = create(c, M, 1)
+assert rc == _capi.SRBCRS_ENOMEM and "out of memory" in error(), error()
+""")
