@@ -60,6 +60,9 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
     lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
+_NO_KNOBS = (0, 0, 0, 0, 0, "default", "default")   # Plan.run's knobs at their defaults
+
+
 class Plan:
     """A device-resident SR-BCRS matrix (owns a ``srbcrs_plan``)."""
 
@@ -190,8 +193,7 @@ class Plan:
         "compact" / "dense" picks the block-value copy the kernel reads; b_stage
         "registers" / "lds" where the ring holds the gathered B rows)."""
         out = self._operands(dense, out)
-        if not (depth or tile_b or wg_cols or grid_order or windows_per_wave or relu or a_operand != "default"
-                or b_stage != "default"):
+        if not relu and (depth, tile_b, wg_cols, grid_order, windows_per_wave, a_operand, b_stage) == _NO_KNOBS:
             opts = None   # srbcrs_run_ex: NULL = defaults
         else:
             opts = _capi.RunOpts(int(depth), int(tile_b), int(wg_cols), int(grid_order), int(windows_per_wave),

@@ -198,6 +198,21 @@ def test_csr_row_groups(gpu, shape):
     assert_gate(gate(out[:M].cpu().numpy(), rowptr, colind, values, np.ascontiguousarray(B[:, :N]), M))
 
 
+def test_values_that_are_no_knobs_are_refused(gpu):
+    """Also those that are false in a condition, like the knobs' defaults."""
+    torch = _torch()
+    from mask_amd.SRBCRSSpMM import Plan
+    rowptr, colind, values = random_csr(64, 64, 0.1, 3)
+    plan = Plan(*(torch.from_numpy(a).cuda() for a in (rowptr, colind, values)), 64)
+    B = torch.ones((64, 16), device="cuda")
+    _say("no knobs")
+    for kw in (dict(depth=None), dict(tile_b=""), dict(wg_cols=[]), dict(grid_order=None), dict(windows_per_wave={}),
+               dict(a_operand=None), dict(b_stage="")):
+        with pytest.raises((TypeError, ValueError, KeyError)):
+            plan.run(B, **kw)
+    assert torch.equal(plan.run(B, depth=0.0, tile_b=False), plan.run(B))
+
+
 @pytest.mark.parametrize("blk", [(16, 8), (32, 32)])
 def test_knobs_are_bitwise_invariant(gpu, blk):
     """Depth, tile_b, workgroup width, grid order and windows-per-wave change
