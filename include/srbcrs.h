@@ -216,7 +216,8 @@ int srbcrs_plan_set_schedule(srbcrs_plan *plan, const char *policy, int32_t para
  * included); it needs ldb, ldc multiples of 4, 16-byte aligned B and C and
  * K * ldb * 4 < 2^32, and runs from a width's second run on, which builds its
  * entry stream: it allocates 8 bytes per stored value plus up to 7 entries of
- * padding per list (16 bytes a value in all on rows of 4).  Widths share
+ * padding per list (16 bytes a value in all on rows of 4; streams under 16 MB
+ * take room for the most they may need).  Widths share
  * streams where their layout is the same, and always once a schedule's streams
  * together hold as many bytes as the plan's block values.  Capture after two
  * eager runs to capture the sweep.  Elsewhere, under

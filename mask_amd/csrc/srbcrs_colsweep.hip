@@ -330,8 +330,15 @@ hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc
   constexpr int64_t kLongMin = 128;
   const int64_t long_len = std::max<int64_t>(kLongMin, in.n_values / n_lists);
   const int long_bin = sweep_bin((int)long_len);
-  // rows past kLongMin values; explicit zeros count (k_sweep_len)
-  const int64_t long_cap = (in.n_values + in.n_values / 16 + 4096) / kLongMin + 1;
+  // stored values, and room for explicit zeros (k_sweep_len counts them)
+  const int64_t most = in.n_values + in.n_values / 16 + 4096;
+  const int64_t long_cap = most / kLongMin + 1;   // rows past kLongMin values
+  // Small streams take room for the most their lists may need, which saves a
+  // wait for the sum (25 us of the 110 of a 4096-row matrix); large ones, where
+  // it would be a third more than they need, wait.
+  int64_t cap = most + kSweepBatch * n_lists + kSweepLongBatch * long_cap;
+  const bool ahead = cap * 8 <= (16 << 20);
+  if (!ahead) cap = INT32_MAX;
   int *len = nullptr, *hist = nullptr, *vrow = nullptr, *list_len = nullptr, *lvrow = nullptr;
   unsigned long long* total = nullptr;
   bool idle = true;
@@ -379,6 +386,7 @@ hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc
   out.lstart = (int*)keep((size_t)long_cap * 4);
   out.lnblk = (int*)keep((size_t)long_cap * 4);
   out.ldest = (int*)keep((size_t)long_cap * 4);
+  if (ahead) out.entries = (uint2*)keep((size_t)(cap + 8) * 8);
   if (!room) return cleanup(hipErrorOutOfMemory);
 #define SRBCRS_STEP(x)                          \
   do {                                          \
@@ -400,28 +408,37 @@ hipError_t build_colsweep(const ColSweepIn& in, ColSweep& out, DeviceAlloc alloc
                      RL, long_bin, in.rowmap, in.M, vrow, out.dest, list_len, lvrow, out.ldest, (int)long_cap, n_long);
   SRBCRS_STEP(hipGetLastError());
   const int n8 = (int)(n_lists / 8);
-  hipLaunchKernelGGL(k_sweep_place, dim3((unsigned)((n8 + 63) / 64)), dim3(64), 0, st, list_len, n8,
-                     (int64_t)INT32_MAX, out.start, out.nblk, out.wblk8, out.wblk4, total);
+  hipLaunchKernelGGL(k_sweep_place, dim3((unsigned)((n8 + 63) / 64)), dim3(64), 0, st, list_len, n8, cap, out.start,
+                     out.nblk, out.wblk8, out.wblk4, total);
   SRBCRS_STEP(hipGetLastError());
   hipLaunchKernelGGL(k_sweep_place_long, dim3((unsigned)((long_cap + 63) / 64)), dim3(64), 0, st, len, lvrow, n_long,
-                     (int)long_cap, (int64_t)INT32_MAX, out.lstart, out.lnblk, total);
+                     (int)long_cap, cap, out.lstart, out.lnblk, total);
   SRBCRS_STEP(hipGetLastError());
   unsigned long long h_total[2] = {0, 0};
-  SRBCRS_STEP(hipMemcpyAsync(h_total, total, 16, hipMemcpyDeviceToHost, st));
-  SRBCRS_STEP(hipStreamSynchronize(st));
-  out.n_long = (int)(h_total[1] & 0xffffffffu);
-  out.n_entries = (int64_t)h_total[0];
-  if (h_total[0] > (unsigned long long)INT32_MAX - 64 || out.n_long > long_cap) return cleanup(hipErrorInvalidValue);
-  out.entries = (uint2*)keep((size_t)(out.n_entries + 8) * 8);
-  if (!out.entries) return cleanup(hipErrorOutOfMemory);
-  hipLaunchKernelGGL(k_sweep_fill, dim3((unsigned)((slots + 7) / 8 + (out.n_long + 7) / 8)), dim3(64),
+  auto fetch_total = [&]() -> hipError_t {
+    const hipError_t e = hipMemcpyAsync(h_total, total, 16, hipMemcpyDeviceToHost, st);
+    return e == hipSuccess ? hipStreamSynchronize(st) : e;
+  };
+  auto fits = [&] {
+    out.n_long = (int)(h_total[1] & 0xffffffffu);
+    out.n_entries = (int64_t)h_total[0];
+    return h_total[0] <= (unsigned long long)cap - (ahead ? 0 : 64) && out.n_long <= long_cap;
+  };
+  if (!ahead) {
+    SRBCRS_STEP(fetch_total());
+    if (!fits()) return cleanup(hipErrorInvalidValue);
+    out.entries = (uint2*)keep((size_t)(out.n_entries + 8) * 8);
+    if (!room) return cleanup(hipErrorOutOfMemory);
+  }
+  const int64_t longs = ahead ? long_cap : out.n_long;
+  hipLaunchKernelGGL(k_sweep_fill, dim3((unsigned)((slots + 7) / 8 + (longs + 7) / 8)), dim3(64),
                      32 * out.phases * 4, st, t, in.words, in.sidx, in.packed, vrow, slots, RL, list_len, out.start,
                      out.nblk, out.phases, out.shift, lvrow, len, out.lstart, out.lnblk, n_long, (int)long_cap,
                      out.entries);
   SRBCRS_STEP(hipGetLastError());
-  SRBCRS_STEP(hipStreamSynchronize(st));
+  SRBCRS_STEP(ahead ? fetch_total() : hipStreamSynchronize(st));
 #undef SRBCRS_STEP
-  return cleanup(hipSuccess);
+  return cleanup(fits() ? hipSuccess : hipErrorInvalidValue);
 }
 
 }  // namespace srbcrs
