@@ -804,6 +804,36 @@ bool sweep_wanted(const srbcrs_plan& plan) {
          plan.max_col < kSweepKeyCols && 9 * plan.n_apacked < plan.total * 128;
 }
 
+// Rows whose B rows hardly any other row in flight reads: nothing for the sweep
+// to share, and the block kernels' 64-column gathers (N a multiple of 64) take
+// less than its lists and its second launch.  Measured on 510 products of
+// uniform matrices (2000 to 600000 rows, 1e4 to 1e6 columns, 4 to 40 values a
+// row, N = 64, 256, 512): 10 of them over 3 % slower than the block kernels, by
+// 12 % at most, and 1 % in the mean behind the faster side.  us, sweep / blocks:
+// - `in_flight`: the rows whose sums an XCD holds at a time (1280 on each of 32
+//   CUs, or its part of all), times the values a row over the columns = how
+//   often a B row is read while they are in flight.
+// - too few rows to fill the chip with lists, though the blocks do: 20000 x
+//   300000, 16 per row, N = 256 58 / 51 (sharing 1.1); 60000 x 300000, 16 per row,
+//   N = 64 44 / 37 (0.8); on the other side 60000 x 100000, 16 per row 36 / 36 (2.4).
+//   Where the blocks do not fill it either: 2000 x 100000, 40 per row, N = 256
+//   17 / 43 (0.8).
+// - very short rows: 200000 x 300000, 4 per row, N = 512 331 / 283 (0.55); 100000
+//   columns, 283 / 274 (1.6); but 1000000 columns, 24 per row 1441 / 1781 (1.0).
+// - and the short ones with less than two values a column: 60000 x 1000000, 8 per
+//   row, N = 256 97 / 86, N = 512 204 / 189; but N = 96, where the block kernels
+//   take 32 columns, 20000 x 300000, 10 per row 19 / 25.
+bool blocks_share_enough(const srbcrs_plan& plan, int64_t N) {
+  const int64_t M = plan.num_nodes, K = (int64_t)plan.max_col + 1, nv = plan.n_apacked;
+  const int64_t chunks = (N + 31) / 32;
+  const int64_t in_flight = std::min<int64_t>(M * std::min<int64_t>(chunks, 8) / 8, 1280 * 32);
+  const double sharing = (double)in_flight * (double)nv / ((double)M * (double)K);
+  const bool blocks_fill = M / 16 * (N / 64) >= 2000, lists_fill = M / 64 * chunks >= 3000;
+  if (blocks_fill && !lists_fill && sharing < 2.0) return true;
+  if (blocks_fill && sharing < 0.8 && nv <= 6 * M) return true;
+  return nv <= 2 * K && nv <= 11 * M;
+}
+
 // The column sweep stream for a run of N columns; null: run the block
 // kernels, which give the same bits.  The first run of a width does that: a
 // plan run once (a sampled graph) does not pay for the stream, which takes
@@ -825,15 +855,7 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
   capturing = !known || cs != hipStreamCaptureStatusNone;
   const srbcrs::ColSweepTasks t = sweep_tasks(plan);
   const int64_t rows = (int64_t)t.n * 16;
-  // Short rows whose B rows hardly any other row reads: nothing to share, and
-  // the block kernels' 64-column gathers take less than the sweep's lists and
-  // its second launch (us, sweep / block: 5710 x 141462, 9 per row, N = 512 26 /
-  // 23; 100000 x 400000, 4 per row, N = 256 98 / 81; but 3000 x 200000, 30 per
-  // row, N = 256 19 / 39, and N = 96, where the block kernels take 32 columns,
-  // 20000 x 300000, 10 per row 19 / 25).
-  if (N % 64 == 0 && plan.n_apacked <= 2 * ((int64_t)plan.max_col + 1) &&
-      plan.n_apacked <= 11 * (int64_t)plan.num_nodes)
-    return nullptr;
+  if (N % 64 == 0 && blocks_share_enough(plan, N)) return nullptr;
   // the layouts to try: the phase sweep's, where it is the faster one, and the
   // lists' (keyed by minus the rows per half, and the rows per list)
   const int layouts[2] = {-srbcrs::phasesweep_rows(rows, (int)N, (int64_t)plan.max_col + 1),
@@ -847,13 +869,23 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
   for (int layout : layouts) {
     if (!layout) continue;
     srbcrs_plan::Sweep& w = plan.sweeps[{plan.sched.policy, plan.sched.param, layout}];
-    if (!w.longest)
-      for (int32_t i = 0; i < plan.Mo; ++i) w.longest = std::max(w.longest, plan.h_soff[i + 1] - plan.h_soff[i]);
+    if (!w.longest) {
+      const Schedule& d = plan.sched;
+      for (size_t i = 0; i < d.task_begin.size(); ++i) w.longest = std::max(w.longest, d.task_end[i] - d.task_begin[i]);
+      if (d.policy == "row")
+        for (int32_t i = 0; i < plan.Mo; ++i) w.longest = std::max(w.longest, plan.h_soff[i + 1] - plan.h_soff[i]);
+    }
     // Small products stay with the block kernel's one launch (the sweep's repair
     // pass is a second one, 4 us of host time): under 64 MB of gathers both take
-    // less than their launches, unless long windows make the block kernel a
-    // chain (about 0.4 us a block: 40 blocks 17.9 us, sweep 8 + 1.5).
-    if (plan.n_apacked * N < (16 << 20) && w.longest < 24) return nullptr;
+    // less than their launches, unless long tasks make the block kernel a
+    // chain (about 0.4 us a block: 40 blocks 17.9 us, sweep 8 + 1.5; power-law
+    // graph of 4096 nodes and 153 K values, N = 64, blocks / sweep: whole windows
+    // 67 / 16, split:64 27 / 20, split:32 17.8 / 20.9, split:16 15.1 / 21.7).
+    // Tasks of 8 blocks and less cost the sweep a list row each for a few
+    // values: it is slower up to 64 columns (8000 nodes, 377 K values, split:8,
+    // N = 64 32 / 40, N = 256 74 / 69).
+    if (w.longest < 24 && plan.n_apacked * N < (16 << 20)) return nullptr;
+    if (w.longest <= 8 && plan.sched.policy != "row" && N <= 64) return nullptr;
     if (w.built) return take(w);
     if (w.unfit) continue;
     srbcrs_plan::Sweep* near = nullptr;   // built, of this schedule

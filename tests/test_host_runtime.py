@@ -204,3 +204,31 @@ fake.fake_fail_malloc(0, 1 << 30)
 rc, h = create(c, M, 1)
 assert rc == _capi.SRBCRS_ENOMEM and "out of memory" in error(), error()
 """)
+
+
+# (M, K, values a row, N, schedule, whether the second run is a sweep): both sides of the dispatch rules
+@pytest.mark.parametrize("M,K,per_row,N,schedule,sweep", [
+    (20000, 300000, 16, 256, "row:0", False), (20000, 60000, 10, 256, "row:0", True),     # too few rows for the lists
+    (60000, 300000, 16, 64, "row:0", False), (60000, 100000, 16, 64, "row:0", True),
+    (2000, 100000, 40, 256, "row:0", True), (20000, 300000, 10, 224, "row:0", True),
+    (200000, 300000, 4, 256, "row:0", False), (200000, 300000, 12, 256, "row:0", True),   # very short rows
+    (100000, 400000, 7, 256, "row:0", False),                                             # few values a column
+    (4096, 4096, 20, 64, "row:0", True), (4096, 4096, 20, 64, "split:16", False),         # small: long tasks only
+    (4096, 4096, 20, 64, "split:32", True), (4096, 4096, 20, 16, "row:0", True),
+    (20000, 20000, 20, 64, "split:8", False), (20000, 20000, 20, 64, "split:9", True),    # short tasks
+    (20000, 20000, 20, 128, "split:8", True), (1000, 1000, 4, 64, "row:0", False),
+])
+def test_which_runs_are_sweeps(fake_hip, M, K, per_row, N, schedule, sweep):
+    _run(fake_hip, f"""
+M, K, N = {M}, {K}, {N}
+big = dict(B=np.zeros(N * K + 8, np.float32), C=np.zeros(N * M + 8, np.float32))
+h = sparse_plan(M, K, {per_row})
+d2h(np.array([M * {per_row} * 5 // 4, 0], np.uint64))
+d2h(np.array([M * {per_row} * 5 // 4, 0, M * {per_row}, M * {per_row}], np.uint64))
+policy, param = "{schedule}".split(":")
+assert L.srbcrs_plan_set_schedule(h, policy.encode(), int(param)) == 0, error()
+for i in range(2):
+    assert run(h, M, K, N, **big) == 0, error()
+assert launches("spmm_colsweep") + launches("spmm_phasesweep") == {int(sweep)}
+assert launches("spmm_stream") == {2 - int(sweep)}
+""")
