@@ -490,6 +490,8 @@ struct srbcrs_plan {
   // then four words for each of up to kCapturedMarks runs recorded into graphs
   // (any past those are numbered, and repair on every replay once marked)
   unsigned long long* d_sweep_marks = nullptr;
+  int32_t longest_window = 0;   // in blocks (0: not counted yet)
+  double window_span = 0;       // mean of the windows' column spans, once the marks are there
   std::atomic<unsigned long long> sweep_runs{0}, sweep_captures{0};
 
   template <class T>
@@ -795,21 +797,26 @@ srbcrs::ColSweepTasks sweep_tasks(const srbcrs_plan& plan) {
 }
 
 // Whether the default launch of this plan is the column sweep: 16x8 blocks
-// with the compact copy, less than a ninth of the block positions stored.
-// Measured at 65536 rows of 16 with window-clustered columns (us, sweep / block
-// kernel): fill 0.094 N = 64 28 / 31, N = 512 152 / 187; fill 0.116 28 / 27,
-// 150 / 156, and above it the block kernel shares each B row among more rows.
+// with the compact copy, less than a ninth of the block positions stored
+// (above it the block kernels share each B row among more rows: 65536 rows of 16
+// with window-clustered columns, us, sweep / block kernel: fill 0.094 N = 64
+// 28 / 31, N = 512 152 / 187; fill 0.116 28 / 27, 150 / 156), and not where
+// blocks_faster knows better.
 bool sweep_wanted(const srbcrs_plan& plan) {
   return plan.blk_h == 16 && plan.packing == SRBCRS_PACK_CONDENSED && plan.d_awords && plan.total > 0 &&
          plan.max_col < kSweepKeyCols && 9 * plan.n_apacked < plan.total * 128;
 }
 
-// Rows whose B rows hardly any other row in flight reads: nothing for the sweep
+// Where the block kernels take less than the sweep.  From products of uniform
+// matrices (2000 to 600000 rows, 1e4 to 1e6 columns, 4 to 40 values a row) and of
+// matrices whose windows' columns lie together, near the diagonal or anywhere
+// (4000 to 600000 rows, 4 to 60 values a row, fill 0.063 to 0.11), N = 16 to 512:
+// 3988 products, 2.4 % behind the faster side in the mean, 58 of them more than 5 %
+// slower than the block kernels, by 26 % at most.  us, sweep / blocks:
+//
+// Rows whose B rows hardly any other row in flight reads leave the sweep nothing
 // to share, and the block kernels' 64-column gathers (N a multiple of 64) take
-// less than its lists and its second launch.  Measured on 510 products of
-// uniform matrices (2000 to 600000 rows, 1e4 to 1e6 columns, 4 to 40 values a
-// row, N = 64, 256, 512): 10 of them over 3 % slower than the block kernels, by
-// 12 % at most, and 1 % in the mean behind the faster side.  us, sweep / blocks:
+// less than its lists and its second launch:
 // - `in_flight`: the rows whose sums an XCD holds at a time (1280 on each of 32
 //   CUs, or its part of all), times the values a row over the columns = how
 //   often a B row is read while they are in flight.
@@ -823,15 +830,66 @@ bool sweep_wanted(const srbcrs_plan& plan) {
 // - and the short ones with less than two values a column: 60000 x 1000000, 8 per
 //   row, N = 256 97 / 86, N = 512 204 / 189; but N = 96, where the block kernels
 //   take 32 columns, 20000 x 300000, 10 per row 19 / 25.
-bool blocks_share_enough(const srbcrs_plan& plan, int64_t N) {
+// At 16 columns a lane group is mostly idle: 600000 x 300000, 4 per row 70 / 49 (0.55);
+// 60000 x 100000, 12 per row 19 / 17 (0.9); but 600000 x 10000, 16 per row 109 / 142.
+//
+// Where a window's columns lie together its B rows come from the L2 under the
+// block kernels as well, and it gathers `reuse` times fewer of them:
+// - rows in flight are dealt by length from all over the matrix; past three
+//   rounds of them they no longer share the band: 200000 rows of 16 near the
+//   diagonal, reuse 1.07, N = 512 1.45 times the blocks' time (60000: 0.79).
+// - reuse against what a row's values give the sweep: 60000 rows of 16, N = 256 at
+//   reuse 1.2, 1.46, 1.6, 1.76 0.72, 0.87, 0.95, 1.06 times the blocks' time; of 8, at
+//   1.17, 1.31, 1.57 0.85, 0.90, 1.02; of 4, at 1.0, 1.14, 1.26 0.98, 1.01, 1.08; N = 16,
+//   16 per row, at 1.07, 1.2, 1.33 0.85, 0.98, 1.05.
+//   (N = 48 and other widths that the block kernels take 16 columns at a time
+//   stay with the sweep at every reuse.)
+// None of this holds for windows of unlike length: the block kernels' longest
+// ones are chains, and a power-law graph's hub columns are shared far beyond the
+// mean (40000 nodes, 9 per row, N = 16 22 / 46, N = 512 70 / 168).
+bool blocks_faster(srbcrs_plan& plan, int64_t N) {
   const int64_t M = plan.num_nodes, K = (int64_t)plan.max_col + 1, nv = plan.n_apacked;
+  const bool whole = N % 64 == 0;
+  if (whole && nv <= 2 * K && nv <= 11 * M) return true;
+  if (!plan.longest_window)
+    for (int32_t i = 0; i < plan.Mo; ++i)
+      plan.longest_window = std::max(plan.longest_window, plan.h_soff[i + 1] - plan.h_soff[i]);
+  if ((int64_t)plan.longest_window * plan.Mo > 4 * plan.total) return false;
+  constexpr int64_t kInFlight = 1280 * 32;
   const int64_t chunks = (N + 31) / 32;
-  const int64_t in_flight = std::min<int64_t>(M * std::min<int64_t>(chunks, 8) / 8, 1280 * 32);
-  const double sharing = (double)in_flight * (double)nv / ((double)M * (double)K);
-  const bool blocks_fill = M / 16 * (N / 64) >= 2000, lists_fill = M / 64 * chunks >= 3000;
-  if (blocks_fill && !lists_fill && sharing < 2.0) return true;
-  if (blocks_fill && sharing < 0.8 && nv <= 6 * M) return true;
-  return nv <= 2 * K && nv <= 11 * M;
+  const int64_t in_flight = std::min<int64_t>(M * std::min<int64_t>(chunks, 8) / 8, kInFlight);
+  const double per_row = (double)nv / (double)M, sharing = (double)in_flight * per_row / (double)K;
+  if (whole && M / 16 * (N / 64) >= 2000) {
+    if (M / 64 * chunks < 3000 && sharing < 2.0) return true;
+    if (sharing < 0.8 && nv <= 6 * M) return true;
+  }
+  if (N == 16 && sharing < 16.0 && nv < 20 * M) return true;
+  if (plan.window_span > 0 && 8 * plan.window_span < (double)K && (whole || N <= 32)) {
+    if (N >= 64 && M > 3 * kInFlight) return true;
+    const double reuse = (double)nv / (8.0 * (double)plan.total);
+    return reuse > 1.0 + 0.3 * std::log2(per_row / (N >= 64 ? 4 : N == 32 ? 5 : 10));
+  }
+  return false;
+}
+
+// The marks, and what blocks_faster asks about the windows' columns.
+hipError_t prepare_sweeps(srbcrs_plan& plan, hipStream_t st) {
+  constexpr size_t words = kMarkBytes / 8;
+  auto* marks = static_cast<unsigned long long*>(srbcrs::pool_alloc(kMarkBytes + 24));
+  if (!marks) return hipErrorOutOfMemory;
+  unsigned long long spans[3] = {0, 0, 0};
+  hipError_t e = hipMemsetAsync(marks, 0, kMarkBytes + 24, st);
+  if (e == hipSuccess) e = srbcrs::launch_window_spans(plan.d_soff, plan.d_sidx, plan.Mo, marks + words, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(spans, marks + words, 24, hipMemcpyDeviceToHost, st);
+  const hipError_t w = hipStreamSynchronize(st);   // runs on other streams may use the marks next
+  if (e == hipSuccess) e = w;
+  if (e != hipSuccess) {
+    srbcrs::pool_drop(marks);
+    return e;
+  }
+  if (spans[1]) plan.window_span = (double)spans[0] / (double)spans[1];
+  plan.d_sweep_marks = marks;
+  return hipSuccess;
 }
 
 // The column sweep stream for a run of N columns; null: run the block
@@ -855,12 +913,12 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
   capturing = !known || cs != hipStreamCaptureStatusNone;
   const srbcrs::ColSweepTasks t = sweep_tasks(plan);
   const int64_t rows = (int64_t)t.n * 16;
-  if (N % 64 == 0 && blocks_share_enough(plan, N)) return nullptr;
   // the layouts to try: the phase sweep's, where it is the faster one, and the
   // lists' (keyed by minus the rows per half, and the rows per list)
   const int layouts[2] = {-srbcrs::phasesweep_rows(rows, (int)N, (int64_t)plan.max_col + 1),
                           srbcrs::colsweep_rows_per_list(rows, (int)N)};
   std::lock_guard<std::mutex> lock(plan.sweep_mu);
+  if (blocks_faster(plan, N)) return nullptr;
   auto take = [&](srbcrs_plan::Sweep& w) {
     w.captured = w.captured || capturing;
     return &w.s;
@@ -911,6 +969,11 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
       return nullptr;
     }
     const RelaxedCapture relaxed;
+    hipError_t e = hipSuccess;
+    if (!plan.d_sweep_marks) {
+      e = prepare_sweeps(plan, st);
+      if (e == hipSuccess && blocks_faster(plan, N)) return nullptr;
+    }
     srbcrs::ColSweep s;
     if (layout < 0) {
       s.rows = -layout;
@@ -922,16 +985,6 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
       while ((plan.max_col >> s.shift) >= 128) ++s.shift;
       if (plan.max_col < 16384) s.shift = 24;
       s.phases = (plan.max_col >> s.shift) + 1;
-    }
-    hipError_t e = hipSuccess;
-    if (!plan.d_sweep_marks) {
-      plan.d_sweep_marks = static_cast<unsigned long long*>(srbcrs::pool_alloc(kMarkBytes));
-      e = plan.d_sweep_marks ? hipMemsetAsync(plan.d_sweep_marks, 0, kMarkBytes, st) : hipErrorOutOfMemory;
-      if (e == hipSuccess) e = hipStreamSynchronize(st);   // runs on other streams may use them next
-      if (e != hipSuccess) {
-        srbcrs::pool_drop(plan.d_sweep_marks);
-        plan.d_sweep_marks = nullptr;
-      }
     }
     srbcrs::ColSweepIn in{t, plan.d_awords, plan.d_sidx, plan.d_apacked, plan.n_apacked, plan.d_rowmap,
                           (int)plan.packed_rows, plan.total, plan.max_col};

@@ -79,6 +79,13 @@ static void pick_launch(int64_t rows, int RL, const StreamArgs& a, int64_t K, in
   swept = cols == 32 && rows >= kSweptRows;
 }
 
+hipError_t launch_window_spans(const int* soff, const int* sidx, int Mo, unsigned long long* out, hipStream_t st) {
+  const int64_t g = ((int64_t)Mo + 255) / 256;
+  if (g == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_window_spans, dim3((unsigned)(g < 1024 ? g : 1024)), dim3(256), 0, st, soff, sidx, Mo, out);
+  return hipGetLastError();
+}
+
 int colsweep_rows_per_list(int64_t rows, int N) {
   const int64_t chunks32 = (N + 31) / 32;
   int RL = 8;

@@ -370,6 +370,28 @@ static __global__ __launch_bounds__(64) void k_sweep_repair(unsigned long long* 
 // ---------------------------------------------------------------------------
 // Building the stream.
 
+// See launch_window_spans.
+static __global__ __launch_bounds__(256) void k_window_spans(const int* __restrict__ soff,
+                                                             const int* __restrict__ sidx, int Mo,
+                                                             unsigned long long* __restrict__ out) {
+  unsigned long long span = 0, n = 0;
+  for (int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x; w < Mo; w += (int64_t)gridDim.x * 256) {
+    const int64_t b0 = soff[w], b1 = soff[w + 1];
+    if (b0 == b1) continue;
+    span += (unsigned long long)(sidx[8 * b1 - 1] - sidx[8 * b0]) + 1;
+    ++n;
+  }
+#pragma unroll
+  for (int d = 32; d; d >>= 1) {
+    span += __shfl_xor(span, d);
+    n += __shfl_xor(n, d);
+  }
+  if ((threadIdx.x & 63) == 0 && n) {
+    atomicAdd(out, span);
+    atomicAdd(out + 1, n);
+  }
+}
+
 // Bins of row lengths: exact below 256, 8 per octave above.
 constexpr int kSweepBins = 512;
 __host__ __device__ inline int sweep_bin(int n) {

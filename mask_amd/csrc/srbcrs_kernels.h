@@ -132,6 +132,9 @@ struct ColSweepTasks {   // block ranges; window null = window t, slot null = no
   const int *begin, *end, *window, *slot;
   int n;
 };
+// out[0] += the spans (last column - first + 1) of the windows that hold a
+// block, out[1] += their number (16x8 blocks, columns ascending per window).
+hipError_t launch_window_spans(const int* soff, const int* sidx, int Mo, unsigned long long* out, hipStream_t st);
 // Rows per list for a launch of N columns over this many task rows: the most
 // that leave 2000 waves (256 CUs hold 5120; below that the lists' chains set
 // the time: 16384 rows of 20, N = 64: 27 us at 8 rows, 22 at 4 or 2).

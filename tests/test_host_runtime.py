@@ -146,11 +146,11 @@ d2h(np.array([entries, 0, M * 16, M * 16], np.uint64))              # a phase st
 trim = lambda: L.srbcrs_plan_trim(h, None)
 live = lambda: (trim(), fake.fake_live_bytes())[1]
 base = live()
-for N in range(16, 513, 16):
+for N in range(32, 513, 16):
     for i in range(3):
         assert run(h, M, K, N, **big) == 0, error()
     assert launches("spmm_stream") <= 2 * N // 16
-    assert launches("spmm_colsweep") + launches("spmm_phasesweep") >= N // 16   # at least the last of the three
+    assert launches("spmm_colsweep") + launches("spmm_phasesweep") >= N // 16 - 1   # at least the last of the three
     assert live() - base <= d.total_blocks * 512 + 8 * entries
 row = live()
 assert row - base > 3 * 8 * entries
@@ -206,29 +206,57 @@ assert rc == _capi.SRBCRS_ENOMEM and "out of memory" in error(), error()
 """)
 
 
-# (M, K, values a row, N, schedule, whether the second run is a sweep): both sides of the dispatch rules
-@pytest.mark.parametrize("M,K,per_row,N,schedule,sweep", [
-    (20000, 300000, 16, 256, "row:0", False), (20000, 60000, 10, 256, "row:0", True),     # too few rows for the lists
-    (60000, 300000, 16, 64, "row:0", False), (60000, 100000, 16, 64, "row:0", True),
-    (2000, 100000, 40, 256, "row:0", True), (20000, 300000, 10, 224, "row:0", True),
-    (200000, 300000, 4, 256, "row:0", False), (200000, 300000, 12, 256, "row:0", True),   # very short rows
-    (100000, 400000, 7, 256, "row:0", False),                                             # few values a column
-    (4096, 4096, 20, 64, "row:0", True), (4096, 4096, 20, 64, "split:16", False),         # small: long tasks only
-    (4096, 4096, 20, 64, "split:32", True), (4096, 4096, 20, 16, "row:0", True),
-    (20000, 20000, 20, 64, "split:8", False), (20000, 20000, 20, 64, "split:9", True),    # short tasks
-    (20000, 20000, 20, 128, "split:8", True), (1000, 1000, 4, 64, "row:0", False),
+# (M, K, values a row, N, schedule, span of a window's columns, whether the second run is a sweep):
+# both sides of the dispatch rules
+@pytest.mark.parametrize("M,K,per_row,N,schedule,span,sweep", [
+    (20000, 300000, 16, 256, "row:0", 0, False), (20000, 60000, 10, 256, "row:0", 0, True),   # too few rows for lists
+    (60000, 300000, 16, 64, "row:0", 0, False), (60000, 100000, 16, 64, "row:0", 0, True),
+    (2000, 100000, 40, 256, "row:0", 0, True), (20000, 300000, 10, 224, "row:0", 0, True),
+    (200000, 300000, 4, 256, "row:0", 0, False), (200000, 300000, 12, 256, "row:0", 0, True),  # very short rows
+    (100000, 400000, 7, 256, "row:0", 0, False),                                             # few values a column
+    (60000, 100000, 19, 16, "row:0", 0, False), (60000, 100000, 20, 16, "row:0", 0, True),    # 16 columns
+    (200000, 10000, 12, 16, "row:0", 0, True),
+    (200000, 200000, 16, 128, "row:0", 20000, False), (200000, 200000, 16, 128, "row:0", 30000, True),   # local, many rows
+    (60000, 60000, 16, 128, "row:0", 400, True), (200000, 200000, 16, 48, "row:0", 400, True),
+    (60000, 60000, 3, 256, "row:0", 400, False), (60000, 60000, 5, 256, "row:0", 400, True),  # reuse 1 of short local rows
+    (4096, 4096, 20, 64, "row:0", 0, True), (4096, 4096, 20, 64, "split:16", 0, False),       # small: long tasks only
+    (4096, 4096, 20, 64, "split:32", 0, True),
+    (20000, 20000, 20, 64, "split:8", 0, False), (20000, 20000, 20, 64, "split:9", 0, True),  # short tasks
+    (20000, 20000, 20, 128, "split:8", 0, True), (1000, 1000, 4, 64, "row:0", 0, False),
 ])
-def test_which_runs_are_sweeps(fake_hip, M, K, per_row, N, schedule, sweep):
+def test_which_runs_are_sweeps(fake_hip, M, K, per_row, N, schedule, span, sweep):
     _run(fake_hip, f"""
 M, K, N = {M}, {K}, {N}
 big = dict(B=np.zeros(N * K + 8, np.float32), C=np.zeros(N * M + 8, np.float32))
 h = sparse_plan(M, K, {per_row})
-d2h(np.array([M * {per_row} * 5 // 4, 0], np.uint64))
-d2h(np.array([M * {per_row} * 5 // 4, 0, M * {per_row}, M * {per_row}], np.uint64))
+windows = (M + 15) // 16
+d2h(np.array([windows * {span}, windows if {span} else 0, 0], np.uint64))            # the window spans
+d2h(np.array([M * {per_row} * 5 // 4, 0], np.uint64))                                # a list stream
+d2h(np.array([M * {per_row} * 5 // 4, 0, M * {per_row}, M * {per_row}], np.uint64))  # a phase stream
 policy, param = "{schedule}".split(":")
 assert L.srbcrs_plan_set_schedule(h, policy.encode(), int(param)) == 0, error()
-for i in range(2):
+for i in range(3):
     assert run(h, M, K, N, **big) == 0, error()
-assert launches("spmm_colsweep") + launches("spmm_phasesweep") == {int(sweep)}
-assert launches("spmm_stream") == {2 - int(sweep)}
+assert launches("spmm_colsweep") + launches("spmm_phasesweep") == 2 * {int(sweep)}
+assert launches("spmm_stream") == 3 - 2 * {int(sweep)}
+""")
+
+
+def test_windows_of_unlike_length_keep_the_sweep(fake_hip):
+    """Rows that would stay with the block kernels, but for a window 20 times as long."""
+    for heavy, sweep in ((10, 0), (4000, 2)):
+        _run(fake_hip, f"""
+M, K, N = 60000, 60000, 16
+rp, cols, vals = csr(M, K, 10)
+cols = np.concatenate([np.sort(np.random.default_rng(1).choice(K, {heavy}, replace=False)).astype(np.int32), cols[10:]])
+rp[1:] += {heavy} - 10
+vals = np.ones(cols.size, np.float32)
+d2h(np.array([0, cols.size], np.uint32))
+rc, h = create((rp, cols, vals), M, 0)
+assert rc == 0, error()
+d2h(np.array([M * 13, 0], np.uint64))
+d2h(np.array([M * 13, 0, M * 10, M * 10], np.uint64))
+for i in range(3):
+    assert run(h, M, K, N) == 0, error()
+assert launches("spmm_colsweep") + launches("spmm_phasesweep") == {sweep}
 """)
