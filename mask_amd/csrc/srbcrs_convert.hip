@@ -17,14 +17,16 @@
 // Bound: the dense values, 512 bytes a block, written once (11.7 M edges of a
 // power-law graph, 232965 rows, 1.4 M blocks: 0.71 GB of 0.95 GB moved, 190 us
 // at the rate of a copy).  Measured on that graph (one MI355X): the windows 460
-// us, the sort, ranks and second scan of the 15 windows longer than LDS holds
-// 350, blocks 380, scan 21; the whole call 1.40 ms.  Sorting the whole matrix
+// us, blocks 380, scan 21 twice, the keys and ranks of the 15 windows longer than
+// LDS holds 80 and their sort; the whole call 1.34 ms.  Sorting the whole matrix
 // by (window, column, edge) with a device-wide sort, writing the blocks entry
 // by entry over a fill, and copying the stored values out in a pass of their
 // own took 43.5 ms; on 5000 rows with a product 535 us, now 203.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "srbcrs_convert.h"
 
@@ -173,39 +175,49 @@ __device__ __forceinline__ void radix_sort(uint64_t* key, int n, int bits, uint3
   }
 }
 
-// Tile of sorted keys -> ranks, stored counts and the per-entry outputs.
-// col(i) / edge(i): sorted entry i of the window; first and stored carry the
-// window's counts over the tiles before this one.
+// Sorted entry i of a window: col(i) / edge(i).  flag: bit 0 the first of its
+// column, bit 16 a stored value.
+struct Entry {
+  int c, e, row;
+  float v;
+  bool last;   // of its (row, column) run
+  uint32_t flag;
+};
+template <class Col, class Edge>
+__device__ __forceinline__ Entry entry_at(const ConvArgs& a, const int* rp, int rows, int n, int i, Col col,
+                                          Edge edge) {
+  Entry x;
+  x.c = col(i);
+  x.e = edge(i);
+  x.row = row_of(rp, rows, x.e);
+  const bool first = i == 0 || col(i - 1) != x.c;
+  x.last = i + 1 == n || col(i + 1) != x.c || row_of(rp, rows, edge(i + 1)) != x.row;
+  x.v = a.values[x.e];
+  x.flag = (first ? 1u : 0u) | (x.last && __float_as_uint(x.v) != 0u ? 1u << 16 : 0u);
+  return x;
+}
+
+// Tile of sorted keys -> ranks, stored counts and the per-entry outputs; firsts
+// and stored carry the window's counts over the tiles before this one.
 template <int T, class Col, class Edge>
 __device__ __forceinline__ void rank_tile(const ConvArgs& a, const int* rp, int rows, int n, int i0,
                                           uint32_t& firsts, uint32_t& stored, uint32_t* part, Col col, Edge edge) {
   const int e0 = rp[0];
   const int i = i0 + (int)threadIdx.x;
-  uint32_t flag = 0;
-  int c = 0, e = 0, row = 0;
-  float v = 0.f;
-  bool last = false;
-  if (i < n) {
-    c = col(i);
-    e = edge(i);
-    row = row_of(rp, rows, e);
-    const bool first = i == 0 || col(i - 1) != c;
-    last = i + 1 == n || col(i + 1) != c || row_of(rp, rows, edge(i + 1)) != row;
-    v = a.values[e];
-    flag = (first ? 1u : 0u) | (last && __float_as_uint(v) != 0u ? 1u << 16 : 0u);
-  }
+  Entry x{0, 0, 0, 0.f, false, 0u};
+  if (i < n) x = entry_at(a, rp, rows, n, i, col, edge);
   uint32_t total;
-  const uint32_t incl = block_scan<T>(flag, part, total);
+  const uint32_t incl = block_scan<T>(x.flag, part, total);
   if (i < n) {
     const int p = (int)(firsts + (incl & 0xffffu)) - 1;
     const int64_t at = (int64_t)e0 + i;
-    a.s.col[at] = c;
-    a.s.val[at] = v;
+    a.s.col[at] = x.c;
+    a.s.val[at] = x.v;
     a.s.rank[at] = p;
-    a.s.stored[at] = (int)(stored + ((incl - flag) >> 16));
-    a.s.row[at] = (uint8_t)(row | (last ? 0x80 : 0));
-    if ((flag & 1u) && p % a.bw == 0) a.s.block[(int64_t)e0 + p / a.bw] = i;
-    if (a.e2c) a.e2c[e] = p;
+    a.s.stored[at] = (int)(stored + ((incl - x.flag) >> 16));
+    a.s.row[at] = (uint8_t)(x.row | (x.last ? 0x80 : 0));
+    if ((x.flag & 1u) && p % a.bw == 0) a.s.block[(int64_t)e0 + p / a.bw] = i;
+    if (a.e2c) a.e2c[x.e] = p;
   }
   firsts += total & 0xffffu;
   stored += total >> 16;
@@ -332,8 +344,8 @@ __global__ __launch_bounds__(64) void k_big_offsets(ConvArgs a, int64_t* __restr
 
 // Windows too long for LDS: (index in a.big << 32 | column) keys of all of
 // them, one after the other, for one device-wide stable sort.  A row of the
-// grid takes every kBigRows-th window.
-constexpr int kBigRows = 64;   // times 16 workgroups a window: 4 per CU
+// grid takes every kBigRows-th window; 1024 workgroups in all.
+constexpr int kBigRows = 64;
 __global__ __launch_bounds__(256) void k_big_keys(ConvArgs a, int n_big, const int64_t* __restrict__ off,
                                                   uint64_t* __restrict__ keys, int* __restrict__ edges) {
   for (int b = blockIdx.y; b < n_big; b += gridDim.y) {
@@ -356,23 +368,56 @@ __global__ __launch_bounds__(256) void k_big_keys(ConvArgs a, int n_big, const i
   }
 }
 
-__global__ __launch_bounds__(1024) void k_big_rank(ConvArgs a, const int64_t* __restrict__ off,
-                                                   const uint64_t* __restrict__ keys, const int* __restrict__ edges) {
+// The long windows' tiles of 1024 sorted keys over `segs` workgroups each: pass 0
+// counts the firsts and stored values of a segment, pass 1 ranks it behind the
+// segments before it.  (With one workgroup a window the conversion of one of 16 M
+// entries took 60 ms, now 2.0; of 15 of 17000 and more in the graph above the pass
+// took 340 us of 1.40 ms, now 75.)
+template <int PASS>
+__global__ __launch_bounds__(1024) void k_big_rank(ConvArgs a, int segs, const int64_t* __restrict__ off,
+                                                   const uint64_t* __restrict__ keys, const int* __restrict__ edges,
+                                                   unsigned long long* __restrict__ counts) {
   __shared__ uint32_t part[16];
+  __shared__ uint32_t before[2];
   __shared__ int rp[33];
-  const int b = blockIdx.x, w = a.big[b];
+  const int b = (int)(blockIdx.x / (unsigned)segs), g = (int)(blockIdx.x % (unsigned)segs), w = a.big[b];
+  unsigned long long* cnt = counts + (int64_t)b * segs;
   int rows;
   if (!window_rows(a, w, rp, rows)) return;
   const int n = rp[rows] - rp[0];
+  const int tiles = (n + 1023) / 1024, per = (tiles + segs - 1) / segs;
+  const int t0 = g * per, t1 = t0 + per < tiles ? t0 + per : tiles;
   const uint64_t* k = keys + off[b];
   const int* ed = edges + off[b];
-  uint32_t firsts = 0, stored = 0;
-  for (int i0 = 0; i0 < n; i0 += 1024)
-    rank_tile<1024>(a, rp, rows, n, i0, firsts, stored, part, [&](int i) { return (int)(uint32_t)k[i]; },
-                    [&](int i) { return ed[i]; });
-  if (threadIdx.x == 0) {
-    put_count(a, w, firsts, stored);
-    note_max(&a.head->max_col1, (unsigned)(uint32_t)k[n - 1] + 1u);   // (negative columns refuse the matrix)
+  auto col = [&](int i) { return (int)(uint32_t)k[i]; };
+  auto edge = [&](int i) { return ed[i]; };
+  if (threadIdx.x < 2) before[threadIdx.x] = 0;
+  __syncthreads();
+  if constexpr (PASS == 0) {
+    uint32_t firsts = 0, stored = 0;
+    for (int64_t i = (int64_t)t0 * 1024 + threadIdx.x; i < (int64_t)t1 * 1024 && i < n; i += 1024) {
+      const uint32_t flag = entry_at(a, rp, rows, n, (int)i, col, edge).flag;
+      firsts += flag & 1u;
+      stored += flag >> 16;
+    }
+    uint32_t all_firsts, all_stored;
+    block_scan<1024>(firsts, part, all_firsts);
+    block_scan<1024>(stored, part, all_stored);
+    if (threadIdx.x == 0) cnt[g] = (unsigned long long)all_firsts | ((unsigned long long)all_stored << 32);
+  } else {
+    if (t0 >= t1) return;
+    if ((int)threadIdx.x < g) {   // segs <= 256
+      const unsigned long long c = cnt[threadIdx.x];
+      atomicAdd(&before[0], (uint32_t)c);
+      atomicAdd(&before[1], (uint32_t)(c >> 32));
+    }
+    __syncthreads();
+    uint32_t firsts = before[0], stored = before[1];
+    for (int t = t0; t < t1; ++t) rank_tile<1024>(a, rp, rows, n, t * 1024, firsts, stored, part, col, edge);
+    if (threadIdx.x == 0 && t1 == tiles) {
+      put_count(a, w, firsts, stored);
+      note_max(&a.head->max_col1, (unsigned)(uint32_t)k[n - 1] + 1u);   // (negative columns refuse the matrix)
+    }
   }
 }
 
@@ -627,8 +672,11 @@ hipError_t device_convert(const DeviceConvertIn& in, DeviceConvertOut& out, Devi
     if (!k0 || !k1 || !i0 || !i1 || !d_off) return hipErrorOutOfMemory;
     hipLaunchKernelGGL(k_big_offsets, dim3(1), dim3(64), 0, st, a, d_off);
     SRBCRS_TRY(hipGetLastError());
-    hipLaunchKernelGGL(k_big_keys, dim3(16, (unsigned)(h.n_big < kBigRows ? h.n_big : kBigRows)), dim3(256), 0, st, a,
-                       h.n_big, d_off, k0, i0);
+    const int grid_y = h.n_big < kBigRows ? h.n_big : kBigRows, segs = std::max(1, std::min(256, 2048 / h.n_big));
+    unsigned long long* counts = t.get<unsigned long long>((size_t)h.n_big * segs);
+    if (!counts) return hipErrorOutOfMemory;
+    hipLaunchKernelGGL(k_big_keys, dim3((unsigned)(1024 / grid_y), (unsigned)grid_y), dim3(256), 0, st, a, h.n_big,
+                       d_off, k0, i0);
     SRBCRS_TRY(hipGetLastError());
     hipcub::DoubleBuffer<uint64_t> kb(k0, k1);
     hipcub::DoubleBuffer<int> ib(i0, i1);
@@ -638,7 +686,10 @@ hipError_t device_convert(const DeviceConvertIn& in, DeviceConvertOut& out, Devi
     void* tmp = t.get<char>(bytes);
     if (!tmp) return hipErrorOutOfMemory;
     SRBCRS_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, bytes, kb, ib, (int)n, 0, end_bit, st));
-    hipLaunchKernelGGL(k_big_rank, dim3((unsigned)h.n_big), dim3(1024), 0, st, a, d_off, kb.Current(), ib.Current());
+    const dim3 grid((unsigned)(h.n_big * segs));
+    hipLaunchKernelGGL(k_big_rank<0>, grid, dim3(1024), 0, st, a, segs, d_off, kb.Current(), ib.Current(), counts);
+    SRBCRS_TRY(hipGetLastError());
+    hipLaunchKernelGGL(k_big_rank<1>, grid, dim3(1024), 0, st, a, segs, d_off, kb.Current(), ib.Current(), counts);
     SRBCRS_TRY(hipGetLastError());
     SRBCRS_TRY(scan());
   }

@@ -124,6 +124,26 @@ def test_device_conversion_many_long_windows(gpu):
     _same(_arrays(Plan(t(rp), t(ci), t(vv), M)), oracle.convert(rp, ci, vv, M))
 
 
+@pytest.mark.parametrize("lens", [(16385,), (300_000, 17000, 0, 1_048_577), (1_000_003,)])
+def test_device_conversion_very_long_windows(gpu, lens):
+    """Windows cut into segments over many workgroups: segments without a
+    tile, duplicate columns across tile ends, explicit zeros."""
+    import torch
+    from mask_amd.SRBCRSSpMM import Plan
+    rng = np.random.default_rng(lens[0])
+    M = 16 * len(lens) - 3
+    counts = []
+    for w, n in enumerate(lens):
+        rows = min(16, M - 16 * w)
+        counts.append(np.bincount(rng.integers(0, rows, n), minlength=rows))
+    rp = np.concatenate([[0], np.cumsum(np.concatenate(counts))]).astype(np.int32)
+    ci = rng.integers(0, 50_000, rp[-1]).astype(np.int32)      # unsorted, every column several times in a row
+    vv = np.where(rng.random(rp[-1]) < 0.2, 0.0, rng.uniform(-1, 1, rp[-1])).astype(np.float32)
+    _say("convert very long windows", lens)
+    t = lambda a: torch.from_numpy(a).cuda()
+    _same(_arrays(Plan(t(rp), t(ci), t(vv), M)), oracle.convert(rp, ci, vv, M))
+
+
 @pytest.mark.parametrize("n", [3, 3000, 17000])   # windows sorted by 256 and 512 threads, and past LDS
 def test_device_conversion_largest_column(gpu, n):
     """max_col is exact up to the largest column index: a dense operand must
