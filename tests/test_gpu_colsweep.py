@@ -110,6 +110,30 @@ def test_phase_sweep(gpu, shape, policy):
     assert not bool(torch.isfinite(_check(plan, B, (shape, "inf"))).all())
 
 
+# (M, K, columns per row, N): lists of 4 rows (too few rows for 8), and lists of 8 in workgroups of 16 waves in
+# step (more columns than the phase sweep's entries can name) at 32 and at 64 columns
+@pytest.mark.parametrize("shape", [(60000, 60000, 16, 64), (240500, 2_200_000, 8, 32), (120500, 2_200_000, 8, 48)])
+def test_list_layouts(gpu, shape):
+    """The list layouts and launches that the other shapes here do not take."""
+    import torch
+    M, K, per_row, N = shape
+    rng = np.random.default_rng(M)
+    lens = rng.integers(0, 2 * per_row + 1, M)
+    lens[[7, M // 3]] = 2000    # rows outside the lists
+    cols = rng.integers(0, K, int(lens.sum()))
+    row = np.repeat(np.arange(M), lens)
+    cols = cols[np.lexsort((cols, row))].astype(np.int32)
+    csr = (np.concatenate([[0], np.cumsum(lens)]).astype(np.int32), cols,
+           rng.uniform(-1, 1, cols.size).astype(np.float32))
+    print("[case] list layouts", shape, cols.size, flush=True)
+    plan = _plan(csr, M)
+    B = torch.rand((K, N), device="cuda") - 0.5
+    _check(plan, B, shape)
+    _check(plan, B, (shape, "relu"), relu=True)
+    B[int(cols[777]), 7] = float("nan")
+    assert not bool(torch.isfinite(_check(plan, B, (shape, "nan"))).all())
+
+
 @pytest.mark.parametrize("K,N,built", [(300000, 256, False), (300000, 224, True), (60000, 256, True)])
 def test_short_rows_without_shared_columns(gpu, K, N, built):
     """Ten values a row and under two a column at whole 64-column chunks: the
