@@ -295,8 +295,8 @@ struct SweepTasks {
 // ahead, its values and B rows one ahead.
 //
 // Bound as the block kernels are (gathers' L2 misses); one MI355X, the pass
-// alone: 65536 x 65536, 16 per row, N = 512 295 us (block kernels 275); 232965
-// of 50, N = 256 1680; 8000 of 16, N = 128 17.  One multiply-add per position
+// alone: 65536 x 65536, 16 per row, N = 512 370 us (block kernels 275); 232965
+// of 50, N = 256 2010; 8000 of 16, N = 128 17.  One multiply-add per position
 // and column, its A values by scalar loads, took 1615, 8080 and 104.
 static __global__ __launch_bounds__(64) void k_sweep_repair(unsigned long long* __restrict__ mark,
                                                             unsigned long long token, SweepTasks t,
