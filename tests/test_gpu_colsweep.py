@@ -302,5 +302,60 @@ def test_replay_after_a_non_finite_one(gpu, M, per_row, N):
     before = replay(0)
     for _ in range(2):
         replay(1)
-        # the repair pass took ten times the sweep where it ran on
+        # (a repair pass more than doubles a replay)
         assert replay(0) < 1.5 * before + 0.01
+
+
+def test_widths_that_share_streams(gpu):
+    """Once a schedule's streams hold as much as the block values, a width runs
+    on the stream of another one, of either kind: the same bits."""
+    import torch
+    M = K = 65536
+    rng = np.random.default_rng(11)
+    cols = np.sort(rng.integers(0, K, (M, 16)), axis=1).astype(np.int32).ravel()
+    plan = _plan((np.arange(M + 1, dtype=np.int32) * 16, cols, rng.uniform(-1, 1, cols.size).astype(np.float32)), M)
+    wide = torch.rand((K, 512), device="cuda") - 0.5
+    plan.trim()
+    torch.cuda.synchronize()
+    out, free = torch.empty((M, 512), device="cuda"), torch.cuda.mem_get_info()[0]
+    widths = list(range(512, 95, -32)) + [80, 64, 48, 32, 16]
+    for N in widths:
+        for _ in range(2):
+            plan.run(wide[:, :N], out[:, :N])
+    plan.trim()   # the builds' temporaries
+    streams = free - torch.cuda.mem_get_info()[0]
+    assert 2 * 8 * cols.size < streams < plan.total_blocks * 512 + 8 * cols.size, streams
+    for N in widths:
+        print("[case] shared stream", N, flush=True)
+        _check(plan, wide[:, :N].contiguous(), N)
+
+
+def test_more_captured_runs_than_marks(gpu):
+    """Runs recorded past the 1024th of a plan have no mark of their own: their
+    replays are repaired as well."""
+    import torch
+    M = K = 2000
+    csr = _csr(M, K, 20, 2, 4)
+    plan = _plan(csr, M)
+    fine = torch.rand((K, 64), device="cuda") - 0.5
+    bad = fine.clone()
+    bad[int(csr[1][7])] = float("inf")
+    B, C = fine.clone(), [torch.empty((M, 64), device="cuda") for _ in range(2)]
+    refs = [plan.run(b, grid_order=1, depth=2, wg_cols=128) for b in (fine, bad)]
+    for _ in range(2):
+        plan.run(B, C[0])
+    torch.cuda.synchronize()
+    print("[case] more captured runs than marks", flush=True)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        for _ in range(1030):
+            plan.run(B, C[0])
+        plan.run(B, C[1])
+    for i in (0, 1, 0, 1, 0):
+        B.copy_((fine, bad)[i])
+        for c in C:
+            c.fill_(7.0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(_same(c, refs[i]) for c in C), i
+        plan.run(B)   # eager work between replays
