@@ -213,15 +213,16 @@ int srbcrs_plan_set_schedule(srbcrs_plan *plan, const char *policy, int32_t para
  * On matrices of low block fill (16x8 blocks, under a ninth of the positions
  * stored) the default launch is the column sweep, a vector kernel over the
  * stored values that gives the block kernels' bits (infinities and NaNs of B
- * included); it needs ldb, ldc multiples of 4, 16-byte aligned B and C and
+ * included; a sum of nothing but underflowed products, zero, may differ in its
+ * sign); it needs ldb, ldc multiples of 4, 16-byte aligned B and C and
  * K * ldb * 4 < 2^32, and runs from a width's second run on, which builds its
  * entry stream: it allocates 8 bytes per stored value plus up to 7 entries of
  * padding per list (16 bytes a value in all on rows of 4; streams under 16 MB
- * take room for the most they may need).  Widths share
- * streams where their layout is the same, and always once a schedule's streams
- * together hold as many bytes as the plan's block values.  Capture after two
- * eager runs to capture the sweep.  Elsewhere, under
- * capture before that, and on small products, the block kernels run.  A call
+ * take room for the most they may need).  Widths share streams where their
+ * layout is the same, and always once a schedule's streams together hold as
+ * many bytes as the plan's block values.  Capture after two eager runs to
+ * capture the sweep.  Elsewhere, under capture before that, on small products
+ * and where the block kernels are known to be the faster, those run.  A call
  * that is refused (a negative status) has launched nothing and left C
  * untouched. */
 int srbcrs_run(srbcrs_plan *plan, const float *d_B, int64_t K, int64_t N, int64_t ldb,
@@ -232,12 +233,12 @@ int srbcrs_run(srbcrs_plan *plan, const float *d_B, int64_t K, int64_t N, int64_
  * Retired buffers are what graphs captured on earlier runs may still
  * address: call this only when no such graph will be replayed again and no
  * launch that used them is in flight on another stream.  Without it they
- * are freed with the plan.  So are, by this call, the column sweep's entry
+ * are freed with the plan.  The call also frees the column sweep's entry
  * streams of schedules that the plan no longer has, unless a run recorded into
- * a graph used them (those stay until the plan is destroyed).  Also gives back to the driver the device memory
- * that destroyed plans and conversions have left (kept, up to 4 GiB a
- * process, for the next ones).  No reference counterpart (the reference
- * keeps one global cache entry). */
+ * a graph used them (those stay until the plan is destroyed), and gives back
+ * to the driver the device memory that destroyed plans and conversions have
+ * left (kept, up to 4 GiB a process, for the next ones).  No reference
+ * counterpart (the reference keeps one global cache entry). */
 int srbcrs_plan_trim(srbcrs_plan *plan, void *stream);
 
 /* Give that kept device memory of the current device back to the driver, with

@@ -214,7 +214,8 @@ class Plan:
     def tune(self, dense: Tensor, out: Optional[Tensor] = None, reps: int = 3, nonzero_sweep: bool = False) -> dict:
         """Time the launch candidates for dense.shape[1] on this plan (see
         srbcrs_plan_tune) and keep the fastest for later default-knob runs
-        at that width; returns the choice.  out (or a scratch tensor) is
+        at that width; returns the choice (where the default launch itself is
+        the fastest it stays, and the best knob setting is returned).  out (or a scratch tensor) is
         overwritten with A @ dense.  nonzero_sweep=True also times the
         nonzero sweep (srbcrs_plan_tune_ex, SRBCRS_TUNE_NONZERO_SWEEP),
         whose bits are the fp32 CSR product's."""
@@ -363,9 +364,14 @@ def _preprocess(colind: Tensor, rowptr: Tensor, values: Tensor, num_nodes: int, 
 
 # Block fill (stored values / (blocks * 128)) below which the nonzero sweep
 # beats the tuned MFMA kernels at N = 512 on one MI355X (bench.py
-# --sweep-crossover, 16 values per row, window-clustered columns; sustained ms,
-# sweep / tuned MFMA): fill 0.062 0.136 / 0.213, 0.095 0.136 / 0.158, 0.137
-# 0.135 / 0.121, 0.250 0.136 / 0.082.
+# --sweep-crossover, 65536 rows of 16, window-clustered columns; sustained ms,
+# nonzero sweep / tuned MFMA / default launch): fill 0.062 0.136 / 0.213 / 0.157,
+# 0.095 0.136 / 0.157 / 0.155, 0.137 0.136 / 0.122 / 0.138, 0.250 0.138 / 0.083 /
+# 0.092.  The default launch there is the phase or column sweep by now, which
+# takes less away from this shape (us, nonzero sweep / default: 4096 rows of 20,
+# N = 64 36 / 9; 100000 of 30, N = 256 236 / 204; 300000 of 16, N = 512 1369 /
+# 1221): a caller who wants the faster one and not the CSR product's bits leaves
+# SPARSENE_ALLOW_CSR_FALLBACK unset.
 SWEEP_FILL = 0.125
 
 

@@ -894,8 +894,12 @@ hipError_t prepare_sweeps(srbcrs_plan& plan, hipStream_t st) {
 
 // The column sweep stream for a run of N columns; null: run the block
 // kernels, which give the same bits.  The first run of a width does that: a
-// plan run once (a sampled graph) does not pay for the stream, which takes
-// about as long as a few runs gain.  Not built under graph capture or for a
+// plan run once (a sampled graph) does not pay for the stream, which takes as
+// long as 1.5 to 10 runs gain (us of a new plan's first run / the second, which
+// builds the stream / the later ones: uniform 65536 x 65536, 16 per row, N = 512
+// 271 / 462 / 164; power-law, 2^20 nodes, N = 512 12130 / 15620 / 8680; 232965
+// nodes, N = 256 1894 / 3127 / 1025; 100003 x 30011, 10 per row, N = 128 76 / 256
+// / 50; 4096 x 4096, 20 per row, N = 64 29 / 153 / 14).  Not built under graph capture or for a
 // caller that may not allocate.  A build that fails, for want of memory say,
 // costs the run nothing but its time: the block kernels take it, and the next
 // attempts come after 1, 2, 4, ... 1024 runs more.

@@ -8,22 +8,24 @@
 // included), and a zero of A adds +-0, which changes no finite sum.  So the
 // chain of fmaf over a row's stored values alone, blocks in ascending order
 // and the columns of a block in the order 0 2 4 6 1 3 5 7 (spmm_stream's two
-// k-steps), gives the same bits.  What differs is B's infinities and NaNs:
-// the block kernels multiply them by A's zeros and so poison every row of a
-// window whose blocks hold the column.  Each wave therefore checks the sums
-// it stores, and a non-finite one raises a mark on which k_sweep_repair
-// (below) recomputes the product with A's zeros in it.
+// k-steps), gives the same bits, but for the sign of a zero: a sum whose every
+// product so far rounded to -0 (negative, under half the smallest denormal)
+// stays -0 here, where a zero term of the block kernels may lift it to +0.  What
+// differs is B's infinities and NaNs: the block kernels multiply them by A's
+// zeros and so poison every row of a window whose blocks hold the column.  Each
+// wave therefore checks the sums it stores, and a non-finite one raises a mark
+// on which k_sweep_repair (below) recomputes the product with A's zeros in it.
 //
 // Why this order.  Every gathered segment comes through the L2, and what
 // bounds the SpMM on matrices without block structure is the rate of L2
-// misses (6.5-7.5 TB/s whatever the gathers' order within a row).  The hits
+// misses (5.6-7.5 TB/s whatever the gathers' order within a row).  The hits
 // can be raised: when the waves of an XCD walk B from its first rows to its
 // last at the same pace, a segment that one of them brings in serves the
 // others.  The more rows are in flight at a time, the more gathers share
 // each pass over B, so the sums of all rows in flight live in LDS (8 rows of
 // 32 or 64 columns per lane group: 1280 or 640 rows per CU), the entry stream
 // is sorted by column phase first and row second, and the waves of a
-// workgroup keep step with a barrier every other batch.  Within a phase a
+// workgroup keep step with a barrier every fourth batch.  Within a phase a
 // row's values are consecutive, so the sum stays in registers and goes to
 // LDS once per row and phase.
 //
@@ -35,16 +37,16 @@
 // lists do not depend on C: a wave takes 8 (C = 32) or 4 (C = 64)
 // neighbouring ones.
 //
-// Measured against the block kernels at their default knobs (one MI355X,
-// back-to-back runs on one B, us): uniform 65536 x 65536, 16 per row, N = 512
-// 264 -> 160 (three B in turn, so that none stays in the memory-side cache:
-// 264 -> 190); power-law graph of 232965 nodes and 11.7 M values, N = 256
-// 1755 -> 1290; of 2^20 nodes and 34.6 M values, N = 512 11560 -> 10400; of
-// 116483 nodes, N = 48 295 -> 71; of 58241 nodes, N = 256 403 -> 240.
-// Phases and the barrier give uniform 218 -> 160 and the 232965-node graph
-// 1430 -> 1290.  Rejected: pacing the waves of an XCD against a shared
-// counter (its atomics cost more than the hits gained: 1430 -> 1660 before
-// any wave waits).
+// Measured against the block kernels at their default knobs (one MI355X, us):
+// 4096 x 4096, 20 per row, N = 64 kernel 22.9 -> 7.6;
+// 100003 x 30011, 10 per row, N = 128 68.9 -> 43.3, 21 % of L2 requests miss.  On
+// the large matrices that the phase sweep (srbcrs_phasesweep.hpp) has taken
+// since: uniform 65536 x 65536, 16 per row, N = 512 264 -> 190; power-law graph
+// of 232965 nodes and 11.7 M values, N = 256 1755 -> 1290; of 2^20 nodes and
+// 34.6 M values, N = 512 11560 -> 10400; phases and the barrier gave the
+// 232965-node graph 1430 -> 1290.  Rejected: pacing the waves of an XCD against
+// a shared counter (its atomics cost more than the hits gained: 1430 -> 1660
+// before any wave waits).
 #pragma once
 #include "srbcrs_merged.hpp"
 

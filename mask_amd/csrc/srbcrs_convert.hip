@@ -16,9 +16,9 @@
 //
 // Bound: the dense values, 512 bytes a block, written once (11.7 M edges of a
 // power-law graph, 232965 rows, 1.4 M blocks: 0.71 GB of 0.95 GB moved, 190 us
-// at the rate of a copy).  Measured on that graph (one MI355X): the windows 460
-// us, blocks 380, scan 21 twice, the keys and ranks of the 15 windows longer than
-// LDS holds 80 and their sort; the whole call 1.34 ms.  Sorting the whole matrix
+// at the rate of a copy).  Measured on that graph (one MI355X): the windows 455
+// us, blocks 382, scan 21 twice, of the 15 windows longer than LDS holds the keys
+// and ranks 46 and the sort's 21 launches 130; the whole call 1.34 ms.  Sorting the whole matrix
 // by (window, column, edge) with a device-wide sort, writing the blocks entry
 // by entry over a fill, and copying the stored values out in a pass of their
 // own took 43.5 ms; on 5000 rows with a product 535 us, now 203.
@@ -371,8 +371,8 @@ __global__ __launch_bounds__(256) void k_big_keys(ConvArgs a, int n_big, const i
 // The long windows' tiles of 1024 sorted keys over `segs` workgroups each: pass 0
 // counts the firsts and stored values of a segment, pass 1 ranks it behind the
 // segments before it.  (With one workgroup a window the conversion of one of 16 M
-// entries took 60 ms, now 2.0; of 15 of 17000 and more in the graph above the pass
-// took 340 us of 1.40 ms, now 75.)
+// entries took 60 ms, now 2.0; on the 15 of the graph above the pass took 102 us of
+// 1.40 ms, now 39.)
 template <int PASS>
 __global__ __launch_bounds__(1024) void k_big_rank(ConvArgs a, int segs, const int64_t* __restrict__ off,
                                                    const uint64_t* __restrict__ keys, const int* __restrict__ edges,

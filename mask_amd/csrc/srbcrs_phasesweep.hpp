@@ -4,7 +4,7 @@
 // The column sweep's lists advance through B entry by entry, and lists whose
 // rows favour other columns drift apart: on a power-law graph of 232965 nodes
 // the rows in flight on an XCD touch a tenth as many B rows as they have
-// values, yet 58 % of the gathers missed the L2.  Here B is cut into phases of
+// values, yet 58 % of the L2 requests missed.  Here B is cut into phases of
 // equally many values.  A unit is two halves of up to 640 rows; a workgroup
 // holds the sums of one half (16 waves at 64 columns, 8 at 32) or of both (16
 // waves at 32) in LDS, and any lane group may add to any row of its half: per
@@ -24,8 +24,8 @@
 // follow each other on a list, both happen in one step.
 //
 // Measured against the column sweep (one MI355X, three B in turn, us): the
-// 232965-node graph, N = 256 1284 -> 988 (misses 58 % -> 30 %), N = 128 666 ->
-// 482; 2^20 nodes, 34.4 M values, N = 512 10570 -> 8680; 116483 nodes, N = 256
+// 232965-node graph, N = 256 1284 -> 988 (misses 58 % -> 48 %), N = 128 666 ->
+// 482; 2^20 nodes, 34.4 M values, N = 512 10570 -> 8680 (78 % -> 58 %); 116483 nodes, N = 256
 // 292 -> 245; uniform 100000 x 100000, 30 per row, N = 256 276 -> 221; 65536 x
 // 65536, 16 per row, N = 512 189 -> 182.
 //
