@@ -806,6 +806,12 @@ __global__ __launch_bounds__(256) void zero_rows(T* __restrict__ C, const int* _
 // chunk (one MI355X, us): 50021 x 65536, 24 per row, N = 256 169 -> 138, N = 64
 // 48 -> 35, N = 16 40 -> 15; power-law, 200000 nodes, N = 256 925 -> 611.
 //
+// A wave runs as long as the longest row of its groups, so a workgroup with a
+// row of more than twice the mean deals its 16 or 32 rows to them by length
+// (30000 rows of which a tenth hold 600 values, K = 1000, N = 512 392 -> 241, a
+// wave per row and 256 columns 196; of 348 products of rows like these 6 take
+// more than 5 % longer than dealt as they come, by 9 % at most).
+//
 // A group's lanes load 8 entries of its row at a time and broadcast them; past
 // the row's end the gather lies past B's end (it returns 0 and fetches
 // nothing) and the value is -0, which changes no sum.
@@ -821,12 +827,26 @@ __global__ __launch_bounds__(256) void csr_spmm_rowgroup(const int* __restrict__
   sweep_chunk((int)blockIdx.x, (int)gridDim.x, n_wg, n_chunks, 0, wg, c);
   if (wg >= n_wg) return;
   const int lane = threadIdx.x & 63, grp = lane / LPG, sub = lane % LPG;
-  const int64_t row = ((int64_t)wg * 4 + (threadIdx.x >> 6)) * LG + grp;
-  int e0 = 0, n = 0;
-  if (row < M) {
-    e0 = rowptr[row];
-    n = rowptr[row + 1] - e0;
+  // the workgroup's R rows, one a lane (past the last: none), then each group's
+  constexpr int R = 4 * LG;
+  const int64_t r0 = (int64_t)wg * R;
+  const int own = lane & (R - 1);
+  const int own_e0 = rowptr[r0 + own < M ? r0 + own : M];
+  const int own_e1 = rowptr[r0 + own + 1 < M ? r0 + own + 1 : M];
+  const int len = own_e1 - own_e0;
+  const uint32_t total = (uint32_t)(__builtin_amdgcn_readlane(own_e1, R - 1) - __builtin_amdgcn_readlane(own_e0, 0));
+  int at = (int)(threadIdx.x >> 6) * LG + grp;
+  if (__any((uint32_t)len / 2 > total / R)) {
+    int rank = 0;   // of row `own`, longest first
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const int o = __builtin_amdgcn_readlane(len, k);
+      rank += o > len || (o == len && k < own) ? 1 : 0;
+    }
+    at = __shfl(__builtin_amdgcn_ds_permute(4 * rank, own), at);
   }
+  const int64_t row = r0 + at;
+  const int e0 = __shfl(own_e0, at), n = __shfl(len, at);
   int most = n;
 #pragma unroll
   for (int d = LPG; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d));

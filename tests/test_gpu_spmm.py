@@ -198,6 +198,69 @@ def test_csr_row_groups(gpu, shape):
     assert_gate(gate(out[:M].cpu().numpy(), rowptr, colind, values, np.ascontiguousarray(B[:, :N]), M))
 
 
+# (M, K, N): workgroups of 16 rows of 64 columns and of 32 rows of 32, the last ones not whole
+@pytest.mark.parametrize("shape", [(16, 1000, 64), (4099, 1000, 100), (32, 20000, 64), (4099, 20000, 96)])
+def test_csr_rows_of_unlike_length(gpu, shape):
+    """A workgroup ranks its rows by length: every row keeps its own sum, the
+    same bits wherever it stands."""
+    torch = _torch()
+    from mask_amd.SRBCRSSpMM import csr_spmm
+    M, K, N = shape
+    rng = np.random.default_rng(M + N)
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    dB = torch.from_numpy(B).cuda()
+    for kind, lens in (("equal", np.full(M, 5)), ("few", np.where(rng.random(M) < 0.1, 90, 0)),
+                       ("rising", np.arange(M) % 41), ("falling", 40 - np.arange(M) % 41),
+                       ("last", np.where(np.arange(M) == M - 1, 300, 0))):
+        rows = [(rng.integers(0, K, n).astype(np.int32), rng.uniform(-1, 1, n).astype(np.float32)) for n in lens]
+
+        def product(order):
+            rp = np.concatenate([[0], np.cumsum(lens[order])]).astype(np.int32)
+            csr = rp, np.concatenate([rows[i][0] for i in order]), np.concatenate([rows[i][1] for i in order])
+            return csr, csr_spmm(*(torch.from_numpy(a).cuda() for a in csr), dB, M)
+
+        _say("csr unlike rows", shape, kind)
+        csr, out = product(np.arange(M))
+        assert_gate(gate(out.cpu().numpy(), *csr, B, M))
+        order = rng.permutation(M)
+        assert torch.equal(product(order)[1], out[torch.from_numpy(order).cuda()]), kind
+
+
+def test_csr_few_long_rows_among_empty_ones(gpu):
+    """Long rows scattered among empty ones take about what they take in a row:
+    a wave whose other rows are empty runs at a quarter of its width."""
+    torch = _torch()
+    from mask_amd.SRBCRSSpMM import csr_spmm
+    M, K, N, per = 30000, 1000, 512, 600
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    colind = torch.randint(0, K, (M // 10 * per,), generator=g, device="cuda", dtype=torch.int32)
+    values = torch.rand(colind.numel(), generator=g, device="cuda") - 0.5
+    B = torch.rand((K, N), generator=g, device="cuda") - 0.5
+    _say("csr few long rows")
+    times, outs = [], []
+    for rows in (torch.arange(M // 10), torch.sort(torch.randperm(M, generator=torch.Generator().manual_seed(2))[: M // 10]).values):
+        rows = rows.cuda()
+        lens = torch.zeros(M, dtype=torch.int64, device="cuda")
+        lens[rows] = per
+        rowptr = torch.zeros(M + 1, dtype=torch.int32, device="cuda")
+        rowptr[1:] = torch.cumsum(lens, 0)
+        out = torch.empty((M, N), device="cuda")
+        best = float("inf")
+        for _ in range(12):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            csr_spmm(rowptr, colind, values, B, M, max_col=K - 1, out=out)
+            e[1].record()
+            torch.cuda.synchronize()
+            best = min(best, e[0].elapsed_time(e[1]))
+        times.append(best)
+        outs.append(out[rows])
+    print("[case] in a row, scattered (ms):", times, flush=True)
+    assert torch.equal(*outs)
+    assert times[1] < 1.5 * times[0] + 0.01, times
+
+
 def test_values_that_are_no_knobs_are_refused(gpu):
     """Also those that are false in a condition, like the knobs' defaults."""
     torch = _torch()
