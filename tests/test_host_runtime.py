@@ -206,6 +206,41 @@ assert rc == _capi.SRBCRS_ENOMEM and "out of memory" in error(), error()
 """)
 
 
+def test_kept_memory_of_many_sizes_costs_no_time(fake_hip):
+    """A conversion takes what it took before 400 graphs of other sizes were
+    dropped, whose arrays are all kept."""
+    _run(fake_hip, """
+import time
+c = csr(64, 500, 5)
+def once():
+    head(200, c[1].size, 499)
+    rc, h = create(c, 64, 1)
+    assert rc == 0, error()
+    L.srbcrs_plan_destroy(h)
+def best():
+    times = []
+    for _ in range(200):
+        t = time.perf_counter()
+        once()
+        times.append(time.perf_counter() - t)
+    return sorted(times)[20]
+before = best()
+plans = []
+for i in range(400):
+    o = csr(640 + 48 * i, 500, 5)
+    head(200 + 7 * i, o[1].size, 499)
+    rc, h = create(o, 640 + 48 * i, 1)
+    assert rc == 0, error()
+    plans.append(h)
+for h in plans:
+    L.srbcrs_plan_destroy(h)
+assert fake.fake_live_blocks() > 2000
+after = best()
+print(before, after)
+assert after < 1.5 * before + 2e-5, (before, after)
+""")
+
+
 # (M, K, values a row, N, schedule, span of a window's columns, whether the second run is a sweep):
 # both sides of the dispatch rules
 @pytest.mark.parametrize("M,K,per_row,N,schedule,span,sweep", [
