@@ -942,11 +942,14 @@ const srbcrs::ColSweep* sweep_stream(srbcrs_plan& plan, int64_t N, bool may_buil
     // less than their launches, unless long tasks make the block kernel a
     // chain (about 0.4 us a block: 40 blocks 17.9 us, sweep 8 + 1.5; power-law
     // graph of 4096 nodes and 153 K values, N = 64, blocks / sweep: whole windows
-    // 67 / 16, split:64 27 / 20, split:32 17.8 / 20.9, split:16 15.1 / 21.7).
+    // 67 / 16, split:64 27 / 20, split:32 17.8 / 20.9, split:16 15.1 / 21.7; over 171
+    // small products of 3000 to 300000 rows of unlike length, longest window of 24
+    // to 31 blocks: sweep 1.055 times the blocks' time, by up to 1.6; 32 to 39 0.93;
+    // 40 to 63 0.81).
     // Tasks of 8 blocks and less cost the sweep a list row each for a few
     // values: it is slower up to 64 columns (8000 nodes, 377 K values, split:8,
     // N = 64 32 / 40, N = 256 74 / 69).
-    if (w.longest < 24 && plan.n_apacked * N < (16 << 20)) return nullptr;
+    if (w.longest < 32 && plan.n_apacked * N < (16 << 20)) return nullptr;
     if (w.longest <= 8 && plan.sched.policy != "row" && N <= 64) return nullptr;
     if (w.built) return take(w);
     if (w.unfit) continue;

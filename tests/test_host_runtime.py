@@ -255,7 +255,7 @@ assert after < 1.5 * before + 2e-5, (before, after)
     (60000, 60000, 16, 128, "row:0", 400, True), (200000, 200000, 16, 48, "row:0", 400, True),
     (60000, 60000, 3, 256, "row:0", 400, False), (60000, 60000, 5, 256, "row:0", 400, True),  # reuse 1 of short local rows
     (4096, 4096, 20, 64, "row:0", 0, True), (4096, 4096, 20, 64, "split:16", 0, False),       # small: long tasks only
-    (4096, 4096, 20, 64, "split:32", 0, True),
+    (4096, 4096, 20, 64, "split:31", 0, False), (4096, 4096, 20, 64, "split:32", 0, True),
     (20000, 20000, 20, 64, "split:8", 0, False), (20000, 20000, 20, 64, "split:9", 0, True),  # short tasks
     (20000, 20000, 20, 128, "split:8", 0, True), (1000, 1000, 4, 64, "row:0", 0, False),
 ])
