@@ -18,7 +18,7 @@
 // power-law graph, 232965 rows, 1.4 M blocks: 0.71 GB of 0.95 GB moved, 190 us
 // at the rate of a copy).  Measured on that graph (one MI355X): the windows 455
 // us, blocks 382, scan 21 twice, of the 15 windows longer than LDS holds the keys
-// and ranks 46 and the sort's 21 launches 130; the whole call 1.34 ms.  Sorting the whole matrix
+// and ranks 46 and the sort's 21 launches 130; the whole call 1.32 ms.  Sorting the whole matrix
 // by (window, column, edge) with a device-wide sort, writing the blocks entry
 // by entry over a fill, and copying the stored values out in a pass of their
 // own took 43.5 ms; on 5000 rows with a product 535 us, now 203.
